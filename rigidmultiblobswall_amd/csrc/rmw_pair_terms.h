@@ -90,6 +90,11 @@ RMW_HD double rcp(double x) { return 1.0 / x; }
 RMW_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 RMW_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
+// The smaller of x and a constant; a NaN x gives the constant (the pairs
+// concerned keep an unclamped factor that carries the NaN).
+RMW_HD float min_(float x, float c) { return __builtin_fminf(x, c); }
+RMW_HD double min_(double x, double c) { return __builtin_fmin(x, c); }
+
 // ---------------------------------------------------------------------------
 // Shared geometry of one (target, source) pair.
 // ---------------------------------------------------------------------------
@@ -97,9 +102,19 @@ template <typename T> struct Geom {
   T dx, dy, dz;   // d = r_i - r_j (units of a)
   T Rz;           // z_i + z_j
   T r2, invr, r;  // |d|^2, 1/|d|, |d|
+  T ic, rm;       // min(1/|d|, 1/2) and min(|d|, 2): see "overlapping blobs"
   T invR;         // 1/|R|
-  T ez, ez2;      // R_z/|R| and its square
 };
+
+// Overlapping blobs.  Every RPY coefficient has a far form (|d| > 2) and an
+// overlap form that meet at |d| = 2.  Instead of evaluating both and
+// selecting, the far form is taken at |d| clamped from below at 2 (through
+// ic = min(1/|d|, 1/2)) and the overlap form's difference from its value at
+// 2 is added through rm = min(|d|, 2).  The constants are chosen so that the
+// added polynomial is exactly 0 in binary arithmetic at rm = 2, so far pairs
+// get the far form bit for bit.  On gfx950 a compare and each select take
+// two issue cycles against one for an FMA: the two minima replace three
+// compares and five selects of the four blocks (UF 2 selects and 1 compare).
 
 template <typename T>
 RMW_HD Geom<T> make_geom(T dx, T dy, T dz, T zi, T zj)
@@ -111,10 +126,10 @@ RMW_HD Geom<T> make_geom(T dx, T dy, T dz, T zi, T zj)
   g.r2 = p2 + dz * dz;
   g.invr = rsq(g.r2);
   g.r = g.r2 * g.invr;
+  g.ic = min_(g.invr, T(0.5));
+  g.rm = min_(g.r, T(2));
   T R2 = p2 + g.Rz * g.Rz;
   g.invR = rsq(R2);
-  g.ez = g.Rz * g.invR;
-  g.ez2 = g.ez * g.ez;
   return g;
 }
 
@@ -134,11 +149,11 @@ RMW_HD Geom<T> make_geom_on(T dx, T dy, T dz, T zi, T zj, bool on)
   const T ir = rsq(g.r2);
   g.invr = on ? ir : T(0);
   g.r = on ? g.r2 * ir : T(3);
+  g.ic = min_(g.invr, T(0.5));
+  g.rm = min_(g.r, T(2));
   T R2 = p2 + g.Rz * g.Rz;
   const T iR = rsq(R2);
   g.invR = on ? iR : T(0);
-  g.ez = g.Rz * g.invR;
-  g.ez2 = g.ez * g.ez;
   return g;
 }
 
@@ -154,20 +169,19 @@ template <typename T> struct CoefUF {
   T g4;     // f4 / |R|    -> coefficient of (R.v) z
 };
 
-// RPY translational coefficients A I + B r r^T at distance r (units of a):
-// far (r > 2) and overlapping branches as selects.
+// RPY translational coefficients A I + B r r^T (units of a):
+//   far      A = (1 + 2/(3 r^2))/r,  B = (1 - 2/r^2)/r^3
+//   overlap  A = 4/3 - 3 r/8,        B = 1/(8 r)
+// With ic and rm, A = ic + 2 ic^3/3 + (3/4 - 3 rm/8) and B = (1 - 2 ic^2)
+// ic^2 / r.  Returned is A - sub: above a wall far pairs lose most of A to
+// the image's 1/|R|, and taking that off ic first (sub = 1/|R|) leaves the
+// difference free of the rounding of A.
 template <typename T>
-RMW_HD void rpy_tt(T r, T invr, T& A, T& B)
+RMW_HD void rpy_tt(T invr, T ic, T rm, T sub, T& A, T& B)
 {
-  const T one = T(1), two = T(2);
-  T invr2 = invr * invr;
-  T A_far = (one + T(2.0 / 3.0) * invr2) * invr;
-  T B_far = (one - two * invr2) * (invr2 * invr);
-  T A_near = T(4.0 / 3.0) - T(4.0 / 3.0 * 0.28125) * r;
-  T B_near = T(4.0 / 3.0 * 0.09375) * invr;
-  bool far = r > two;
-  A = far ? A_far : A_near;
-  B = far ? B_far : B_near;
+  const T w = ic * ic;
+  A = fma_(T(2.0 / 3.0), w * ic, (ic - sub) + fma_(T(-0.375), rm, T(0.75)));
+  B = fma_(T(-2), w, T(1)) * w * invr;
 }
 
 template <typename T>
@@ -176,7 +190,7 @@ RMW_HD CoefUF<T> coef_uf(const Geom<T>& g, T zi, T zj, int dom = kDomWall)
   const T one = T(1);
   CoefUF<T> c;
   T A;
-  rpy_tt(g.r, g.invr, A, c.Bc);
+  rpy_tt(g.invr, g.ic, g.rm, dom_has_wall(dom) ? g.invR : T(0), A, c.Bc);
   if (dom == kDomNoWall) {
     c.s = A; c.s5 = A; c.g2 = T(0); c.g3 = T(0); c.g4 = T(0);
     return c;
@@ -184,7 +198,7 @@ RMW_HD CoefUF<T> coef_uf(const Geom<T>& g, T zi, T zj, int dom = kDomWall)
   if (dom == kDomFreeSurface) {
     // + RPY(R) D v = A_R (v - 2 v_z z) + B_R R (R.v) - 2 B_R R_z v_z R
     T AR, BR;
-    rpy_tt(one / g.invR, g.invR, AR, BR);
+    rpy_tt(g.invR, min_(g.invR, T(0.5)), min_(one / g.invR, T(2)), T(0), AR, BR);
     c.s = A + AR; c.s5 = A - AR; c.g2 = BR; c.g3 = T(-2) * BR * g.Rz; c.g4 = T(0);
     return c;
   }
@@ -194,70 +208,73 @@ RMW_HD CoefUF<T> coef_uf(const Geom<T>& g, T zi, T zj, int dom = kDomWall)
   // h_hat = z_j/R_z the h_hat factors combine into division-free monomials:
   //   h_hat (1-h_hat) e_z^2 = z_i z_j w,  h_hat e_z / |R| = z_j w,
   //   (1-h_hat) e_z^2 = z_i R_z w,        h_hat^2 e_z^2 = z_j^2 w,
-  // giving
+  // giving, with q = 1/|R|, zz = z_i z_j, b = R_z w,
+  // P = -6 zz - 2 + 10 E + w (10/3 - 70 E/3) and m = (10/3) b w,
   //   f1 = -q [1 + w (2 zz + 2/3 - 2E) + w^2 (10E/3 - 2/3)]
-  //   f2 = -q [1 + w (-6 zz - 2 + 10E) + w^2 (10/3 - 70E/3)]
-  //   f3 = w [2 z_j + R_z w (-12 zz - 4 + 20E + w (40/3 - 140E/3))]
-  //   f4 = w [2 z_j - (20/3) R_z w^2]
-  //   f5 = -q w [4 z_j^2 + 4E + w (8/3 - 20E)]
-  // with q = 1/|R| and zz = z_i z_j.
+  //   f2 = -q [1 + w P]
+  //   f3 = 2 w [z_j + b P + m]
+  //   f4 = 2 w [z_j - m]
+  //   f5 = -4 q w [z_j^2 + E + w (2/3 - 5E)]
   T q = g.invR;
   T w = q * q;
-  T E = g.ez2;
+  T b = g.Rz * w;
+  T E = g.Rz * b;
   T zz = zi * zj;
   T t1 = fma_(T(2), zz, fma_(T(-2), E, T(2.0 / 3.0)));
   T t2 = fma_(T(10.0 / 3.0), E, T(-2.0 / 3.0));
-  T f1 = -q * fma_(w, fma_(w, t2, t1), one);
+  T qw = q * w;
+  c.s = fma_(-qw, fma_(w, t2, t1), A);                     // RPY's A + f1, the -q of f1 taken off above
   T t3 = fma_(T(-6), zz, fma_(T(10), E, T(-2)));
   T t4 = fma_(T(-70.0 / 3.0), E, T(10.0 / 3.0));
-  T qw = q * w;
-  c.g2 = -qw * fma_(w, fma_(w, t4, t3), one);              // f2 w
-  T Rzw = g.Rz * w;
-  T t5 = fma_(T(-12), zz, fma_(T(20), E, T(-4)));
-  T t6 = fma_(T(-140.0 / 3.0), E, T(40.0 / 3.0));
-  T two_zj = zj + zj;
-  c.g3 = qw * fma_(Rzw, fma_(w, t6, t5), two_zj);          // f3 q
-  c.g4 = qw * fma_(T(-20.0 / 3.0) * Rzw, w, two_zj);       // f4 q
-  T t7 = fma_(T(-20), E, T(8.0 / 3.0));
-  T t8 = fma_(T(4) * zj, zj, T(4) * E);
-  T f5 = -qw * fma_(w, t7, t8);
-  c.s = A + f1;
-  c.s5 = c.s + f5;
+  T P = fma_(w, t4, t3);
+  c.g2 = -qw * fma_(w, P, one);                            // f2 w
+  T c2 = qw + qw;
+  T m = T(10.0 / 3.0) * b * w;
+  c.g3 = c2 * fma_(b, P, zj + m);                          // f3 q
+  c.g4 = c2 * (zj - m);                                    // f4 q
+  T t7 = fma_(T(-5), E, T(2.0 / 3.0));
+  T t8 = fma_(zj, zj, E);
+  c.s5 = fma_(T(-2) * c2, fma_(w, t7, t8), c.s);           // + f5
   return c;
 }
 
-template <typename T>
-RMW_HD Vec3<T> apply_uf(const Geom<T>& g, const CoefUF<T>& c, T vx, T vy, T vz)
+// The products below come in two forms: M v, and (ADD) acc + M v with acc
+// entering the FMA chain, which saves the separate add of every component.
+template <bool ADD, typename T>
+RMW_HD T fma_or_mul(T a, T b, T acc) { return ADD ? fma_(a, b, acc) : a * b; }
+
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_uf(const Geom<T>& g, const CoefUF<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T p = g.dx * vx + g.dy * vy;
-  T dv = p + g.dz * vz;          // d.v
-  T Rv = p + g.Rz * vz;          // R.v
-  T ge = c.g2 * Rv + c.g3 * vz;  // coefficient of R
-  T q = c.Bc * dv;               // coefficient of d
-  T qe = q + ge;                 // x and y rows share d_x = R_x, d_y = R_y
+  T p = fma_(g.dx, vx, g.dy * vy);
+  T dv = fma_(g.dz, vz, p);        // d.v
+  T Rv = fma_(g.Rz, vz, p);        // R.v
+  T ge = fma_(c.g2, Rv, c.g3 * vz);  // coefficient of R
+  T q = c.Bc * dv;                 // coefficient of d
+  T qe = q + ge;                   // x and y rows share d_x = R_x, d_y = R_y
   Vec3<T> u;
-  u.x = c.s * vx + qe * g.dx;
-  u.y = c.s * vy + qe * g.dy;
-  u.z = c.s5 * vz + q * g.dz + ge * g.Rz + c.g4 * Rv;
+  u.x = fma_(c.s, vx, fma_or_mul<ADD>(qe, g.dx, acc.x));
+  u.y = fma_(c.s, vy, fma_or_mul<ADD>(qe, g.dy, acc.y));
+  u.z = fma_(c.s5, vz, fma_(q, g.dz, fma_(ge, g.Rz, fma_or_mul<ADD>(c.g4, Rv, acc.z))));
   return u;
 }
 
 // Transposed block: UF_ij^T v, which is UF_ji v (the mobility is symmetric),
 // so one evaluation of a pair serves both of its blobs.  The coefficients of
 // v_z R and (R.v) z trade places.
-template <typename T>
-RMW_HD Vec3<T> apply_uf_t(const Geom<T>& g, const CoefUF<T>& c, T vx, T vy, T vz)
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_uf_t(const Geom<T>& g, const CoefUF<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T p = g.dx * vx + g.dy * vy;
-  T dv = p + g.dz * vz;
-  T Rv = p + g.Rz * vz;
-  T ge = c.g2 * Rv + c.g4 * vz;
+  T p = fma_(g.dx, vx, g.dy * vy);
+  T dv = fma_(g.dz, vz, p);
+  T Rv = fma_(g.Rz, vz, p);
+  T ge = fma_(c.g2, Rv, c.g4 * vz);
   T q = c.Bc * dv;
   T qe = q + ge;
   Vec3<T> u;
-  u.x = c.s * vx + qe * g.dx;
-  u.y = c.s * vy + qe * g.dy;
-  u.z = c.s5 * vz + q * g.dz + ge * g.Rz + c.g3 * Rv;
+  u.x = fma_(c.s, vx, fma_or_mul<ADD>(qe, g.dx, acc.x));
+  u.y = fma_(c.s, vy, fma_or_mul<ADD>(qe, g.dy, acc.y));
+  u.z = fma_(c.s5, vz, fma_(q, g.dz, fma_(ge, g.Rz, fma_or_mul<ADD>(c.g3, Rv, acc.z))));
   return u;
 }
 
@@ -274,101 +291,113 @@ template <typename T> struct CoefRot {
   T F4;   // F4
 };
 
+// RPY: c = 1/r^3 far, (1 - 3r/8)/2 overlapping: ic^3 + (3/8 - 3 rm/16).
+// Wall, for h = h_hat R_z, with q = 1/|R|, w = q^2, b = R_z w:
+//   F1 = w,  F4 = -2 w q (h - b),  F3 = -2 w q B,  F2 = 2 w^2 (1 + 2 R_z B),
+//   B = 3 h - 5 b   (h_hat e_z^2 = h b and h_hat e_z = h q: no division).
 template <typename T>
 RMW_HD CoefRot<T> coef_rot(const Geom<T>& g, T hnum, int dom = kDomWall)
 {
-  const T one = T(1), two = T(2);
   CoefRot<T> c;
-  T invr3 = g.invr * g.invr * g.invr;
-  T c_near = T(0.5) * (one - T(0.375) * g.r);
-  c.c = (g.r >= two) ? invr3 : c_near;
+  c.c = fma_(g.ic * g.ic, g.ic, fma_(T(-0.1875), g.rm, T(0.375)));
   if (!dom_has_wall(dom)) {
     c.F1r = T(0); c.F2r = T(0); c.F3r2 = T(0); c.F4 = T(0);
     return c;
   }
-  // h_hat = h/R_z enters only as h_hat e_z^2 = h R_z/|R|^2 and
-  // h_hat e_z = h/|R| (no division needed).
-  T invR = g.invR;
-  T invR2 = invR * invR;
-  T invR4 = invR2 * invR2;
-  T ez2 = g.ez2;
-  T F1 = invR2;
-  T F2 = (T(6) * hnum * g.Rz + one - T(10) * ez2) * invR4 * two;
-  T F3 = -(T(3) * hnum * invR * invR2 - T(5) * g.ez * invR4) * two;
-  T F4 = -(hnum * invR * invR2 - g.ez * invR4) * two;
-  c.F1r = F1 * invR;
-  c.F2r = F2 * invR;
-  c.F3r2 = F3 * invR2;
-  c.F4 = F4;
+  T q = g.invR;
+  T w = q * q;
+  T b = g.Rz * w;
+  T qw = q * w;
+  T c2 = qw + qw;
+  T c2w = c2 * w;
+  T B = fma_(T(-5), b, T(3) * hnum);
+  c.F1r = qw;
+  c.F3r2 = -c2w * B;
+  c.F2r = fma_(T(-2) * g.Rz, c.F3r2, c2w);
+  c.F4 = c2 * (b - hnum);
   return c;
 }
 
-// WF v = c (v x d) - [F1 (v x e) + (F2 v_z + F3 (e.v)) (z x e) + F4 (v x z)]
-template <typename T>
-RMW_HD Vec3<T> apply_wf(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz)
+// WF v = c (v x d) - [F1 (v x e) + (F2 v_z + F3 (e.v)) (z x e) + F4 (v x z)]:
+//   x =  G v_y + (h - k v_z) d_y,   y = -G v_x - (h - k v_z) d_x,
+//   z =  k (v_x d_y - v_y d_x)
+// with G = c d_z - F1 R_z/|R| - F4, k = c - F1/|R| and
+// h = F2 v_z/|R| + F3 (R.v)/|R|^2.
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_wf(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T Rv = g.dx * vx + g.dy * vy + g.Rz * vz;
-  T h = c.F2r * vz + c.F3r2 * Rv;           // (F2 v_z + F3 e.v) / |R|
-  T zc = vx * g.dy - vy * g.dx;              // (v x d)_z = (v x R)_z
+  T Rv = fma_(g.dx, vx, fma_(g.dy, vy, g.Rz * vz));
+  T G = fma_(c.c, g.dz, -fma_(c.F1r, g.Rz, c.F4));
+  T k = c.c - c.F1r;
+  T h = fma_(c.F3r2, Rv, (c.F2r - k) * vz);
+  T zc = fma_(vx, g.dy, -(vy * g.dx));       // (v x d)_z = (v x R)_z
   Vec3<T> w;
-  w.x = c.c * (vy * g.dz - vz * g.dy) - c.F1r * (vy * g.Rz - vz * g.dy) + h * g.dy - c.F4 * vy;
-  w.y = c.c * (vz * g.dx - vx * g.dz) - c.F1r * (vz * g.dx - vx * g.Rz) - h * g.dx + c.F4 * vx;
-  w.z = (c.c - c.F1r) * zc;
+  w.x = fma_(G, vy, fma_or_mul<ADD>(h, g.dy, acc.x));
+  w.y = fma_(-G, vx, fma_or_mul<ADD>(-h, g.dx, acc.y));
+  w.z = fma_or_mul<ADD>(k, zc, acc.z);
   return w;
 }
 
 // UT v = c (v x d) - [F1 (e' x v) + (F2 z + F3 e') ((z x e').v) + F4 (z x v)],
-// e' = (-d_x, -d_y, R_z)/|R|, coefficients built with h_hat = z_i / R_z.
-template <typename T>
-RMW_HD Vec3<T> apply_ut(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz)
+// e' = (-d_x, -d_y, R_z)/|R|, coefficients built with h_hat = z_i / R_z:
+//   x =  G v_y - k d_y v_z + m d_x,   y = -G v_x + k d_x v_z + m d_y,
+//   z = (k - F2/|R|) q - m R_z
+// with G = c d_z + F1 R_z/|R| + F4, k = c - F1/|R|, q = d_y v_x - d_x v_y
+// (= |R| (z x e').v) and m = F3 q/|R|^2.
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_ut(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T q = g.dy * vx - g.dx * vy;               // |R| (z x e').v
-  T m3 = c.F3r2 * q;                          // F3 ((z x e').v) / |R|
+  T q = fma_(g.dy, vx, -(g.dx * vy));
+  T m = c.F3r2 * q;
+  T G = fma_(c.c, g.dz, fma_(c.F1r, g.Rz, c.F4));
+  T k = c.c - c.F1r;
+  T kv = k * vz;
   Vec3<T> u;
-  u.x = c.c * (vy * g.dz - vz * g.dy) + c.F1r * (g.dy * vz + g.Rz * vy) + m3 * g.dx + c.F4 * vy;
-  u.y = c.c * (vz * g.dx - vx * g.dz) - c.F1r * (g.Rz * vx + g.dx * vz) + m3 * g.dy - c.F4 * vx;
-  u.z = (c.c - c.F1r - c.F2r) * q - m3 * g.Rz;
+  u.x = fma_(G, vy, fma_(m, g.dx, fma_or_mul<ADD>(-kv, g.dy, acc.x)));
+  u.y = fma_(-G, vx, fma_(m, g.dy, fma_or_mul<ADD>(kv, g.dx, acc.y)));
+  u.z = fma_(k - c.F2r, q, fma_or_mul<ADD>(-m, g.Rz, acc.z));
   return u;
 }
 
 // Transposes of the rotational couplings, read off the component forms
 // above.  Reciprocity gives UT_ji = WF_ij^T and WF_ji = UT_ij^T, so with
 // the coefficients of the pair (i, j) these are the blocks of (j, i).
-// WF_ij^T v, with p = d_x v_x + d_y v_y, q = d_y v_x - d_x v_y:
-//   x = F3 d_x q / |R|^2 + (F1 R_z / |R| - c d_z + F4) v_y + (c - F1/|R|) d_y v_z
-//   y = F3 d_y q / |R|^2 - (F1 R_z / |R| - c d_z + F4) v_x - (c - F1/|R|) d_x v_z
-//   z = (F1/|R| + F2/|R| + F3 R_z/|R|^2 - c) q
-template <typename T>
-RMW_HD Vec3<T> apply_wf_t(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz)
+// WF_ij^T v, with G and k of WF, q = d_y v_x - d_x v_y and m = F3 q/|R|^2:
+//   x = m d_x - G v_y + k d_y v_z,   y = m d_y + G v_x - k d_x v_z,
+//   z = (F2/|R| + F3 R_z/|R|^2 - k) q
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_wf_t(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T q = g.dy * vx - g.dx * vy;
-  T m3 = c.F3r2 * q;
-  T G = c.F1r * g.Rz - c.c * g.dz + c.F4;
-  T cf = c.c - c.F1r;
+  T q = fma_(g.dy, vx, -(g.dx * vy));
+  T m = c.F3r2 * q;
+  T G = fma_(c.c, g.dz, -fma_(c.F1r, g.Rz, c.F4));
+  T k = c.c - c.F1r;
+  T kv = k * vz;
   Vec3<T> w;
-  w.x = m3 * g.dx + G * vy + cf * g.dy * vz;
-  w.y = m3 * g.dy - G * vx - cf * g.dx * vz;
-  w.z = (c.F1r + c.F2r + c.F3r2 * g.Rz - c.c) * q;
+  w.x = fma_(-G, vy, fma_(m, g.dx, fma_or_mul<ADD>(kv, g.dy, acc.x)));
+  w.y = fma_(G, vx, fma_(m, g.dy, fma_or_mul<ADD>(-kv, g.dx, acc.y)));
+  w.z = fma_or_mul<ADD>(fma_(c.F3r2, g.Rz, c.F2r - k), q, acc.z);
   return w;
 }
 
-// UT_ij^T v:
-//   x =  F3 d_y p / |R|^2 - G v_y + K d_y v_z
-//   y = -F3 d_x p / |R|^2 + G v_x - K d_x v_z
-//   z = (F1/|R| - c) q
-// with G = c d_z + F1 R_z / |R| + F4 and K = c - F1/|R| - F2/|R| - F3 R_z/|R|^2.
-template <typename T>
-RMW_HD Vec3<T> apply_ut_t(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz)
+// UT_ij^T v, with G and k of UT, p = d_x v_x + d_y v_y, q as above and
+// K = k - F2/|R| - F3 R_z/|R|^2:
+//   x =  F3 d_y p/|R|^2 - G v_y + K d_y v_z
+//   y = -F3 d_x p/|R|^2 + G v_x - K d_x v_z
+//   z = -k q
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_ut_t(const Geom<T>& g, const CoefRot<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T p = g.dx * vx + g.dy * vy;
-  T q = g.dy * vx - g.dx * vy;
-  T m3 = c.F3r2 * p;
-  T G = c.c * g.dz + c.F1r * g.Rz + c.F4;
-  T K = c.c - c.F1r - c.F2r - c.F3r2 * g.Rz;
+  T p = fma_(g.dx, vx, g.dy * vy);
+  T q = fma_(g.dy, vx, -(g.dx * vy));
+  T G = fma_(c.c, g.dz, fma_(c.F1r, g.Rz, c.F4));
+  T k = c.c - c.F1r;
+  T K = k - fma_(c.F3r2, g.Rz, c.F2r);
+  T m = fma_(c.F3r2, p, K * vz);
   Vec3<T> u;
-  u.x = m3 * g.dy - G * vy + K * g.dy * vz;
-  u.y = -m3 * g.dx + G * vx - K * g.dx * vz;
-  u.z = (c.F1r - c.c) * q;
+  u.x = fma_(-G, vy, fma_or_mul<ADD>(m, g.dy, acc.x));
+  u.y = fma_(G, vx, fma_or_mul<ADD>(-m, g.dx, acc.y));
+  u.z = fma_or_mul<ADD>(-k, q, acc.z);
   return u;
 }
 
@@ -383,71 +412,69 @@ template <typename T> struct CoefWT {
   T G4r;  // G4 / |R|^2 -> ((z x R).v)(z x R)
 };
 
+// RPY:  far      A = -1/(2 r^3),                  B = 3/(2 r^5)
+//       overlap  A = 1 - 27 r/32 + 5 r^3/64,      B = 9/(32 r) - 3 r/64
+// A = -ic^3/2 + (17/16 + rm (-27/32 + 5 rm^2/64)),
+// B = (3 ic^4/2 + (3/16 - 3 rm^2/64)) / r.
+// Wall, with q = 1/|R|, w = q^2: G1 = (1 - 6 e_z^2) q^3/2, G2 = -3 q^3/2,
+// G3 = 3 q^3 e_z, G4 = 3 q^3.
 template <typename T>
 RMW_HD CoefWT<T> coef_wt(const Geom<T>& g, int dom = kDomWall)
 {
-  const T one = T(1), two = T(2);
   CoefWT<T> c;
-  T invr2 = g.invr * g.invr;
-  T invr3 = invr2 * g.invr;
-  T r3 = g.r2 * g.r;
-  T A_far = T(-0.5) * invr3;
-  T B_far = T(1.5) * invr2 * invr3;
-  T A_near = one - T(0.84375) * g.r + T(0.078125) * r3;
-  T B_near = T(0.28125) * g.invr - T(0.046875) * g.r;
-  bool far = g.r >= two;
-  T A = far ? A_far : A_near;
-  c.Bc = far ? B_far : B_near;
+  T w2 = g.ic * g.ic;
+  T m2 = g.rm * g.rm;
+  T A = fma_(T(-0.5) * w2, g.ic, fma_(fma_(T(0.078125), m2, T(-0.84375)), g.rm, T(1.0625)));
+  c.Bc = fma_(T(1.5) * w2, w2, fma_(T(-0.046875), m2, T(0.1875))) * g.invr;
   if (!dom_has_wall(dom)) {
     c.s = A; c.G2r = T(0); c.G3r = T(0); c.G4r = T(0);
     return c;
   }
-  T invR = g.invR;
-  T invR2 = invR * invR;
-  T invR3 = invR2 * invR;
-  T G1 = (one - T(6) * g.ez2) * invR3 * T(0.5);
-  T G2 = T(-1.5) * invR3;
-  T G3 = T(3) * invR3 * g.ez;
-  T G4 = T(3) * invR3;
-  c.s = A + G1;
-  c.G2r = G2 * invR2;
-  c.G3r = G3 * invR;
-  c.G4r = G4 * invR2;
+  T q = g.invR;
+  T w = q * q;
+  T b = g.Rz * w;
+  T qw = q * w;
+  c.s = fma_(qw, fma_(T(-3) * g.Rz, b, T(0.5)), A);
+  c.G4r = T(3) * qw * w;
+  c.G2r = T(-0.5) * c.G4r;
+  c.G3r = T(3) * qw * b;
   return c;
 }
 
-template <typename T>
-RMW_HD Vec3<T> apply_wt(const Geom<T>& g, const CoefWT<T>& c, T vx, T vy, T vz)
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_wt(const Geom<T>& g, const CoefWT<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T p = g.dx * vx + g.dy * vy;
-  T dv = p + g.dz * vz;
-  T Rv = p + g.Rz * vz;
-  T zt = g.dx * vy - g.dy * vx;      // (z x R).v
+  T p = fma_(g.dx, vx, g.dy * vy);
+  T dv = fma_(g.dz, vz, p);
+  T Rv = fma_(g.Rz, vz, p);
+  T zt = fma_(g.dx, vy, -(g.dy * vx));   // (z x R).v
   T q = c.Bc * dv;
   T ge = c.G2r * Rv;
+  T qe = q + ge;
   T gz = c.G4r * zt;
   Vec3<T> w;
-  w.x = c.s * vx + (q + ge) * g.dx - gz * g.dy;
-  w.y = c.s * vy + (q + ge) * g.dy + gz * g.dx;
-  w.z = c.s * vz + q * g.dz + ge * g.Rz + c.G3r * Rv;
+  w.x = fma_(c.s, vx, fma_(qe, g.dx, fma_or_mul<ADD>(-gz, g.dy, acc.x)));
+  w.y = fma_(c.s, vy, fma_(qe, g.dy, fma_or_mul<ADD>(gz, g.dx, acc.y)));
+  w.z = fma_(c.s, vz, fma_(q, g.dz, fma_(ge, g.Rz, fma_or_mul<ADD>(c.G3r, Rv, acc.z))));
   return w;
 }
 
 // WT_ij^T v = WT_ji v: the (R.v) z term becomes v_z R.
-template <typename T>
-RMW_HD Vec3<T> apply_wt_t(const Geom<T>& g, const CoefWT<T>& c, T vx, T vy, T vz)
+template <bool ADD = false, typename T>
+RMW_HD Vec3<T> apply_wt_t(const Geom<T>& g, const CoefWT<T>& c, T vx, T vy, T vz, const Vec3<T>& acc = Vec3<T>{})
 {
-  T p = g.dx * vx + g.dy * vy;
-  T dv = p + g.dz * vz;
-  T Rv = p + g.Rz * vz;
-  T zt = g.dx * vy - g.dy * vx;
+  T p = fma_(g.dx, vx, g.dy * vy);
+  T dv = fma_(g.dz, vz, p);
+  T Rv = fma_(g.Rz, vz, p);
+  T zt = fma_(g.dx, vy, -(g.dy * vx));
   T q = c.Bc * dv;
-  T ge = c.G2r * Rv + c.G3r * vz;
+  T ge = fma_(c.G2r, Rv, c.G3r * vz);
+  T qe = q + ge;
   T gz = c.G4r * zt;
   Vec3<T> w;
-  w.x = c.s * vx + (q + ge) * g.dx - gz * g.dy;
-  w.y = c.s * vy + (q + ge) * g.dy + gz * g.dx;
-  w.z = c.s * vz + q * g.dz + ge * g.Rz;
+  w.x = fma_(c.s, vx, fma_(qe, g.dx, fma_or_mul<ADD>(-gz, g.dy, acc.x)));
+  w.y = fma_(c.s, vy, fma_(qe, g.dy, fma_or_mul<ADD>(gz, g.dx, acc.y)));
+  w.z = fma_(c.s, vz, fma_(q, g.dz, fma_or_mul<ADD>(ge, g.Rz, acc.z)));
   return w;
 }
 
@@ -702,7 +729,7 @@ RMW_HD Vec3<T> self_uf_dom(int dom, T h, T vx, T vy, T vz)
   if (dom == kDomFreeSurface) {
     const T R = h + h;
     T AR, BR;
-    rpy_tt(R, T(1) / R, AR, BR);
+    rpy_tt(T(1) / R, min_(T(1) / R, T(0.5)), min_(R, T(2)), T(0), AR, BR);
     return Vec3<T>{(s + AR) * vx, (s + AR) * vy, (s - AR - R * R * BR) * vz};
   }
   return self_uf(h, vx, vy, vz);
