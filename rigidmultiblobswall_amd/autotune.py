@@ -26,8 +26,9 @@ whenever the caller passes no tuning.
 
   python -m rigidmultiblobswall_amd.autotune [--workloads c1,c2,c3,c4,c5] [--out FILE]
 
-writes the cache for the benchmark workloads (the package ships
-``tuning_gfx950.json`` made this way on an MI355X).  RMW_TUNING_FILE
+writes the cache for the benchmark workloads where a shape beats the
+built-in rule by 2 % or more (the package ships ``tuning_gfx950.json`` made
+this way on an MI355X).  RMW_TUNING_FILE
 selects another cache file; RMW_AUTOTUNE=off ignores every cache.
 """
 from __future__ import annotations
@@ -319,8 +320,14 @@ def main(argv=None):
         res = tune(mask, prec, r, offsets=off, k=k, eta=eta, a=a, reps=args.reps, log=log)
         key = cache_key(arch, mask, prec, k, res["pairs"], res["ragged"])
         entry = dict(res["best"], workload=label)
+        if entry["ms"] > 0.98 * entry["heuristic_ms"]:
+            # the built-in rule does as well, and it follows the size
+            log("  no entry: the built-in rule is within 2 %")
+            cache.entries.pop(key, None)
+            continue
         cache.store(key, entry)
         cache.save(path)
+    cache.save(path)
     log(f"wrote {path} ({len(cache.entries)} entries) in {time.perf_counter() - t0:.1f} s")
     return 0
 

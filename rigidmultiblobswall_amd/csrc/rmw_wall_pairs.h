@@ -28,6 +28,9 @@ enum : int { kUF = 1, kUT = 2, kWF = 4, kWT = 8 };
 __device__ __forceinline__ void scale_blob(double x, double y, double z, double a, double inva, double& X, double& Y,
                                            double& Z, double& B, int dom)
 {
+  // the scaled coordinates are rounded here: were the product fused into a
+  // later difference, blobs at one position would not be at distance 0
+#pragma clang fp contract(off)
   const bool wall = dom_has_wall(dom);
   const double ze = wall && z <= a ? a : z;
   X = x * inva;
@@ -41,6 +44,27 @@ __device__ __forceinline__ void load_blob(const double* __restrict__ r, int64_t 
 {
   scale_blob(r[3 * g], r[3 * g + 1], r[3 * g + 2], a, inva, X, Y, Z, B, dom);
 }
+
+// A blob's position and its K forces and torques as they lie in memory:
+// loaded ahead of their use, scaled when they are staged.
+template <int K, bool NF, bool NT>
+struct RawBlob {
+  double r[3];
+  double f[NF ? K : 1][3], t[NT ? K : 1][3];
+  __device__ __forceinline__ void load(const double* __restrict__ rr, const double* __restrict__ ff,
+                                       const double* __restrict__ tt, int64_t stride, int64_t g)
+  {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r[c] = rr[3 * g + c];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if constexpr (NF) f[k][c] = ff[k * stride + 3 * g + c];
+        if constexpr (NT) t[k][c] = tt[k * stride + 3 * g + c];
+      }
+  }
+};
 
 template <int K, int ACC>
 __device__ __forceinline__ void flush_all(Acc<ACC> (&u)[K][3], Acc<ACC> (&w)[K][3])
@@ -340,5 +364,40 @@ __device__ __forceinline__ void finish_output(const double* __restrict__ r, cons
     omg[k * rhs_stride + 3 * gi + comp] = B * inva * (sum + self);
   }
 }
+
+// ---------------------------------------------------------------------------
+// Launches of the kernels for few blobs (rmw_wall_direct.hip) and for the
+// middle sizes (rmw_wall_blocks.hip).
+// ---------------------------------------------------------------------------
+// One independent suspension of a direct launch.
+struct DirectSys {
+  int64_t b0, n;        // first blob, blobs
+  int64_t item0;        // first workgroup
+};
+
+struct DirectParams {
+  const double* r;
+  const double* f;          // K right-hand sides rhs_stride apart, or null
+  const double* t;
+  double* vel;              // outputs, same stride, or null
+  double* omg;
+  int64_t rhs_stride;
+  double a, inva, c1, c2;
+  const DirectSys* table;   // nullptr -> single
+  DirectSys single;
+  int nsys;
+  int periodic;             // bit d set when L_d > 0
+  double L[3];              // periodic lengths / a
+};
+
+// Targets per workgroup of the direct kernel for these blocks and
+// right-hand sides, and the largest number of right-hand sides per launch.
+int direct_targets(int mask, int K);
+int direct_max_k(int mask, int domain);
+void launch_direct(int domain, int mask, int prec, int K, const DirectParams& q, int64_t wgs, hipStream_t st);
+
+// Symmetric kernel on pairs of 64-blob blocks; q counts tiles and work
+// items in blocks (MutSys::n_t, MutParams::chunk_blocks).
+void launch_blocks(int domain, int mask, int prec, int K, const MutParams& q, int grid, hipStream_t st);
 
 }  // namespace rmw

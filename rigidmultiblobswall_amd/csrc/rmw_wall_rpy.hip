@@ -730,7 +730,9 @@ constexpr int kRedGroups = 8, kRedOut = 256 / kRedGroups;
 // image loop takes 168 VGPRs, so calls without images run an instantiation
 // without it (70 VGPRs: seven waves per SIMD instead of three for this
 // latency-bound loop).
-template <bool PER>
+// BS: blobs per tile of the pair kernel (256, or the 64-blob blocks of
+// rmw_wall_blocks.hip, whose work items are runs of chunk_blocks tiles).
+template <bool PER, int BS>
 __global__ __launch_bounds__(256) void mutual_reduce_kernel(MutReduceParams p)
 {
   __shared__ double part[kRedGroups][kRedOut];
@@ -760,12 +762,14 @@ __global__ __launch_bounds__(256) void mutual_reduce_kernel(MutReduceParams p)
       Sy = p.table[lo];
     }
     const int64_t il = gi - Sy.b0;
-    const int64_t X = il / kBlock, l = il - X * kBlock;
-    const int64_t it0 = items_before_blocks(X, Sy.n_t, p.chunk_blocks);
-    const int64_t it1 = items_before_blocks(X + 1, Sy.n_t, p.chunk_blocks);
-    const int64_t step = (int64_t)p.K * kBlock * OC;
-    const double* Pi = p.part_i + (((Sy.pi0 + it0) * p.K + k) * kBlock + l) * OC + c;
-    const double* Pj = p.part_j + (((Sy.pj0 + tri_index(X, 0)) * p.K + k) * kBlock + l) * OC + c;
+    const int64_t X = il / BS, l = il - X * BS;
+    auto before = [&](int64_t x) {
+      return BS == kBlock ? items_before_blocks(x, Sy.n_t, p.chunk_blocks) : items_before(x, Sy.n_t, p.chunk_blocks);
+    };
+    const int64_t it0 = before(X), it1 = before(X + 1);
+    const int64_t step = (int64_t)p.K * BS * OC;
+    const double* Pi = p.part_i + (((Sy.pi0 + it0) * p.K + k) * BS + l) * OC + c;
+    const double* Pj = p.part_j + (((Sy.pj0 + tri_index(X, 0)) * p.K + k) * BS + l) * OC + c;
     // four loads in flight per thread (the loop is latency-bound: one
     // dependent load per slot took ~2x longer at 32768 blobs)
     auto strided_sum = [&](const double* P, int64_t cnt) {
@@ -851,8 +855,14 @@ class SmallVec {
   size_t n_ = 0;
 };
 
+// Kernels a plan runs: the ordered kernel (source chunks, two launches), the
+// symmetric kernel on 256-blob tiles or on 64-blob blocks, or the direct
+// kernel (one launch).
+enum : int { kOrderedPath, kTilesPath, kBlocksPath, kDirectPath };
+
 struct Plan {
   int domain = kDomWall;
+  int path = kOrderedPath;
   int mask = 0, prec = 0, kmax = 1;
   int slots = 0;             // resident pair-kernel workgroups on the device
   int64_t ntot = 0;
@@ -860,12 +870,16 @@ struct Plan {
   int64_t total_items = 0;
   size_t partial_doubles = 0;
   size_t off_partial = 0, off_table = 0, total = 0;
-  // symmetric path (UF or all four blocks, no periodic images)
-  bool mut_ok = false;
+  // symmetric paths
   int kmax_mut = 1;
   int64_t mut_items = 0, chunk_blocks = 4;   // symmetric work item: chunk_blocks 64-source blocks
   SmallVec<MutSys> msys;     // non-empty systems only
   size_t off_pi = 0, off_pj = 0, off_mtable = 0;
+  // direct path
+  int kmax_direct = 1;
+  SmallVec<DirectSys> dsys;  // non-empty systems only
+  int64_t direct_wgs = 0;
+  size_t off_dtable = 0;
   // RMW_FLAG_CHECK_FINITE: a counter of non-finite outputs after the rest
   bool check_finite = false;
   size_t off_status = 0;
@@ -950,11 +964,63 @@ static int64_t default_chunk(double pairs, int cu_count)
   return std::max<int64_t>(kBlock, (int64_t)std::ceil(c / kChunkQuantum) * kChunkQuantum);
 }
 
+// Blocks with a symmetric kernel: the UF block alone, UF + UT, the single UT,
+// WF and WT blocks (UT_ji = WF_ij^T, WT_ji = WT_ij^T: a pair's source side
+// of one of them is the transposed other) and all four, as far as the
+// boundary serves them (the free surface: UF only; in plane: UF, UT, UF +
+// UT); several right-hand sides per pass for UF and all four blocks above
+// the wall, one otherwise.
+static bool symmetric_mask(int mask, int domain)
+{
+  const bool single_rot = mask == kUT || mask == kWF || mask == kWT;
+  return mask == kUF || ((mask == (kUF | kUT) || single_rot) && domain != kDomFreeSurface) ||
+         (mask == (kUF | kUT | kWF | kWT) && (domain == kDomWall || domain == kDomNoWall));
+}
+
+// Ordered pairs up to which one direct launch is taken: the symmetric
+// kernel on blocks evaluates half the pairs but takes two launches.  Measured
+// (direct against blocks, us per product): UF fp32_blocked 6.5 / 11.4 at 1024
+// blobs, 14.3 / 16.9 at 2048, 26.4 / 23.8 at 3000; FP64 17.9 / 20.8 and 34.3 /
+// 31.4 at 2048 and 3000; all four blocks 26.1 / 28.0 and 50.0 / 40.2; UF + UT
+// with nine images 39 / 59 at 1024, 99.6 / 96.9 at 2048.  Batches, whose
+// workgroups are more than fit at once, up to a quarter of that, counting
+// whole passes over 256 sources (all four blocks: 64 systems of 16 to 100
+// blobs 19.7 / 24.9, 32 of 203 to 381 blobs 42 / 31).
+constexpr double kDirectPairs = 2304.0 * 2304.0;
+
+// Mean suspension size (weighted by blobs) up to which the symmetric kernel
+// works on 64-blob blocks instead of 256-blob tiles.  Measured (blocks
+// against tiles with 64-source items, us): UF fp32_blocked 36 / 39 at 4200,
+// 55.2 / 54.2 at 6000, 133 / 129 at 10752; FP64 45 / 52, 77 / 81, 212 / 217;
+// all four blocks 59 / 71, 105 / 108, 279 / 281; four right-hand sides of
+// them 150 / 169 at 4200, 463 / 451 at 8192; UF + UT with images 478 / 574 at
+// 6151, 800 / 850 at 8192.
+static double block_kernel_blobs(int mask, int prec, int K, bool periodic)
+{
+  const bool light = K > 1 || (mask == kUF && prec != RMW_PREC_F64 && !periodic);
+  return light ? 5632.0 : 9216.0;
+}
+
+// Non-empty systems of a direct launch with tt targets per workgroup.
+static SmallVec<DirectSys> direct_table(const int64_t* offsets, int nsys, int tt, int64_t& wgs)
+{
+  SmallVec<DirectSys> table;
+  wgs = 0;
+  for (int s = 0; s < nsys; ++s) {
+    const int64_t n = offsets[s + 1] - offsets[s];
+    if (n == 0) continue;
+    table.push_back(DirectSys{offsets[s], n, wgs});
+    wgs += (n + tt - 1) / tt;
+  }
+  return table;
+}
+
 // offsets: host array of nsys + 1 blob offsets (offsets[0] = 0).  periodic:
 // the call has pseudo-periodic images (the symmetric wall kernels then take
 // one right-hand side per pass, so their partial sums are sized for one).
 static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int k,
-                      const rmw_tuning* tuning, bool ragged, int domain = kDomWall, bool periodic = false)
+                      const rmw_tuning* tuning, bool ragged, int domain = kDomWall, bool periodic = false,
+                      bool fine_blocks = true)
 {
   RMW_REQUIRE(valid_mask(mask), "mask must be a non-empty subset of UF|UT|WF|WT");
   RMW_REQUIRE(domain >= kDomWall && domain <= kDomFreeSurface, "unknown domain");
@@ -1010,82 +1076,109 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
   pl.total_items = item;
   pl.partial_doubles = (size_t)part;
 
-  // Symmetric layout, unless switched off: the UF block alone, UF + UT, the
-  // single UT, WF and WT blocks (UT_ji = WF_ij^T, WT_ji = WT_ij^T: a pair's
-  // source side of one of them is the transposed other) and all four
-  // blocks, as far as the boundary serves them (the free surface: UF only;
-  // in plane: UF, UT, UF + UT); several right-hand sides per pass for UF
-  // and all four blocks above the wall, one otherwise
+  // The path.  A tuning that names a launch shape (chunk_len, max_wgs or
+  // symmetric) gets the ordered or the tile kernel it was made for; the
+  // built-in choice goes by the number of ordered pairs.
+  const bool shaped = tuning && (tuning->chunk_len > 0 || tuning->max_wgs > 0 || tuning->symmetric != 0);
   const int sym = tuning ? tuning->symmetric : 0;
-  const bool single_rot = mask == kUT || mask == kWF || mask == kWT;
-  pl.mut_ok = (mask == kUF || ((mask == (kUF | kUT) || single_rot) && domain != kDomFreeSurface) ||
-               (mask == (kUF | kUT | kWF | kWT) && (domain == kDomWall || domain == kDomNoWall))) &&
-              pl.ntot > 0 && sym >= 0;
-  RMW_REQUIRE(!(sym > 0 && !pl.mut_ok),
+  const bool sym_mask = symmetric_mask(mask, domain);
+  RMW_REQUIRE(!(sym > 0 && !(sym_mask && pl.ntot > 0)),
               "symmetric evaluation needs the UF block alone, UF + UT, one of UT, WF, WT, or all four blocks");
-  int64_t tile_pairs = 0;
+  const bool sym_ok = sym_mask && pl.ntot > 0 && (!periodic || domain == kDomWall);
+  int64_t tile_pairs = 0, block_pairs = 0;
+  double direct_work = 0.0;   // pairs, with the idle threads of a system's last 256 sources
   for (int s = 0; s < nsys; ++s) {
+    const double n = (double)(offsets[s + 1] - offsets[s]);
+    direct_work += n * (nsys > 1 ? std::ceil(n / kBlock) * kBlock : n);
     const int64_t nt = (offsets[s + 1] - offsets[s] + kBlock - 1) / kBlock;
+    const int64_t nb = (offsets[s + 1] - offsets[s] + 63) / 64;
     tile_pairs += nt * (nt + 1) / 2;
+    block_pairs += nb * (nb + 1) / 2;
   }
-  // automatic choice: only with enough tile pairs to fill the device
-  if (pl.mut_ok && sym == 0) pl.mut_ok = tile_pairs >= device_props().cu_count;
-  size_t mut_total = 0;
-  if (pl.mut_ok) {
+  const int cu = std::max(device_props().cu_count, 1);
+  const int kgroup = periodic || domain != kDomWall || (mask != kUF && mask != 15) ? 1 : group_k(k, 4);
+  if (!shaped && direct_work <= (nsys > 1 ? 0.25 : 1.0) * kDirectPairs)
+    pl.path = kDirectPath;
+  else if (!shaped && sym_ok && fine_blocks &&
+           pairs <= block_kernel_blobs(mask, prec, kgroup, periodic) * (double)pl.ntot)
+    pl.path = kBlocksPath;
+  else if (sym_ok && (sym > 0 || (sym == 0 && tile_pairs >= cu)))
+    pl.path = kTilesPath;
+
+  size_t o = 0;
+  if (pl.path == kTilesPath || pl.path == kBlocksPath) {
     // up to 4 right-hand sides per pass (each pair's blocks formed once as
     // 3x3 matrices and applied to all of them), fewer when the tuning caps it
     const int rc = rhs_cap(tuning);
+    const bool single_rot = mask == kUT || mask == kWF || mask == kWT;
     pl.kmax_mut = domain == kDomWall && mask != (kUF | kUT) && !single_rot && !periodic
                       ? group_k(k, rc > 0 ? std::min(rc, 4) : 4)
                       : 1;
-    if (tuning && tuning->chunk_len > 0) {
+    const bool blk = pl.path == kBlocksPath;
+    const int64_t bs = blk ? 64 : kBlock;
+    if (blk) {
+      // runs of one source block while that leaves a CU fewer than 12 work
+      // items, then two (fewer target-side sums: UF fp32_blocked 141.6 ->
+      // 132.5 us at 10752 blobs), four for large batches; with images one
+      // up to twice that (478 against 501 us at 6151)
+      const int64_t fine = (periodic ? 36 : 12) * (int64_t)cu;
+      pl.chunk_blocks = block_pairs <= fine ? 1 : (block_pairs <= 144 * (int64_t)cu ? 2 : 4);
+    } else if (tuning && tuning->chunk_len > 0) {
       // 64 or 128 sources: a quarter or half of a tile pair per work item
       // (finer work for suspensions of few tiles); else whole source tiles
       const int64_t blocks = (tuning->chunk_len + 63) / 64;
       pl.chunk_blocks = blocks <= 2 ? blocks : (blocks + 3) / 4 * 4;
     } else {
-      const DeviceProps& dp = device_props();
-      pl.chunk_blocks = 4 * std::max<int64_t>(1, tile_pairs / (16 * (int64_t)std::max(dp.cu_count, 1)));
+      // quarter tiles while they balance the CUs better than they cost in
+      // partial sums, then half and whole tiles (us at 64 / 128 / 256 sources:
+      // UF fp32_blocked 129 / 139 / 152 at 10752 blobs, 618 / 575 / 589 at 24576,
+      // 1777 / 1694 / 1676 at 43008; four right-hand sides of all four blocks
+      // 882 / 866 / 967 at 12000, 6271 / 6089 / 6081 at 32768)
+      const int64_t quarter = (pl.kmax_mut > 1 ? 4 : 8) * (int64_t)cu + 64;
+      pl.chunk_blocks = tile_pairs <= quarter ? 1
+                        : tile_pairs <= 36 * (int64_t)cu ? 2
+                                                         : 4 * std::max<int64_t>(1, tile_pairs / (48 * (int64_t)cu));
     }
-    int64_t item = 0, pi = 0, pj = 0;
+    int64_t item = 0, pj = 0;
     for (int s = 0; s < nsys; ++s) {
       MutSys M;
       M.b0 = offsets[s];
       M.n = offsets[s + 1] - offsets[s];
       if (M.n == 0) continue;
-      M.n_t = (M.n + kBlock - 1) / kBlock;
+      M.n_t = (M.n + bs - 1) / bs;
       M.item0 = item;
-      M.pi0 = pi;
+      M.pi0 = item;
       M.pj0 = pj;
-      const int64_t its = items_before_blocks(M.n_t, M.n_t, pl.chunk_blocks);
-      item += its;
-      pi += its;
+      item += blk ? items_before(M.n_t, M.n_t, pl.chunk_blocks)
+                  : items_before_blocks(M.n_t, M.n_t, pl.chunk_blocks);
       pj += M.n_t * (M.n_t + 1) / 2;
       pl.msys.push_back(M);
     }
     pl.mut_items = item;
-    const int OCm = (mask & (kWF | kWT)) ? 6 : 3;
-    if (rc <= 0 && pl.kmax_mut > 2 &&
-        (size_t)(pi + pj) * pl.kmax_mut * kBlock * OCm * sizeof(double) > kMutAutoBytes)
+    const size_t slot = (size_t)bs * ((mask & (kWF | kWT)) && (mask & (kUF | kUT)) ? 6 : 3) * sizeof(double);
+    if (rc <= 0 && pl.kmax_mut > 2 && (size_t)(item + pj) * pl.kmax_mut * slot > kMutAutoBytes)
       pl.kmax_mut = group_k(k, 2);   // partial sums of 4 RHS too large: 2 per pass
-    size_t o = 0;
-    pl.off_pi = o; o = align_up(o + (size_t)pi * pl.kmax_mut * kBlock * OCm * sizeof(double));
-    pl.off_pj = o; o = align_up(o + (size_t)pj * pl.kmax_mut * kBlock * OCm * sizeof(double));
+    pl.off_pi = o; o = align_up(o + (size_t)item * pl.kmax_mut * slot);
+    pl.off_pj = o; o = align_up(o + (size_t)pj * pl.kmax_mut * slot);
     if (pl.msys.size() > 1) { pl.off_mtable = o; o = align_up(o + pl.msys.size() * sizeof(MutSys)); }
-    mut_total = o;
-    // the source-side slots grow as N^2 / kBlock: the automatic choice
-    // keeps them within kMutAutoBytes and uses the ordered kernel beyond
-    if (sym == 0 && mut_total > kMutAutoBytes) {
-      pl.mut_ok = false;
+    // the source-side slots grow as N^2: the automatic choice keeps them
+    // within kMutAutoBytes and uses the ordered kernel beyond
+    if (sym == 0 && o > kMutAutoBytes) {
+      pl.path = kOrderedPath;
       pl.msys.clear();
-      mut_total = 0;
+      o = 0;
     }
   }
-
-  size_t o = 0;
-  pl.off_partial = o; o = align_up(o + pl.partial_doubles * sizeof(double));
-  if (ragged) { pl.off_table = o; o = align_up(o + pl.sys.size() * sizeof(SysInfo)); }
-  pl.total = std::max(o, mut_total);
+  if (pl.path == kDirectPath) {
+    pl.kmax_direct = group_k(k, std::min(direct_max_k(mask, domain), rhs_cap(tuning) > 0 ? rhs_cap(tuning) : 4));
+    pl.dsys = direct_table(offsets, nsys, direct_targets(mask, pl.kmax_direct), pl.direct_wgs);
+    if (pl.dsys.size() > 1) { pl.off_dtable = o; o = align_up(o + pl.dsys.size() * sizeof(DirectSys)); }
+  }
+  if (pl.path == kOrderedPath) {
+    pl.off_partial = o; o = align_up(o + pl.partial_doubles * sizeof(double));
+    if (ragged) { pl.off_table = o; o = align_up(o + pl.sys.size() * sizeof(SysInfo)); }
+  }
+  pl.total = o;
   pl.check_finite = tuning && (tuning->flags & RMW_FLAG_CHECK_FINITE) != 0;
   if (pl.check_finite) {
     pl.off_status = align_up(pl.total);
@@ -1361,8 +1454,7 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
   }
   int grid = (int)std::min<int64_t>(pl.mut_items, (int64_t)INT32_MAX);
   if (tuning && tuning->max_wgs > 0) grid = std::min(grid, tuning->max_wgs);
-  // periodic images: one right-hand side per pass
-  const int kmax = periodic ? 1 : pl.kmax_mut;
+  const int kmax = pl.kmax_mut;
   for (int k0 = 0, K = group_k(k, kmax); k0 < k; k0 += K) {
     K = group_k(k - k0, kmax);
     MutParams q{};
@@ -1383,7 +1475,8 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st);
-    if (periodic) dispatch_mutual_periodic(pl.mask, pl.prec, q, grid, st);
+    if (pl.path == kBlocksPath) launch_blocks(pl.domain, pl.mask, pl.prec, K, q, grid, st);
+    else if (periodic) dispatch_mutual_periodic(pl.mask, pl.prec, q, grid, st);
     else dispatch_mutual(pl.domain, pl.mask, pl.prec, K, q, grid, st);
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
@@ -1410,11 +1503,65 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     const int OC = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
     const int64_t nout = pl.ntot * K * OC;
     const dim3 rgrid((unsigned)((nout + kRedOut - 1) / kRedOut));
-    if (periodic)
-      hipLaunchKernelGGL(mutual_reduce_kernel<true>, rgrid, dim3(256), 0, st, rp);
-    else
-      hipLaunchKernelGGL(mutual_reduce_kernel<false>, rgrid, dim3(256), 0, st, rp);
+    const dim3 rb(256);
+    if (pl.path == kBlocksPath) {
+      if (periodic) hipLaunchKernelGGL((mutual_reduce_kernel<true, 64>), rgrid, rb, 0, st, rp);
+      else hipLaunchKernelGGL((mutual_reduce_kernel<false, 64>), rgrid, rb, 0, st, rp);
+    } else {
+      if (periodic) hipLaunchKernelGGL((mutual_reduce_kernel<true, kBlock>), rgrid, rb, 0, st, rp);
+      else hipLaunchKernelGGL((mutual_reduce_kernel<false, kBlock>), rgrid, rb, 0, st, rp);
+    }
     RMW_CHECK_HIP(hipGetLastError());
+  }
+}
+
+static void run_direct(const Plan& pl, const double* r, const double* f, const double* t, double* vel, double* omg,
+                       int k, int64_t stride, double a, double inva, double c1, double c2, char* base, hipStream_t st,
+                       int periodic, const double* Lp)
+{
+  SmallVec<DirectSys> table = pl.dsys;
+  int64_t wgs = pl.direct_wgs;
+  DirectSys* dtable = nullptr;
+  auto upload = [&] {
+    if (table.size() > 1) {
+      dtable = (DirectSys*)(base + pl.off_dtable);
+      stage_upload(dtable, table.data(), table.size() * sizeof(DirectSys), st);
+    }
+  };
+  upload();
+  int tt = direct_targets(pl.mask, pl.kmax_direct);
+  for (int k0 = 0, K = pl.kmax_direct; k0 < k; k0 += K) {
+    K = group_k(k - k0, pl.kmax_direct);
+    if (direct_targets(pl.mask, K) != tt) {   // a smaller last group: more targets per workgroup
+      tt = direct_targets(pl.mask, K);
+      wgs = 0;
+      SmallVec<DirectSys> t2;
+      for (size_t s = 0; s < table.size(); ++s) {
+        t2.push_back(DirectSys{table[s].b0, table[s].n, wgs});
+        wgs += (table[s].n + tt - 1) / tt;
+      }
+      table = t2;
+      upload();
+    }
+    DirectParams q{};
+    q.r = r;
+    q.f = f ? f + (size_t)k0 * stride : nullptr;
+    q.t = t ? t + (size_t)k0 * stride : nullptr;
+    q.vel = vel ? vel + (size_t)k0 * stride : nullptr;
+    q.omg = omg ? omg + (size_t)k0 * stride : nullptr;
+    q.rhs_stride = stride;
+    q.a = a; q.inva = inva; q.c1 = c1; q.c2 = c2;
+    q.table = dtable;
+    q.single = table[0];
+    q.nsys = (int)table.size();
+    q.periodic = periodic;
+    for (int d = 0; d < 3; ++d) q.L[d] = Lp[d];
+    ProfRec rec{};
+    bool prof = false;
+    prof_begin(rec, prof, st);
+    launch_direct(pl.domain, pl.mask, pl.prec, K, q, wgs, st);
+    RMW_CHECK_HIP(hipGetLastError());
+    prof_end(rec, prof, st);
   }
 }
 
@@ -1492,7 +1639,13 @@ static void run_plan(const Plan& pl, const double* r, const double* f, const dou
   const double c2 = c1 / a;
 
   const int64_t stride = ld > 0 ? ld : 3 * pl.ntot;
-  if (pl.mut_ok && (periodic == 0 || pl.domain == kDomWall)) {
+  if (pl.path == kDirectPath) {
+    run_direct(pl, r, NF ? f : nullptr, NT ? t : nullptr, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, a, inva, c1,
+               c2, base, st, periodic, Lp);
+    check_outputs(pl, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, base, st);
+    return;
+  }
+  if (pl.path != kOrderedPath) {
     run_mutual(pl, r, f, t, vel, omg, k, stride, a, inva, c1, c2, tuning, base, st, periodic, Lp);
     check_outputs(pl, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, base, st);
     return;
@@ -1598,6 +1751,10 @@ static Plan plan_within(int mask, int prec, int64_t n, int k, const rmw_tuning* 
   const int64_t off[2] = {0, n};
   Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic);
   if (pl.total <= cap) return pl;
+  if (pl.path == kBlocksPath) {   // the tile kernel writes fewer partial sums
+    pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, false);
+    if (pl.total <= cap) return pl;
+  }
   const bool sym_required = tuning && tuning->symmetric > 0;
   if (!sym_required) {
     const int OC = 3 * (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0));
@@ -1651,11 +1808,11 @@ extern "C" int rmw_wall_rpy_describe(int mask, int prec, int64_t n, int k, const
     RMW_REQUIRE(n >= 0, "n must be >= 0");
     const int64_t off[2] = {0, n};
     Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic != 0);
-    const bool mut = pl.mut_ok && (!periodic || pl.domain == kDomWall);
+    const bool mut = pl.path == kTilesPath || pl.path == kBlocksPath, direct = pl.path == kDirectPath;
     info->symmetric = mut ? 1 : 0;
-    info->rhs_group = mut ? (periodic ? 1 : pl.kmax_mut) : pl.kmax;
-    info->chunk_len = mut ? pl.chunk_blocks * 64 : (pl.sys.empty() ? 0 : pl.sys[0].chunk_len);
-    info->work_items = mut ? pl.mut_items : pl.total_items;
+    info->rhs_group = mut ? pl.kmax_mut : (direct ? pl.kmax_direct : pl.kmax);
+    info->chunk_len = mut ? pl.chunk_blocks * 64 : (pl.sys.empty() ? 0 : (direct ? n : pl.sys[0].chunk_len));
+    info->work_items = mut ? pl.mut_items : (direct ? pl.direct_wgs : pl.total_items);
     info->workspace_bytes = (int64_t)pl.total;
   });
 }
@@ -1692,7 +1849,7 @@ extern "C" int rmw_wall_rpy_apply_noalloc(int mask, int prec, const double* r_ve
     // the plan may differ from the caller's tuning (longer ordered chunks);
     // run_plan reads only max_wgs and rhs_group from it
     rmw_tuning t = tuning ? *tuning : rmw_tuning{};
-    if (!pl.mut_ok) t.rhs_group = pl.kmax;
+    if (pl.path == kOrderedPath) t.rhs_group = pl.kmax;
     run_plan(pl, r_vectors, force, torque, velocity, omega, k, ld, eta, a, L, &t, scratch_address(),
              RMW_NOALLOC_SCRATCH_BYTES, (hipStream_t)stream, false);
   });
