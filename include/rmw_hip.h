@@ -269,10 +269,14 @@ int rmw_radii_self_apply(int prec, int boundary, const double* r_vectors, const 
  * as selected by set_blob_blob_forces, multi_bodies_functions.py:249-279.
  */
 int rmw_blob_forces_workspace_size(int prec, int64_t n, const rmw_tuning* tuning, size_t* bytes);
-/* Launch plan of rmw_blob_forces: symmetric (each unordered pair once, the
- * default when there are at least as many tile pairs as CUs and the
- * workspace stays within 2 GiB; tuning->symmetric 1 requires it, -1 turns
- * it off) or ordered, chunk length, work items, workspace bytes. */
+/* Launch plan of rmw_blob_forces over all pairs: symmetric (each unordered
+ * pair once, the default when there are at least as many tile pairs as CUs
+ * and the workspace stays within 2 GiB; tuning->symmetric 1 requires it, -1
+ * turns it off) or ordered, chunk length, work items, workspace bytes.
+ * Without a launch shape in the tuning, a few thousand blobs take one launch
+ * over all pairs (reported as ordered) and larger suspensions are sorted into
+ * cells of the force's range within the call; the plan reported is then the
+ * one for suspensions that the cells do not suit. */
 int rmw_blob_forces_describe(int prec, int64_t n, const rmw_tuning* tuning, rmw_plan_info* info);
 int rmw_blob_forces(int prec, const double* r_vectors, const double* radius_blobs, double* force, int64_t n,
                     double repulsion_strength, double debye_length, double blob_radius, double cutoff,

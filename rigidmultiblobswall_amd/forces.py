@@ -99,8 +99,8 @@ def calc_blob_blob_forces_radii_hip(r_vectors, radius_blobs, *args, precision: s
 
 def calc_blob_blob_forces_tree_hip(r_vectors, *args, precision: str = "fp32", **kwargs) -> np.ndarray:
     """Drop-in for calc_blob_blob_forces_tree_numba (forces_numba.py:200-241):
-    only pairs closer than d_max = 2a + 30b interact.  Every pair is
-    visited on the GPU, so no neighbour list is built or cached."""
+    only pairs closer than d_max = 2a + 30b interact.  Larger suspensions are
+    sorted into cells on the GPU within the call; nothing is cached."""
     k = _kw(kwargs)
     d_max = 2 * k["blob_radius"] + 30 * k["debye_length"]
     return blob_forces(np.asarray(r_vectors, dtype=np.float64), k["repulsion_strength"], k["debye_length"],

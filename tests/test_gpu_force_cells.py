@@ -1,0 +1,104 @@
+"""The blob forces by cells and in one launch, against the kernels over all
+pairs (which the other tests hold to the oracle): open and periodic boxes, the
+cutoff, different radii, boxes of few cells, blobs outside the box, dense
+suspensions, which fall back to all pairs, and positions that do not fit the
+cell arithmetic.
+
+Tolerances: the terms are the same, only the order of FP64 sums differs:
+1e-12; the FP32 exponential does not change that.
+"""
+import numpy as np
+import pytest
+import torch
+
+from rigidmultiblobswall_amd import _lib, forces
+
+pytestmark = pytest.mark.gpu
+
+ALL_PAIRS = _lib.Tuning(256, 0, 0, -1, 0)
+EPS, B, A = 0.3, 0.07, 0.6
+
+
+def _layout(n, seed, spread=1.6, flat=True):
+    rng = np.random.default_rng(seed)
+    m = int(np.ceil(n ** (0.5 if flat else 1 / 3)))
+    idx = rng.permutation(m ** (2 if flat else 3))[:n]
+    g = np.stack([idx % m, (idx // m) % m, idx // m ** 2 if not flat else 0 * idx], axis=1) * spread
+    return g + rng.uniform(-0.5, 0.5, (n, 3)) - 0.3 * m * spread      # about a third below zero
+
+
+def _rel(a, b):
+    return float(torch.linalg.vector_norm(a - b) / torch.linalg.vector_norm(b))
+
+
+def _check(r, what, L=None, cutoff=0.0, radii=None, b=B, tol=1e-12):
+    for prec in ("fp32", "fp64"):
+        print(f"case forces {what} n={r.shape[0]} L={L} cutoff={cutoff:.3g} {prec}", flush=True)
+        kw = dict(periodic_length=L, cutoff=cutoff, radius_blobs=radii, precision=prec)
+        got = forces.blob_forces(r, EPS, b, A, **kw)
+        ref = forces.blob_forces(r, EPS, b, A, tuning=ALL_PAIRS, **kw)
+        assert _rel(got, ref) <= tol, (what, prec, _rel(got, ref))
+        assert torch.equal(got, forces.blob_forces(r, EPS, b, A, **kw))   # the same sums every time
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 255, 257, 1000, 4096, 4097, 5003])
+def test_sizes(gpu, n):
+    if n > 1:
+        _check(_layout(n, n), "open")
+        _check(_layout(n, n, flat=False), "open 3d", cutoff=2 * A + 30 * B)
+    else:
+        assert bool((forces.blob_forces(_layout(1, 1), EPS, B, A) == 0).all())
+
+
+@pytest.mark.parametrize("n", [700, 6001])
+def test_periodic_boxes(gpu, n):
+    r = _layout(n, 3)
+    side = 1.6 * np.ceil(np.sqrt(n))
+    cut = 2 * A + 30 * B
+    # whole numbers of cells from 1 up, sides below and just above the range
+    for L in [(side, side, 0), (side, 0, 0), (0, side, 3.0), (3 * cut * 1.001, side, 0), (2.9 * cut, 4.05 * cut, 0),
+              (1.5 * cut, side, 2 * cut), (0, 0, 7 * cut)]:
+        _check(r, "periodic", L=np.array(L, dtype=float), cutoff=cut)
+    _check(r, "periodic, no cutoff", L=np.array([side, side, 0.0]))
+    shifted = r + np.random.default_rng(1).integers(-3, 4, r.shape) * np.array([side, side, 0.0])
+    _check(shifted, "outside the box", L=np.array([side, side, 0.0]), cutoff=cut)
+
+
+def test_radii_with_a_cutoff_and_without(gpu):
+    r = _layout(5000, 5)
+    rad = np.random.default_rng(6).uniform(0.3, 0.8, 5000)
+    _check(r, "radii, cutoff", cutoff=3.5, radii=rad)
+    _check(r, "radii", radii=rad)
+
+
+def test_dense_suspensions_take_all_pairs(gpu):
+    r = _layout(4500, 7, spread=0.05)
+    _check(r, "dense", b=1.0)
+    _check(np.vstack([r, r[:3]]), "dense with coincident blobs", b=1.0)
+    L = np.array([5.0, 5.0, 0.0])
+    _check(r, "dense periodic", L=L, b=1.0)
+
+
+def test_clusters_in_few_cells(gpu):
+    """Two clusters far apart: every blob in one of two cells (half of all
+    pairs), next to an otherwise empty suspension."""
+    rng = np.random.default_rng(8)
+    r = np.vstack([rng.uniform(0, 1.0, (2300, 3)), rng.uniform(0, 1.0, (2300, 3)) + 500.0])
+    _check(r, "two clusters", cutoff=3.0)
+    r[1::2] = _layout(2300, 9, spread=40.0)
+    _check(r, "cluster and dilute", cutoff=3.0)
+
+
+def test_positions_that_do_not_fit(gpu):
+    r = _layout(5000, 10)
+    far = r.copy()
+    far[17] = [1e12, -3e9, 5.0]
+    _check(far, "far blob")
+    _check(far, "far blob, periodic", L=np.array([200.0, 200.0, 0.0]), tol=1e-9)
+    for bad in (np.nan, np.inf):
+        x = r.copy()
+        x[4321, 1] = bad
+        for prec in ("fp32", "fp64"):
+            got = forces.blob_forces(x, EPS, B, A, precision=prec)
+            ref = forces.blob_forces(x, EPS, B, A, precision=prec, tuning=ALL_PAIRS)
+            assert bool((torch.isfinite(got) == torch.isfinite(ref)).all())
