@@ -470,6 +470,11 @@ int rmw_axpby(double alpha, const double* x, double beta, double* y, int64_t n, 
  * h[0..j] = coefficients, h[j+1] = ||w||, V[j+1] = w / ||w||. */
 int rmw_arnoldi_cgs2(double* V, int64_t ldv, int j, double* w, int64_t n, double* h,
                      double* hscratch, void* workspace, size_t workspace_bytes, void* stream);
+/* The same step for k bases in the same launches: basis r at V + r * v_rhs,
+ * its candidate at w + r * w_rhs, its coefficients at h + r * h_rhs. */
+int rmw_arnoldi_cgs2_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, double* w, int64_t w_rhs,
+                           int64_t n, double* h, int64_t h_rhs, double* hscratch, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Segmented (ragged-batch) FP64 Krylov kernels: the vector algebra of many
@@ -525,6 +530,12 @@ int rmw_lanczos_scratch_doubles(int m, int k, size_t* doubles);
 int rmw_lanczos_sqrt_coeffs(const double* H, int64_t h_rhs_stride, int64_t ldh, int m, int k,
                             const double* scale, double* c_out, int64_t c_stride, double* scratch,
                             size_t scratch_doubles, int* status, void* stream);
+/* The same with the numbers of the stop test (stochastic_forcing.py:241-251):
+ * on entry c_out holds the m - 1 coefficients of the step before; test (k, 3)
+ * gets |c - c_prev| and |c_prev| (c_prev padded with 0) and the status. */
+int rmw_lanczos_step_coeffs(const double* H, int64_t h_rhs_stride, int64_t ldh, int m, int k,
+                            const double* scale, double* c_out, int64_t c_stride, double* scratch,
+                            size_t scratch_doubles, double* test, void* stream);
 
 /* ------------------------------------------------------------------------
  * Learned GMRES warm start (no reference counterpart: the network only

@@ -149,6 +149,8 @@ PROTOTYPES = {
     "rmw_seg_dot_many": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _sgp, _dp, _i64, ctypes.c_int, _vp, _sz, _vp]),
     "rmw_seg_combination": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _i64, _dp, _sgp, ctypes.c_int, _vp]),
     "rmw_seg_scale": (ctypes.c_int, [_dp, _dp, _dp, _i64, _sgp, _vp]),
+    "rmw_arnoldi_cgs2_batch": (ctypes.c_int, [_dp, _i64, _i64, ctypes.c_int, ctypes.c_int, _dp, _i64, _i64, _dp, _i64,
+                                              _dp, _vp, _sz, _vp]),
     "rmw_seg_arnoldi_cgs2": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _sgp, _dp, _i64, _dp, _vp, _sz, _vp]),
     # learned warm start
     "rmw_gemm_bf16": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _dp, _i64,
@@ -175,6 +177,8 @@ PROTOTYPES = {
                                           ctypes.c_double, ctypes.c_int, _vp]),
     # Lanczos
     "rmw_lanczos_scratch_doubles": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _szp]),
+    "rmw_lanczos_step_coeffs": (ctypes.c_int, [_dp, _i64, _i64, ctypes.c_int, ctypes.c_int, _dp, _dp, _i64, _dp,
+                                               _sz, _dp, _vp]),
     "rmw_lanczos_sqrt_coeffs": (ctypes.c_int, [_dp, _i64, _i64, ctypes.c_int, ctypes.c_int, _dp, _dp, _i64, _dp,
                                                _sz, _vp, _vp]),
 }

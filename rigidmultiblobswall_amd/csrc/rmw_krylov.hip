@@ -154,6 +154,150 @@ __global__ void axpby_kernel(double alpha, const double* __restrict__ x, double 
   }
 }
 
+// ---------------------------------------------------------------------------
+// One Arnoldi step by CGS2 in four launches, for k independent bases at once
+// (blockIdx.y).  Every block owns one slice of kKBlock * E elements, the same
+// in all four, and adds the blocks' partial sums of the launch before it by
+// itself (a few thousand doubles from L2, in the order of dot_many_final), so
+// no launch in between turns partial sums into coefficients.  The chain of
+// small launches, not the vectors, was the time of the step: ten launches
+// took 35 us at n = 15000 with 11 vectors (13 MB read, 2.7 us at the rate of
+// a copy), these take 17.
+// ---------------------------------------------------------------------------
+struct ArnoldiParams {
+  double* V;            // basis r at V + r * v_rhs, vectors ldv apart
+  int64_t ldv, v_rhs;
+  double* w;            // candidate r at w + r * w_rhs
+  int64_t w_rhs, n;
+  double* h;            // coefficients r at h + r * h_rhs
+  int64_t h_rhs;
+  double* part;         // per basis: part1 [m][G], part2 [m][G], part3 [G]
+  int64_t part_rhs;
+  int m;                // vectors in the basis
+};
+
+// coef[j] = sum_g part[j * G + g], j < m: one wave per j at a time.
+__device__ __forceinline__ void block_coefs(const double* __restrict__ part, int G, int m, double* coef)
+{
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int j = wv; j < m; j += kKBlock / 64) {
+    double s = 0.0;
+    for (int g = lane; g < G; g += 64) s += part[(int64_t)j * G + g];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+    if (lane == 0) coef[j] = s;
+  }
+  __syncthreads();
+}
+
+// part[j * G + block] = V_j . w over this block's slice, w in registers.
+template <int E>
+__device__ __forceinline__ void block_dots(const double* __restrict__ V, int64_t ldv, int m, const double (&wr)[E],
+                                           int64_t base, int64_t n, double* __restrict__ part, int G)
+{
+  __shared__ double red[kDotGroup][kKBlock / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int j0 = 0; j0 < m; j0 += kDotGroup) {
+    const int jn = m - j0 < kDotGroup ? m - j0 : kDotGroup;
+#pragma unroll 4
+    for (int jj = 0; jj < jn; ++jj) {
+      const double* v = V + (int64_t)(j0 + jj) * ldv;
+      double acc = 0.0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int64_t i = base + (int64_t)e * kKBlock;
+        if (i < n) acc = fma(v[i], wr[e], acc);
+      }
+      for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+      if (lane == 0) red[jj][wv] = acc;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < jn) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < kKBlock / 64; ++k) s += red[threadIdx.x][k];
+      part[(int64_t)(j0 + threadIdx.x) * G + blockIdx.x] = s;
+    }
+    __syncthreads();
+  }
+}
+
+// PASS 0: part1 = V . w.  PASS 1: w -= V c1, h = c1, part2 = V . w.  PASS 2:
+// w -= V c2, h += c2, part3 = w . w.  PASS 3: V_m = w / |w| (e_0 if 0),
+// h_m = |w|.
+template <int E, int PASS>
+__global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
+{
+  __shared__ double coef[kMaxVec];
+  const int G = gridDim.x, r = blockIdx.y;
+  double* V = p.V + r * p.v_rhs;
+  double* w = p.w + r * p.w_rhs;
+  double* h = p.h + r * p.h_rhs;
+  double* part1 = p.part + r * p.part_rhs;
+  double* part2 = part1 + (int64_t)p.m * G;
+  double* part3 = part2 + (int64_t)p.m * G;
+  const int64_t base = (int64_t)blockIdx.x * (kKBlock * E) + threadIdx.x;
+  double wr[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int64_t i = base + (int64_t)e * kKBlock;
+    wr[e] = i < p.n ? w[i] : 0.0;
+  }
+  if constexpr (PASS == 0) {
+    block_dots<E>(V, p.ldv, p.m, wr, base, p.n, part1, G);
+  } else if constexpr (PASS == 3) {
+    block_coefs(part3, G, 1, coef);
+    const double norm = sqrt(coef[0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) h[p.m] = norm;
+    const double al = norm > 0.0 ? 1.0 / norm : 0.0;
+    double* v = V + (int64_t)p.m * p.ldv;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int64_t i = base + (int64_t)e * kKBlock;
+      if (i < p.n) v[i] = norm > 0.0 ? al * wr[e] : (i == 0 ? 1.0 : 0.0);
+    }
+  } else {
+    block_coefs(PASS == 1 ? part1 : part2, G, p.m, coef);
+    if (blockIdx.x == 0)
+      for (int j = threadIdx.x; j < p.m; j += kKBlock) h[j] = PASS == 1 ? coef[j] : h[j] + coef[j];
+#pragma unroll 4
+    for (int j = 0; j < p.m; ++j) {
+      const double* v = V + (int64_t)j * p.ldv;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int64_t i = base + (int64_t)e * kKBlock;
+        if (i < p.n) wr[e] -= coef[j] * v[i];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int64_t i = base + (int64_t)e * kKBlock;
+      if (i < p.n) w[i] = wr[e];
+    }
+    if constexpr (PASS == 1) {
+      block_dots<E>(V, p.ldv, p.m, wr, base, p.n, part2, G);
+    } else {
+      __shared__ double red[kKBlock / 64];
+      double acc = 0.0;
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc = fma(wr[e], wr[e], acc);
+      for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+      __syncthreads();
+      if (threadIdx.x == 0) part3[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+    }
+  }
+}
+
+template <int E>
+static void launch_arnoldi(const ArnoldiParams& p, int G, int k, hipStream_t st)
+{
+  const dim3 g(G, k), b(kKBlock);
+  hipLaunchKernelGGL((arnoldi_pass<E, 0>), g, b, 0, st, p);
+  hipLaunchKernelGGL((arnoldi_pass<E, 1>), g, b, 0, st, p);
+  hipLaunchKernelGGL((arnoldi_pass<E, 2>), g, b, 0, st, p);
+  hipLaunchKernelGGL((arnoldi_pass<E, 3>), g, b, 0, st, p);
+}
+
 // h[0..j] = h1 + h2 (CGS2 coefficients)
 __global__ void add_vec(const double* __restrict__ a, double* __restrict__ b, int m)
 {
@@ -213,7 +357,9 @@ extern "C" int rmw_krylov_workspace_size(int64_t n, int max_vectors, size_t* byt
 {
   return guarded([&] {
     RMW_REQUIRE(bytes && n >= 0 && max_vectors >= 1 && max_vectors <= kMaxVec, "bad arguments");
-    *bytes = align_up((size_t)kMaxDotBlocks * max_vectors * sizeof(double)) + align_up(kMaxVec * sizeof(double));
+    // two sets of partial sums of max_vectors and one of a norm (rmw_arnoldi_cgs2)
+    *bytes = align_up((size_t)kMaxDotBlocks * (2 * (size_t)max_vectors + 1) * sizeof(double)) +
+             align_up(kMaxVec * sizeof(double));
   });
 }
 
@@ -269,6 +415,62 @@ extern "C" int rmw_axpby(double alpha, const double* x, double beta, double* y, 
   });
 }
 
+// Partial sums that every block adds up by itself, at most: beyond (a basis of
+// many long vectors) turning them into coefficients once is cheaper.
+constexpr int64_t kSelfSums = 32768;
+
+// One CGS2 step of one basis in the launches of the separate operations.
+static void arnoldi_separate(const DotLaunch& L, hipStream_t st, double* V, int64_t ldv, int m, double* w, int64_t n,
+                             double* h, double* hscratch, double* partial)
+{
+  const int sb = stream_blocks(n);
+  // pass 1
+  launch_dot_partial(L, st, V, ldv, m, w, n, partial);
+  launch_dot_final(st, partial, L.G, m, h, 0, 0);
+  hipLaunchKernelGGL(sub_combination, dim3(sb), dim3(kKBlock), 0, st, V, ldv, m, h, w, n);
+  // pass 2 (re-orthogonalisation)
+  launch_dot_partial(L, st, V, ldv, m, w, n, partial);
+  launch_dot_final(st, partial, L.G, m, hscratch, 0, 0);
+  hipLaunchKernelGGL(sub_combination, dim3(sb), dim3(kKBlock), 0, st, V, ldv, m, hscratch, w, n);
+  hipLaunchKernelGGL(add_vec, dim3((m + 63) / 64), dim3(64), 0, st, hscratch, h, m);
+  // norm and normalisation
+  launch_dot_partial(L, st, w, (int64_t)0, 1, w, n, partial);
+  launch_dot_final(st, partial, L.G, 1, h + m, 0, 1);
+  hipLaunchKernelGGL(axpby_kernel, dim3(sb), dim3(kKBlock), 0, st, 1.0, w, 0.0, V + (int64_t)m * ldv, n,
+                     (const double*)(h + m));
+}
+
+static void arnoldi_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, double* w, int64_t w_rhs, int64_t n,
+                          double* h, int64_t h_rhs, double* hscratch, void* workspace, size_t workspace_bytes,
+                          hipStream_t st)
+{
+  const int m = j + 1;
+  RMW_REQUIRE(m >= 1 && m + 1 <= kMaxVec, "bad Arnoldi index");
+  RMW_REQUIRE(k >= 1 && k <= 65535, "bad number of bases");
+  const DotLaunch L = dot_launch(n);
+  RMW_REQUIRE(workspace_bytes >= (size_t)L.G * (m + 1) * sizeof(double), "workspace too small");
+  const int64_t per = (int64_t)L.G * (2 * m + 1);
+  if (L.E > 0 && (int64_t)L.G * m <= kSelfSums && workspace_bytes >= (size_t)per * sizeof(double)) {
+    // as many bases per launch as the workspace has partial sums for
+    const int fit = (int)std::min<int64_t>(k, (int64_t)(workspace_bytes / sizeof(double)) / per);
+    for (int r0 = 0; r0 < k; r0 += fit) {
+      ArnoldiParams p{V + r0 * v_rhs, ldv, v_rhs, w + r0 * w_rhs, w_rhs, n, h + r0 * h_rhs, h_rhs,
+                      (double*)workspace, per, m};
+      const int kk = std::min(fit, k - r0);
+      switch (L.E) {
+        case 1: launch_arnoldi<1>(p, L.G, kk, st); break;
+        case 2: launch_arnoldi<2>(p, L.G, kk, st); break;
+        case 4: launch_arnoldi<4>(p, L.G, kk, st); break;
+        default: launch_arnoldi<8>(p, L.G, kk, st); break;
+      }
+    }
+  } else {
+    for (int r = 0; r < k; ++r)
+      arnoldi_separate(L, st, V + r * v_rhs, ldv, m, w + r * w_rhs, n, h + r * h_rhs, hscratch, (double*)workspace);
+  }
+  RMW_CHECK_HIP(hipGetLastError());
+}
+
 // Arnoldi step with CGS2: given basis V[0..j] (j+1 vectors, stride ldv) and
 // w, orthogonalise w against the basis twice, store the j+1 coefficients in
 // h[0..j], ||w|| in h[j+1] and w/||w|| in V[j+1] (e_0 if ||w|| = 0).
@@ -277,27 +479,18 @@ extern "C" int rmw_arnoldi_cgs2(double* V, int64_t ldv, int j, double* w, int64_
                                 void* workspace, size_t workspace_bytes, void* stream)
 {
   return guarded([&] {
-    const int m = j + 1;
-    RMW_REQUIRE(m >= 1 && m + 1 <= kMaxVec, "bad Arnoldi index");
-    const DotLaunch L = dot_launch(n);
-    RMW_REQUIRE(workspace_bytes >= (size_t)L.G * (m + 1) * sizeof(double), "workspace too small");
-    hipStream_t st = (hipStream_t)stream;
-    double* partial = (double*)workspace;
-    const int sb = stream_blocks(n);
-    // pass 1
-    launch_dot_partial(L, st, V, ldv, m, w, n, partial);
-    launch_dot_final(st, partial, L.G, m, h, 0, 0);
-    hipLaunchKernelGGL(sub_combination, dim3(sb), dim3(kKBlock), 0, st, V, ldv, m, h, w, n);
-    // pass 2 (re-orthogonalisation)
-    launch_dot_partial(L, st, V, ldv, m, w, n, partial);
-    launch_dot_final(st, partial, L.G, m, hscratch, 0, 0);
-    hipLaunchKernelGGL(sub_combination, dim3(sb), dim3(kKBlock), 0, st, V, ldv, m, hscratch, w, n);
-    hipLaunchKernelGGL(add_vec, dim3((m + 63) / 64), dim3(64), 0, st, hscratch, h, m);
-    // norm and normalisation
-    launch_dot_partial(L, st, w, (int64_t)0, 1, w, n, partial);
-    launch_dot_final(st, partial, L.G, 1, h + m, 0, 1);
-    hipLaunchKernelGGL(axpby_kernel, dim3(sb), dim3(kKBlock), 0, st, 1.0, w, 0.0, V + (int64_t)m * ldv, n,
-                       (const double*)(h + m));
-    RMW_CHECK_HIP(hipGetLastError());
+    arnoldi_batch(V, ldv, 0, j, 1, w, 0, n, h, 0, hscratch, workspace, workspace_bytes, (hipStream_t)stream);
+  });
+}
+
+// The same step for k bases at once: basis r starts at V + r * v_rhs, its
+// candidate at w + r * w_rhs, its coefficients at h + r * h_rhs.
+extern "C" int rmw_arnoldi_cgs2_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, double* w, int64_t w_rhs,
+                                      int64_t n, double* h, int64_t h_rhs, double* hscratch, void* workspace,
+                                      size_t workspace_bytes, void* stream)
+{
+  return guarded([&] {
+    arnoldi_batch(V, ldv, v_rhs, j, k, w, w_rhs, n, h, h_rhs, hscratch, workspace, workspace_bytes,
+                  (hipStream_t)stream);
   });
 }

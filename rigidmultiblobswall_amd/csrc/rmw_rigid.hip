@@ -258,56 +258,70 @@ __global__ void dense_mobility_kernel(int dom, const double* __restrict__ r, con
 }
 
 // ---------------------------------------------------------------------------
-// Symmetric 6x6 pseudo-inverse by cyclic Jacobi (one thread).
+// Symmetric 6x6 pseudo-inverse by Jacobi rotations, run by one whole wave:
+// lane 6 i + j holds element (i, j) of A and of the eigenvectors, and the
+// three disjoint rotations of a round (five rounds of a round robin make a
+// sweep) are applied together through lane exchanges.  By one thread, with
+// the matrices in scratch memory, this was most of the preconditioner build
+// (YY us of 256 for bodies of 42 blobs).  a6: the matrix in LDS, P: output.
 // ---------------------------------------------------------------------------
-__device__ void pinv6(const double* A_in, double* P)
+__device__ void pinv6_wave(const double* a6, double* __restrict__ P)
 {
-  double A[36], V[36];
-  for (int i = 0; i < 36; ++i) { A[i] = A_in[i]; V[i] = (i % 7 == 0) ? 1.0 : 0.0; }
+  const int lane = threadIdx.x & 63;
+  const bool in = lane < 36;
+  const int i = in ? lane / 6 : 0, j = in ? lane % 6 : 0;
+  double A = in ? a6[lane] : 0.0, V = in && i == j ? 1.0 : 0.0;
+  {
+    double top = 0.0, X = A;
+    for (int k = 0; k < 6; ++k) top = fmax(top, __shfl(A, 7 * k, 64));
+    bool regular = true;
+    for (int k = 0; k < 6; ++k) {
+      const double piv = __shfl(X, 7 * k, 64), rj = __shfl(X, 6 * k + j, 64), ci = __shfl(X, 6 * i + k, 64);
+      regular = regular && piv > 1e-8 * top;   // false for NaN
+      const double ip = 1.0 / piv;
+      X = fma(i == k ? ip : -ci * ip, j == k ? 1.0 : rj, i == k || j == k ? 0.0 : X);
+    }
+    if (regular) {
+      if (in) P[lane] = X;
+      return;
+    }
+  }
+  auto wave_sum = [](double v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  };
   for (int sweep = 0; sweep < 60; ++sweep) {
-    double off = 0.0, diag = 0.0;
-    for (int p = 0; p < 6; ++p)
-      for (int q = 0; q < 6; ++q) {
-        if (p == q) diag += A[p * 6 + q] * A[p * 6 + q];
-        else off += A[p * 6 + q] * A[p * 6 + q];
-      }
+    const double off = wave_sum(in && i != j ? A * A : 0.0), diag = wave_sum(in && i == j ? A * A : 0.0);
     if (off <= 1e-32 * diag || off == 0.0) break;
-    for (int p = 0; p < 5; ++p)
-      for (int q = p + 1; q < 6; ++q) {
-        const double apq = A[p * 6 + q];
-        if (apq == 0.0) continue;
-        const double app = A[p * 6 + p], aqq = A[q * 6 + q];
+    for (int r = 0; r < 5; ++r) {
+      auto partner = [r](int x) { return x == 5 ? r : (x == r ? 5 : (2 * r - x + 10) % 5); };
+      const int pi = partner(i), pj = partner(j);
+      const int p = j < pj ? j : pj, q = j < pj ? pj : j;
+      const double apq = __shfl(A, 6 * p + q, 64), app = __shfl(A, 7 * p, 64), aqq = __shfl(A, 7 * q, 64);
+      double cj = 1.0, tj = 0.0;   // column j' = cj col_j + tj col_pj
+      if (apq != 0.0) {
         const double theta = (aqq - app) / (2.0 * apq);
         const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        for (int k = 0; k < 6; ++k) {  // A <- A J (columns p, q)
-          const double akp = A[k * 6 + p], akq = A[k * 6 + q];
-          A[k * 6 + p] = c * akp - s * akq;
-          A[k * 6 + q] = s * akp + c * akq;
-        }
-        for (int k = 0; k < 6; ++k) {  // A <- J^T A (rows p, q)
-          const double apk = A[p * 6 + k], aqk = A[q * 6 + k];
-          A[p * 6 + k] = c * apk - s * aqk;
-          A[q * 6 + k] = s * apk + c * aqk;
-        }
-        for (int k = 0; k < 6; ++k) {
-          const double vkp = V[k * 6 + p], vkq = V[k * 6 + q];
-          V[k * 6 + p] = c * vkp - s * vkq;
-          V[k * 6 + q] = s * vkp + c * vkq;
-        }
+        cj = 1.0 / sqrt(t * t + 1.0);
+        tj = j == p ? -t * cj : t * cj;
       }
+      const double ci = __shfl(cj, i, 64), ti = __shfl(tj, i, 64);   // lane i is (0, i)
+      const double a01 = __shfl(A, 6 * i + pj, 64), a10 = __shfl(A, 6 * pi + j, 64), a11 = __shfl(A, 6 * pi + pj, 64);
+      const double v1 = __shfl(V, 6 * i + pj, 64);
+      A = ci * (cj * A + tj * a01) + ti * (cj * a10 + tj * a11);
+      V = cj * V + tj * v1;
+    }
   }
-  double lmax = 0.0;
-  for (int i = 0; i < 6; ++i) lmax = fmax(lmax, fabs(A[i * 7]));
+  double lmax = in && i == j ? fabs(A) : 0.0;
+  for (int o = 32; o > 0; o >>= 1) lmax = fmax(lmax, __shfl_xor(lmax, o, 64));
   const double cut = 1e-15 * lmax;  // numpy.linalg.pinv default rcond
-  for (int i = 0; i < 36; ++i) P[i] = 0.0;
+  double x = 0.0;
   for (int e = 0; e < 6; ++e) {
-    const double lam = A[e * 7];
-    if (fabs(lam) <= cut) continue;
-    const double il = 1.0 / lam;
-    for (int i = 0; i < 6; ++i)
-      for (int j = 0; j < 6; ++j) P[i * 6 + j] += V[i * 6 + e] * il * V[j * 6 + e];
+    const double lam = __shfl(A, 7 * e, 64);
+    const double vi = __shfl(V, 6 * i + e, 64), vj = __shfl(V, 6 * j + e, 64);
+    if (fabs(lam) > cut) x += vi * (1.0 / lam) * vj;
   }
+  if (in) P[lane] = x;
 }
 
 // ---------------------------------------------------------------------------
@@ -454,46 +468,64 @@ __global__ __launch_bounds__(kRigidBlock) void pc_build_kernel(PcBuildParams p)
     a6[tid] = s;
   }
   __syncthreads();
-  if (tid == 0) {
-    pinv6(a6, p.nbody + 36 * (int64_t)b);
-    p.status[b] = bad;
-  }
+  if (tid < 64) pinv6_wave(a6, p.nbody + 36 * (int64_t)b);
+  if (tid == 0) p.status[b] = bad;
 }
 
 // Preconditioner build for bodies that fit LDS (n = 3 nb <= kLdsMaxN): M_b
 // assembled in LDS, then inverted in registers by Gauss-Jordan elimination
 // without pivoting (M_b is symmetric positive definite: every pivot is a
 // Schur-complement diagonal, positive; a non-positive one flags the body).
-// Thread (ty, tx) of the 16 x 16 grid holds elements (ty + 16 a, tx + 16 c),
-// a, c < R, of the matrix; each elimination step broadcasts the pivot row
-// and column through LDS (double-buffered, one barrier per step) and
-// applies the rank-one update to the R x R register block:
+// Thread (ty, tx) of the 16 x 16 grid holds the R x R block of elements
+// (R ty + a, R tx + c) in registers.  A step publishes the pivot row through
+// LDS (double-buffered, one barrier) and applies the rank-one update
 //   A'_ij = [i != k][j != k] A_ij - c'_i r'_j / A_kk,
 //   c'_i = A_ik (c'_k = -1),  r'_j = A_kj (r'_k = 1),
-// which also writes the scaled pivot row, column and 1/A_kk in place.
+// which also writes the scaled pivot row, column and 1/A_kk in place.  The
+// matrix stays symmetric but for the sign between eliminated and remaining
+// indices (A_ik = -A_ki for i < k), so the pivot column is read from the
+// published row.  One workgroup has a CU to itself (the matrix fills its LDS)
+// and the n steps follow one another, so the step's latency is what counts:
+// contiguous blocks make its LDS reads 16 bytes wide, steps are unrolled by R so
+// that the pivot's place in the block is a constant, and 1/A_kk is the
+// hardware reciprocal refined twice.  Build for 100 bodies of 42 blobs: 256 us
+// (strided blocks, a select per element, the pseudo-inverse by one thread),
+// now 87.
 // Then M^-1 K from LDS, K^T M^-1 K and its pseudo-inverse.
-template <int R>
-__global__ __launch_bounds__(kRigidBlock) void pc_build_gj_kernel(PcBuildParams p)
+constexpr int kGj = 16;
+
+// 1/x of a positive normal x: two Newton steps on the hardware estimate.
+__device__ __forceinline__ double reciprocal(double x)
 {
-  extern __shared__ double smem[];   // A (n x n) | pivot rows/cols during the elimination, then M^-1 K (n x 6)
+  if (!(x > 1e-290 && x < 1e290)) return 1.0 / x;
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+
+template <int R>
+__global__ __launch_bounds__(kGj* kGj) void pc_build_gj_kernel(PcBuildParams p)
+{
+  extern __shared__ __align__(16) double smem[];   // pivot rows [2][kGj R] | A (n x n) | M^-1 K (n x 6)
   const int b = blockIdx.x;
   const int64_t i0 = p.offs[b], nb = p.offs[b + 1] - i0;
   const int n = (int)(3 * nb);
-  if (n > kLdsMaxN || (n + 15) / 16 > R) return;   // another launch owns this body
-  double* A = smem;
-  double* prow = smem + (size_t)n * n;               // [2][16 R]
-  double* pcol = prow + 2 * 16 * R;                  // [2][16 R]
-  double* MK = smem + (size_t)n * n;                 // n x 6, after the elimination
+  if (n > kLdsMaxN || (n + kGj - 1) / kGj > R) return;   // another launch owns this body
+  double* prow = smem;
+  double* A = smem + 2 * kGj * R;
+  double* MK = A + n * n;
   __shared__ double a6[36];
+  __shared__ double s_rel[kLdsMaxN];                 // blob - centre
   __shared__ int bad;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int tx = tid & 15, ty = tid >> 4;
+  const int tid = threadIdx.x, nt = kGj * kGj;
+  const int tx = tid & (kGj - 1), ty = tid / kGj;
   const double inva = 1.0 / p.a, norm = 1.0 / (8.0 * M_PI * p.eta * p.a);
   if (tid == 0) bad = 0;
+  if (tid < n) s_rel[tid] = p.rrel[3 * i0 + tid];
 
   // 1. assemble M_b
-  for (int64_t idx = tid; idx < nb * nb; idx += nt) {
-    const int64_t i = idx / nb, j = idx - (idx / nb) * nb;
+  for (int idx = tid; idx < (int)(nb * nb); idx += nt) {
+    const int i = idx / (int)nb, j = idx - i * (int)nb;
     double m[9];
     uf_block(p.dom, p.r + 3 * (i0 + i), p.r + 3 * (i0 + j), i == j, p.a, inva, norm, m);
     for (int q = 0; q < 3; ++q)
@@ -502,133 +534,135 @@ __global__ __launch_bounds__(kRigidBlock) void pc_build_gj_kernel(PcBuildParams 
   __syncthreads();
   double E[R][R];
 #pragma unroll
-  for (int ra = 0; ra < R; ++ra)
+  for (int q = 0; q < R; ++q)
 #pragma unroll
-    for (int cb = 0; cb < R; ++cb) {
-      const int i = ty + 16 * ra, j = tx + 16 * cb;
-      E[ra][cb] = (i < n && j < n) ? A[i * n + j] : 0.0;
+    for (int c = 0; c < R; ++c) {
+      const int i = R * ty + q, j = R * tx + c;
+      E[q][c] = (i < n && j < n) ? A[i * n + j] : 0.0;
     }
 
-  // 2. in-place Gauss-Jordan inverse
-  for (int k = 0; k < n; ++k) {
-    double* pr = prow + (k & 1) * 16 * R;
-    double* pc = pcol + (k & 1) * 16 * R;
-    const int ka = k >> 4, kt = k & 15;
-    if (ty == kt) {
+  // 2. in-place Gauss-Jordan inverse (elements beyond n are zeros and stay so)
+  int flip = 0;
+  for (int kb = 0; kb < kGj && kb * R < n; ++kb) {
+    const bool row = ty == kb, col = tx == kb;   // the blocks with the pivot row, column
 #pragma unroll
-      for (int ra = 0; ra < R; ++ra)
-        if (ra == ka) {
+    for (int a = 0; a < R; ++a) {
+      const int k = R * kb + a;
+      if (k >= n) break;
+      double* pr = prow + flip * kGj * R;
+      flip ^= 1;
+      if (row) {
 #pragma unroll
-          for (int cb = 0; cb < R; ++cb) pr[tx + 16 * cb] = E[ra][cb];
+        for (int c = 0; c < R; ++c) {
+          pr[R * tx + c] = E[a][c];
+          E[a][c] = 0.0;
         }
-    }
-    if (tx == kt) {
-#pragma unroll
-      for (int cb = 0; cb < R; ++cb)
-        if (cb == ka) {
-#pragma unroll
-          for (int ra = 0; ra < R; ++ra) pc[ty + 16 * ra] = E[ra][cb];
-        }
-    }
-    __syncthreads();
-    double piv = pr[k];
-    if (!(piv > 0.0)) {
-      if (tid == 0) bad = 1;
-      piv = 1.0;
-    }
-    const double ip = 1.0 / piv;
-    double c[R], r[R];
-#pragma unroll
-    for (int ra = 0; ra < R; ++ra) {
-      const int i = ty + 16 * ra;
-      c[ra] = i == k ? -ip : (i < n ? pc[i] * ip : 0.0);
-    }
-#pragma unroll
-    for (int cb = 0; cb < R; ++cb) {
-      const int j = tx + 16 * cb;
-      r[cb] = j == k ? 1.0 : (j < n ? pr[j] : 0.0);
-    }
-#pragma unroll
-    for (int ra = 0; ra < R; ++ra) {
-      const bool rowk = ty + 16 * ra == k;
-#pragma unroll
-      for (int cb = 0; cb < R; ++cb) {
-        const bool keep = !rowk && tx + 16 * cb != k;
-        E[ra][cb] = fma(-c[ra], r[cb], keep ? E[ra][cb] : 0.0);
       }
+      __syncthreads();
+      double r[R], c[R], piv = pr[k];
+#pragma unroll
+      for (int q = 0; q < R; ++q) r[q] = pr[R * tx + q];
+#pragma unroll
+      for (int q = 0; q < R; ++q) c[q] = pr[R * ty + q];
+      if (!(piv > 0.0)) {
+        if (tid == 0) bad = 1;
+        piv = 1.0;
+      }
+      const double ip = reciprocal(piv);
+      // -c'_i / A_kk: the sign of A_ik against A_ki by i < k
+      const double below = ty < kb ? ip : -ip, above = ty <= kb ? ip : -ip;
+#pragma unroll
+      for (int q = 0; q < R; ++q) c[q] *= q < a ? above : below;
+      if (row) c[a] = ip;
+      if (col) {
+        r[a] = 1.0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) E[q][a] = 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int d = 0; d < R; ++d) E[q][d] = fma(c[q], r[d], E[q][d]);
     }
   }
-  __syncthreads();   // the pivot buffers are free; A is rewritten below
+  __syncthreads();   // A is rewritten below
 
-  // 3. M^-1 to LDS and to the output blocks
+  // 3. M^-1 to LDS, and from there, in rows, to the output blocks
   double* Minv = p.minv + p.moff[b];
 #pragma unroll
-  for (int ra = 0; ra < R; ++ra)
+  for (int q = 0; q < R; ++q)
 #pragma unroll
-    for (int cb = 0; cb < R; ++cb) {
-      const int i = ty + 16 * ra, j = tx + 16 * cb;
-      if (i < n && j < n) {
-        A[i * n + j] = E[ra][cb];
-        Minv[(int64_t)i * n + j] = E[ra][cb];
-      }
+    for (int c = 0; c < R; ++c) {
+      const int i = R * ty + q, j = R * tx + c;
+      if (i < n && j < n) A[i * n + j] = E[q][c];
     }
   __syncthreads();
+  for (int idx = tid; idx < n * n; idx += nt) Minv[idx] = A[idx];
 
   // 4. M^-1 K with K rows [e_c | rot_c] (body.py:92-99: rot_i x = -(r_i x x))
-  double* MKg = p.minvk + 3 * i0 * 6;
-  for (int idx = tid; idx < n * 6; idx += nt) {
-    const int i = idx / 6, c = idx - (idx / 6) * 6;
-    const double* row = A + (int64_t)i * n;
-    double s = 0.0;
+  // entries (3 m .. 3 m + 2, c) of K
+  auto k_entries = [&](int m, int c, double& k0, double& k1, double& k2) {
     if (c < 3) {
-      for (int m = 0; m < (int)nb; ++m) s += row[3 * m + c];
+      k0 = c == 0 ? 1.0 : 0.0; k1 = c == 1 ? 1.0 : 0.0; k2 = c == 2 ? 1.0 : 0.0;
     } else {
+      // column d of rot = [[0, rz, -ry], [-rz, 0, rx], [ry, -rx, 0]]
       const int d = c - 3;
-      for (int m = 0; m < (int)nb; ++m) {
-        const double* rr = p.rrel + 3 * (i0 + m);
-        const double rx = rr[0], ry = rr[1], rz = rr[2];
-        // column d of rot = [[0, rz, -ry], [-rz, 0, rx], [ry, -rx, 0]]
-        const double k0 = d == 0 ? 0.0 : (d == 1 ? rz : -ry);
-        const double k1 = d == 0 ? -rz : (d == 1 ? 0.0 : rx);
-        const double k2 = d == 0 ? ry : (d == 1 ? -rx : 0.0);
-        s += row[3 * m] * k0 + row[3 * m + 1] * k1 + row[3 * m + 2] * k2;
+      const double rx = s_rel[3 * m], ry = s_rel[3 * m + 1], rz = s_rel[3 * m + 2];
+      k0 = d == 0 ? 0.0 : (d == 1 ? rz : -ry);
+      k1 = d == 0 ? -rz : (d == 1 ? 0.0 : rx);
+      k2 = d == 0 ? ry : (d == 1 ? -rx : 0.0);
+    }
+  };
+  // two threads per row, each half of the blobs, all six columns
+  double* MKg = p.minvk + 3 * i0 * 6;
+  for (int i0r = 0; i0r < n; i0r += nt / 2) {
+    const int i = i0r + (tid >> 1);
+    double s[6] = {0, 0, 0, 0, 0, 0};
+    if (i < n) {
+      const double* arow = A + i * n;
+#pragma unroll 4
+      for (int m = tid & 1; m < (int)nb; m += 2) {
+        const double ax = arow[3 * m], ay = arow[3 * m + 1], az = arow[3 * m + 2];
+        const double rx = s_rel[3 * m], ry = s_rel[3 * m + 1], rz = s_rel[3 * m + 2];
+        s[0] += ax;
+        s[1] += ay;
+        s[2] += az;
+        s[3] += az * ry - ay * rz;
+        s[4] += ax * rz - az * rx;
+        s[5] += ay * rx - ax * ry;
       }
     }
-    MK[idx] = s;
-    MKg[idx] = s;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      s[c] += __shfl_xor(s[c], 1, 64);
+      if (i < n && (tid & 1) == c / 3) {
+        MK[6 * i + c] = s[c];
+        MKg[6 * i + c] = s[c];
+      }
+    }
   }
   __syncthreads();
-  // K^T M^-1 K
-  if (tid < 36) {
-    const int r6 = tid / 6, c6 = tid - (tid / 6) * 6;
+  // K^T M^-1 K: four threads per entry, added in a fixed order
+  if (tid < 36 * 4) {
+    const int e = tid >> 2, r6 = e / 6, c6 = e - (e / 6) * 6;
     double s = 0.0;
-    if (r6 < 3) {
-      for (int m = 0; m < (int)nb; ++m) s += MK[(3 * m + r6) * 6 + c6];
-    } else {
-      const int d = r6 - 3;
-      for (int m = 0; m < (int)nb; ++m) {
-        const double* rr = p.rrel + 3 * (i0 + m);
-        const double rx = rr[0], ry = rr[1], rz = rr[2];
-        const double k0 = d == 0 ? 0.0 : (d == 1 ? rz : -ry);
-        const double k1 = d == 0 ? -rz : (d == 1 ? 0.0 : rx);
-        const double k2 = d == 0 ? ry : (d == 1 ? -rx : 0.0);
-        s += k0 * MK[(3 * m) * 6 + c6] + k1 * MK[(3 * m + 1) * 6 + c6] + k2 * MK[(3 * m + 2) * 6 + c6];
-      }
+    for (int m = tid & 3; m < (int)nb; m += 4) {
+      double k0, k1, k2;
+      k_entries(m, r6, k0, k1, k2);
+      s += k0 * MK[(3 * m) * 6 + c6] + k1 * MK[(3 * m + 1) * 6 + c6] + k2 * MK[(3 * m + 2) * 6 + c6];
     }
-    a6[tid] = s;
+    for (int o = 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 4);
+    if ((tid & 3) == 0) a6[e] = s;
   }
   __syncthreads();
-  if (tid == 0) {
-    // symmetrise the rounding of K^T M^-1 K before the pseudo-inverse
-    for (int r6 = 0; r6 < 6; ++r6)
-      for (int c6 = r6 + 1; c6 < 6; ++c6) {
-        const double v = 0.5 * (a6[r6 * 6 + c6] + a6[c6 * 6 + r6]);
-        a6[r6 * 6 + c6] = v;
-        a6[c6 * 6 + r6] = v;
-      }
-    pinv6(a6, p.nbody + 36 * (int64_t)b);
-    p.status[b] = bad;
-  }
+  // symmetrise the rounding of K^T M^-1 K before the pseudo-inverse
+  double sym = 0.0;
+  if (tid < 36) sym = 0.5 * (a6[tid] + a6[(tid % 6) * 6 + tid / 6]);
+  __syncthreads();
+  if (tid < 36) a6[tid] = sym;
+  __syncthreads();
+  if (tid < 64) pinv6_wave(a6, p.nbody + 36 * (int64_t)b);
+  if (tid == 0) p.status[b] = bad;
 }
 
 // ---------------------------------------------------------------------------
@@ -700,70 +734,83 @@ __global__ __launch_bounds__(kPfBlock) void point_field_kernel(const double* __r
   }
 }
 
-// Preconditioner apply: y = P^-1 x, one workgroup per body.
+// Preconditioner apply y = P^-1 x: one workgroup per body and slice of
+// kPcRows rows.  With lt = M^-1 s and M^-1 symmetric, K^T lt is (M^-1 K)^T s, so
+// a workgroup has Y = N_b (-F - (M^-1 K)^T s) after reading the body's n x 6
+// block and needs no other rows than its own: one workgroup per body, in
+// three dependent phases, took 28.9 us for 100 bodies of 42 blobs (12.7 MB of
+// M^-1, 2.6 us at the rate of a copy), 9.5 now.  Four rows per wave at a time,
+// lanes across the columns.
+constexpr int kPcRows = 16;
 __global__ __launch_bounds__(kRigidBlock) void pc_apply_kernel(const int64_t* __restrict__ offs,
                                                                const int64_t* __restrict__ moff,
                                                                const double* __restrict__ minv,
                                                                const double* __restrict__ minvk,
                                                                const double* __restrict__ nbody,
-                                                               const double* __restrict__ rrel,
                                                                const double* __restrict__ x,
                                                                double* __restrict__ y, int64_t nblobs)
 {
-  extern __shared__ double sm[];  // s (n) | lt (n)
+  extern __shared__ double s[];   // the body's part of x (n)
   const int b = blockIdx.x;
   const int64_t i0 = offs[b], nb = offs[b + 1] - i0;
   const int n = (int)(3 * nb);
-  double* s = sm;
-  double* lt = sm + n;
-  __shared__ double t6[6], Y[6];
+  const int row0 = blockIdx.y * kPcRows;
+  if (blockIdx.y > 0 && row0 >= n) return;
   __shared__ double red[6][kRigidBlock / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
-  for (int i = tid; i < n; i += blockDim.x) s[i] = x[3 * i0 + i];
-  __syncthreads();
-  // lt = M^-1 s: one wavefront per row, lanes across columns (coalesced)
-  const double* M = minv + moff[b];
-  for (int i = wv; i < n; i += nw) {
-    double acc = 0.0;
-    for (int j = lane; j < n; j += 64) acc += M[(int64_t)i * n + j] * s[j];
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-    if (lane == 0) lt[i] = acc;
-  }
-  __syncthreads();
-  // t = -F - K^T lt
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const double* MK = minvk + 3 * i0 * 6;
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int m = tid; m < nb; m += blockDim.x) {
-    const double* rr = rrel + 3 * (i0 + m);
-    const double lx = lt[3 * m], ly = lt[3 * m + 1], lz = lt[3 * m + 2];
-    acc[0] += lx; acc[1] += ly; acc[2] += lz;
-    acc[3] += rr[1] * lz - rr[2] * ly;
-    acc[4] += rr[2] * lx - rr[0] * lz;
-    acc[5] += rr[0] * ly - rr[1] * lx;
+  for (int i = tid; i < n; i += kRigidBlock) {
+    const double v = x[3 * i0 + i];
+    s[i] = v;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) acc[c] = fma(MK[i * 6 + c], v, acc[c]);
   }
+#pragma unroll
   for (int c = 0; c < 6; ++c) {
-    double v = acc[c];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    if (lane == 0) red[c][wv] = v;
+    for (int o = 32; o > 0; o >>= 1) acc[c] += __shfl_down(acc[c], o, 64);
+    if (lane == 0) red[c][wv] = acc[c];
   }
   __syncthreads();
-  if (tid < 6) {
-    double v = 0.0;
-    for (int w = 0; w < nw; ++w) v += red[tid][w];
-    t6[tid] = -x[3 * nblobs + 6 * (int64_t)b + tid] - v;
+  // Y = N_b (-F - (M^-1 K)^T s), by every thread
+  double t6[6], Y[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c)
+    t6[c] = -x[3 * nblobs + 6 * (int64_t)b + c] - (((red[c][0] + red[c][1]) + red[c][2]) + red[c][3]);
+  const double* Nb = nbody + 36 * (int64_t)b;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    Y[c] = 0.0;
+#pragma unroll
+    for (int d = 0; d < 6; ++d) Y[c] = fma(Nb[c * 6 + d], t6[d], Y[c]);
   }
-  __syncthreads();
-  if (tid < 6) {
-    const double* Nb = nbody + 36 * (int64_t)b;
-    double v = 0.0;
-    for (int c = 0; c < 6; ++c) v += Nb[tid * 6 + c] * t6[c];
-    Y[tid] = v;
+  if (blockIdx.y == 0 && tid < 6) {
+    double v = Y[0];
+#pragma unroll
+    for (int c = 1; c < 6; ++c) v = tid == c ? Y[c] : v;
     y[3 * nblobs + 6 * (int64_t)b + tid] = v;
   }
-  __syncthreads();
-  const double* MK = minvk + 3 * i0 * 6;
-  for (int i = tid; i < n; i += blockDim.x) {
-    double v = lt[i];
-    for (int c = 0; c < 6; ++c) v += MK[i * 6 + c] * Y[c];
+  // rows r0 .. r0 + 3 of M^-1 s (rows beyond n repeat the last and are dropped)
+  const double* M = minv + moff[b];
+  const int r0 = row0 + 4 * wv;
+  if (r0 >= n) return;
+  double a[4] = {0, 0, 0, 0};
+  const double* Mr[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) Mr[q] = M + (int64_t)(r0 + q < n ? r0 + q : n - 1) * n;
+  for (int j = lane; j < n; j += 64) {
+    const double v = s[j];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = fma(Mr[q][j], v, a[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    for (int o = 32; o > 0; o >>= 1) a[q] += __shfl_xor(a[q], o, 64);
+  if (lane < 4 && r0 + lane < n) {
+    const int i = r0 + lane;
+    double v = lane == 0 ? a[0] : (lane == 1 ? a[1] : (lane == 2 ? a[2] : a[3]));
+#pragma unroll
+    for (int c = 0; c < 6; ++c) v = fma(MK[i * 6 + c], Y[c], v);
     y[3 * i0 + i] = v;
   }
 }
@@ -865,7 +912,7 @@ static void launch_pc_gj_r(const PcBuildParams& p, int nbodies, size_t lds, hipS
 {
   RMW_CHECK_HIP(hipFuncSetAttribute((const void*)pc_build_gj_kernel<R>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds));
-  hipLaunchKernelGGL(pc_build_gj_kernel<R>, dim3(nbodies), dim3(kRigidBlock), lds, st, p);
+  hipLaunchKernelGGL(pc_build_gj_kernel<R>, dim3(nbodies), dim3(kGj * kGj), lds, st, p);
   RMW_CHECK_HIP(hipGetLastError());
 }
 
@@ -1081,9 +1128,8 @@ extern "C" int rmw_rigid_pc_build_ex(int domain, const double* r_blobs, const do
     }
     if (max_small && chol == nullptr) {
       // Gauss-Jordan in registers, R x R elements per thread for the largest body
-      const int R = std::max(1, (max_small + 15) / 16);
-      const size_t lds = ((size_t)max_small * max_small + std::max<size_t>(6 * (size_t)max_small, 4 * 16 * (size_t)R)) *
-                         sizeof(double);
+      const int R = std::max(1, (max_small + kGj - 1) / kGj);
+      const size_t lds = ((size_t)max_small * max_small + 6 * (size_t)max_small + 2 * kGj * (size_t)R) * sizeof(double);
       RMW_REQUIRE(lds <= 160 * 1024, "preconditioner build exceeds LDS");
       launch_pc_gj(R, p, nbodies, lds, st);
     } else if (max_small) {
@@ -1164,9 +1210,10 @@ extern "C" int rmw_rigid_pc_apply(const int64_t* body_offsets, int nbodies, cons
     if (lds > 64 * 1024)
       RMW_CHECK_HIP(hipFuncSetAttribute((const void*)pc_apply_kernel,
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(pc_apply_kernel, dim3(nbodies), dim3(kRigidBlock), lds, st,
-                       (const int64_t*)(ws + L.off_offs), (const int64_t*)(ws + L.off_moff), minv, minvk,
-                       nbody, r_rel, x, y, L.nblobs);
+    const unsigned slices = (unsigned)std::max<int64_t>(1, (L.max_n + kPcRows - 1) / kPcRows);
+    hipLaunchKernelGGL(pc_apply_kernel, dim3(nbodies, slices), dim3(kRigidBlock), lds / 2, st,
+                       (const int64_t*)(ws + L.off_offs), (const int64_t*)(ws + L.off_moff), minv, minvk, nbody, x, y,
+                       L.nblobs);
     RMW_CHECK_HIP(hipGetLastError());
   });
 }

@@ -81,24 +81,26 @@ def lanczos_block(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torch
     W = torch.empty((k, dim), dtype=torch.float64, device=dev)
     H = torch.zeros((k, mcap, mcap + 1), dtype=torch.float64, device=dev)
     hs = torch.empty(mmax + 1, dtype=torch.float64, device=dev)
-    C = torch.empty((k, mmax + 1), dtype=torch.float64, device=dev)   # last column: QL status
-    scale = torch.empty(k, dtype=torch.float64, device=dev)
+    C = torch.empty((k, mmax), dtype=torch.float64, device=dev)
     zsrc = Z.to(torch.float64).contiguous()
-    znorm = np.zeros(k)
-    for r in range(k):
-        znorm[r] = ops.norm(zsrc[r])
-        if znorm[r] == 0.0:
-            raise ValueError("a zero right-hand side has no Lanczos basis")
-        ops.axpby(1.0 / znorm[r], zsrc[r], 0.0, V[0, r])
-    scale.copy_(torch.from_numpy(znorm * factor))
     ldv = k * dim
-    status = torch.zeros(k, dtype=torch.int32, device=dev)
+    znorm = torch.empty(k, dtype=torch.float64, device=dev)
+    for r in range(k):
+        _lib.check(lib.rmw_dot_many(zsrc[r].data_ptr(), 0, 1, zsrc[r].data_ptr(), dim, znorm[r].data_ptr(), 1,
+                                    ops.ws.data_ptr(), ops.ws.numel(), _stream()))
+        ops.axpby(1.0, zsrc[r], 0.0, V[0, r], div=znorm[r])
+    if bool((znorm == 0.0).any()):
+        raise ValueError("a zero right-hand side has no Lanczos basis")
+    scale = znorm * factor
     nscr = ctypes.c_size_t()
     # scratch of the tridiagonal solve (k m^2 doubles), grown geometrically,
-    # and a pinned host buffer for the coefficients the stop test reads
+    # and the stop test's numbers with a pinned host copy
     zscr = None
-    c_host = torch.empty((k, mmax + 1), dtype=torch.float64, pin_memory=True)
-    c_prev = [None] * k
+    test = torch.empty((k, 3), dtype=torch.float64, device=dev)
+    t_host = torch.empty((k, 3), dtype=torch.float64, pin_memory=True)
+    t_np = t_host.numpy()
+    eps = np.finfo(float).eps
+    stream = torch.cuda.current_stream(dev)
     converged = np.zeros(k, dtype=bool)
     it_conv = np.full(k, max_iter)
     i_last = 0
@@ -111,44 +113,33 @@ def lanczos_block(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torch
             H2[:, :mcap, :mcap + 1] = H
             V, H, mcap = V2, H2, m2
         matvec(V[i], W)
-        for r in range(k):
-            _lib.check(lib.rmw_arnoldi_cgs2(V[0, r].data_ptr(), ldv, i, W[r].data_ptr(), dim, H[r, i].data_ptr(),
-                                            hs.data_ptr(), ops.ws.data_ptr(), ops.ws.numel(), _stream()))
+        _lib.check(lib.rmw_arnoldi_cgs2_batch(V.data_ptr(), ldv, dim, i, k, W.data_ptr(), dim, dim,
+                                              H.data_ptr() + 8 * i * H.stride(1), H.stride(0), hs.data_ptr(),
+                                              ops.ws.data_ptr(), ops.ws.numel(), _stream()))
         m = i + 1
         _lib.check(lib.rmw_lanczos_scratch_doubles(m, k, ctypes.byref(nscr)))
         if zscr is None or zscr.numel() < nscr.value:
             _lib.check(lib.rmw_lanczos_scratch_doubles(min(mmax, max(2 * m, 32)), k, ctypes.byref(nscr)))
             zscr = torch.empty(nscr.value, dtype=torch.float64, device=dev)
-        _lib.check(lib.rmw_lanczos_sqrt_coeffs(H.data_ptr(), H.stride(0), H.stride(1), m, k, scale.data_ptr(),
+        _lib.check(lib.rmw_lanczos_step_coeffs(H.data_ptr(), H.stride(0), H.stride(1), m, k, scale.data_ptr(),
                                                C.data_ptr(), C.stride(0), zscr.data_ptr(), zscr.numel(),
-                                               status.data_ptr(), _stream()))
-        # one read-back per step: the coefficients and the QL status together
-        C[:, mmax] = status.to(torch.float64)
-        c_host[:, :m].copy_(C[:, :m], non_blocking=True)
-        c_host[:, mmax].copy_(C[:, mmax], non_blocking=True)
-        torch.cuda.current_stream().synchronize()
-        if float(c_host[:, mmax].sum()) != 0.0:
+                                               test.data_ptr(), _stream()))
+        # one read-back per step: the change of the coefficients and the QL status
+        t_host.copy_(test, non_blocking=True)
+        stream.synchronize()
+        if t_np[:, 2].any():
             raise RuntimeError("tridiagonal eigen-solve did not converge")
-        c_now = c_host[:, :m].numpy().copy()
         i_last = i
         if i > 0:
-            for r in range(k):
-                if converged[r]:
-                    continue
-                prev = np.concatenate([c_prev[r], [0.0]])
-                diff = np.linalg.norm(c_now[r] - prev)
-                if diff / max(np.linalg.norm(c_prev[r]), np.finfo(float).eps) < tolerance:
-                    converged[r] = True
-                    it_conv[r] = i
-        c_prev = [c_now[r].copy() for r in range(k)]
+            newly = ~converged & (t_np[:, 0] / np.maximum(t_np[:, 1], eps) < tolerance)
+            it_conv[newly] = i
+            converged |= newly
         if converged.all():
             break
     m = i_last + 1
     noise = torch.empty((k, dim), dtype=torch.float64, device=dev)
-    coef = torch.empty(m, dtype=torch.float64, device=dev)
     for r in range(k):
-        coef.copy_(C[r, :m])
-        ops.combination(V[:, r], m, coef, noise[r], accumulate=False)
+        ops.combination(V[:, r], m, C[r], noise[r], accumulate=False)
     if not converged.all():
         _unconverged(f"{int((~converged).sum())} of {k} right-hand sides after {max_iter} steps", strict)
     if L_mult is not None:
