@@ -786,7 +786,7 @@ static ForcePlan force_plan(int prec, int64_t n, const rmw_tuning* tuning, bool 
   }
   if (pl.direct) {
     pl.total_items = (n + kDT - 1) / kDT;
-    pl.bytes = 0;
+    pl.bytes = align_up((size_t)n * 3 * sizeof(double));   // the forces of a call in place
   }
   if (pl.cells) {
     pl.buckets = 1024;
@@ -913,7 +913,10 @@ extern "C" int rmw_blob_forces(int prec, const double* r_vectors, const double* 
     // the cell arithmetic
     CellParams c{};
     const double range = force_range(f64, radius_blobs != nullptr, blob_radius, debye_length, cutoff);
-    bool cells = pl.cells && range > 0.0 && std::isfinite(range);
+    // forces written over an input: the launches below that write them while
+    // they read the inputs are not taken, or write to the workspace first
+    const bool in_place = overlap(force, 3 * n, r_vectors, 3 * n) || overlap(force, 3 * n, radius_blobs, n);
+    bool cells = pl.cells && !in_place && range > 0.0 && std::isfinite(range);
     if (cells) {
       cells_layout((char*)workspace + pl.off_cells, n, pl.buckets, &c);
       c.mask = pl.buckets - 1;
@@ -936,16 +939,18 @@ extern "C" int rmw_blob_forces(int prec, const double* r_vectors, const double* 
     }
     // what the cells cannot serve goes the same way as what they turn out not
     // to suit
-    const bool direct = pl.direct || (pl.cells && !cells && n <= kDirectFallback);
+    const bool direct = pl.direct || (pl.cells && !cells && !in_place && n <= kDirectFallback);
+    double* const out = direct && in_place ? (double*)workspace : force;
     if (f64) {
-      if (cut) launch_any<true, true>(pl, q, c, direct, cells, scale, force, grid, st);
-      else launch_any<true, false>(pl, q, c, direct, cells, scale, force, grid, st);
+      if (cut) launch_any<true, true>(pl, q, c, direct, cells, scale, out, grid, st);
+      else launch_any<true, false>(pl, q, c, direct, cells, scale, out, grid, st);
     } else {
-      if (cut) launch_any<false, true>(pl, q, c, direct, cells, scale, force, grid, st);
-      else launch_any<false, false>(pl, q, c, direct, cells, scale, force, grid, st);
+      if (cut) launch_any<false, true>(pl, q, c, direct, cells, scale, out, grid, st);
+      else launch_any<false, false>(pl, q, c, direct, cells, scale, out, grid, st);
     }
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
+    if (out != force) launch_copy_rows(out, 3 * n, force, 3 * n, 3 * n, 1, st);
     if (direct || (cells && n <= kDirectFallback)) return;
     const dim3 rg((unsigned)((n * 3 + 255) / 256)), rb(256);
     if (pl.mutual)

@@ -54,6 +54,18 @@ int guarded(F&& body)
 
 inline size_t align_up(size_t x, size_t a = 256) { return (x + a - 1) / a * a; }
 
+// Do [a, a + na) and [b, b + nb), counted in doubles, share memory?
+inline bool overlap(const double* a, int64_t na, const double* b, int64_t nb)
+{
+  return a && b && (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
+// dst[k dst_stride + i] = src[k src_stride + i], i < len, k < K, by a kernel.
+// One-launch products whose output lies over an input go through a copy: a
+// workgroup writes its targets while others still read the input.
+void launch_copy_rows(const double* src, int64_t src_stride, double* dst, int64_t dst_stride, int64_t len, int K,
+                      hipStream_t st);
+
 struct DeviceProps {
   int device = -1;
   int cu_count = 0;

@@ -379,9 +379,9 @@ struct DirectParams {
   const double* r;
   const double* f;          // K right-hand sides rhs_stride apart, or null
   const double* t;
-  double* vel;              // outputs, same stride, or null
+  double* vel;              // outputs, out_stride apart, or null
   double* omg;
-  int64_t rhs_stride;
+  int64_t rhs_stride, out_stride;
   double a, inva, c1, c2;
   const DirectSys* table;   // nullptr -> single
   DirectSys single;

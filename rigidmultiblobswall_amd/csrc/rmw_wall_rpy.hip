@@ -800,6 +800,21 @@ __global__ __launch_bounds__(256) void mutual_reduce_kernel(MutReduceParams p)
 // ---------------------------------------------------------------------------
 // 5. optional check of the outputs (RMW_FLAG_CHECK_FINITE).
 // ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void copy_rows_kernel(const double* __restrict__ src, int64_t src_stride,
+                                                        double* __restrict__ dst, int64_t dst_stride, int64_t len)
+{
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < len) dst[blockIdx.y * dst_stride + i] = src[blockIdx.y * src_stride + i];
+}
+
+void launch_copy_rows(const double* src, int64_t src_stride, double* dst, int64_t dst_stride, int64_t len, int K,
+                      hipStream_t st)
+{
+  hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)((len + 255) / 256), K), dim3(256), 0, st, src, src_stride, dst,
+                     dst_stride, len);
+  RMW_CHECK_HIP(hipGetLastError());
+}
+
 __global__ void zero_count_kernel(unsigned int* count)
 {
   if (threadIdx.x == 0) count[0] = 0u;
@@ -879,7 +894,7 @@ struct Plan {
   int kmax_direct = 1;
   SmallVec<DirectSys> dsys;  // non-empty systems only
   int64_t direct_wgs = 0;
-  size_t off_dtable = 0;
+  size_t off_dtable = 0, off_stage = 0;   // off_stage: outputs of a product in place
   // RMW_FLAG_CHECK_FINITE: a counter of non-finite outputs after the rest
   bool check_finite = false;
   size_t off_status = 0;
@@ -1173,6 +1188,9 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
     pl.kmax_direct = group_k(k, std::min(direct_max_k(mask, domain), rhs_cap(tuning) > 0 ? rhs_cap(tuning) : 4));
     pl.dsys = direct_table(offsets, nsys, direct_targets(mask, pl.kmax_direct), pl.direct_wgs);
     if (pl.dsys.size() > 1) { pl.off_dtable = o; o = align_up(o + pl.dsys.size() * sizeof(DirectSys)); }
+    pl.off_stage = o;
+    o = align_up(o + (size_t)pl.kmax_direct * 3 * pl.ntot * sizeof(double) *
+                         (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0)));
   }
   if (pl.path == kOrderedPath) {
     pl.off_partial = o; o = align_up(o + pl.partial_doubles * sizeof(double));
@@ -1550,6 +1568,7 @@ static void run_direct(const Plan& pl, const double* r, const double* f, const d
     q.vel = vel ? vel + (size_t)k0 * stride : nullptr;
     q.omg = omg ? omg + (size_t)k0 * stride : nullptr;
     q.rhs_stride = stride;
+    q.out_stride = stride;
     q.a = a; q.inva = inva; q.c1 = c1; q.c2 = c2;
     q.table = dtable;
     q.single = table[0];
@@ -1559,9 +1578,26 @@ static void run_direct(const Plan& pl, const double* r, const double* f, const d
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st);
+    // outputs over an input (a product in place): by way of the workspace
+    const int64_t len = 3 * pl.ntot, span = (K - 1) * stride + len;
+    auto over_input = [&](const double* out) {
+      return overlap(out, span, r, len) || overlap(out, span, q.f, span) || overlap(out, span, q.t, span);
+    };
+    double *const vel_k = q.vel, *const omg_k = q.omg;
+    const bool staged = over_input(vel_k) || over_input(omg_k);
+    if (staged) {
+      double* stage = (double*)(base + pl.off_stage);
+      q.out_stride = len;
+      if (vel_k) { q.vel = stage; stage += K * len; }
+      if (omg_k) q.omg = stage;
+    }
     launch_direct(pl.domain, pl.mask, pl.prec, K, q, wgs, st);
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
+    if (staged) {
+      if (vel_k) launch_copy_rows(q.vel, len, vel_k, stride, len, K, st);
+      if (omg_k) launch_copy_rows(q.omg, len, omg_k, stride, len, K, st);
+    }
   }
 }
 
