@@ -54,6 +54,20 @@ template <> struct Acc<RMW_PREC_F64> {
   __device__ __forceinline__ double get() const { return v; }
 };
 
+// The seed of a chained product and the taking of its result (C), or a plain add.
+template <bool C, typename T, class A>
+__device__ __forceinline__ T chain_seed(A& a)
+{
+  if constexpr (C) return a.run();
+  else return T(0);
+}
+template <bool C, typename T, class A>
+__device__ __forceinline__ void chain_take(A& a, T x)
+{
+  if constexpr (C) a.run() = x;
+  else a.add(x);
+}
+
 constexpr int kSub = 16;  // sources per FP32 sub-sum in the blocked mode
 
 // Minimum-image shift count of mobility_numba.py:184-193: int(d/L + 0.5 sign(d)).

@@ -628,25 +628,30 @@ RMW_HD CoefRadii<T> coef_radii(T dx, T dy, T dz, T Rz, T x3, T y3, T a, T b, T i
   CoefRadii<T> c;
   const T r2 = dx * dx + dy * dy + dz * dz;
   rpy_radii(r2, a, b, inva, invb, c.C1, c.C2);
-  const T s = a * a + b * b;
   if (bnd == kRadiiWall) {
-    const T rho2 = dx * dx + dy * dy + Rz * Rz;
+    // powers of w = 1/rho^2 gathered per dyad (Horner), q = 1/rho:
+    //   alpha = q [1 + w (s/3 + 2 x3 y3 + w (-3 m R_z - cab + 5 cab R_z^2 w))]
+    //   beta  = q^3 [1 - w (s + 6 x3 y3 - w (15 m R_z + 5 cab - 35 cab R_z^2 w))]
+    //   g1 = q^3 [x3 (t - 2) + z],  g2 = q^3 [y3 (-t - 2) + z],
+    //   t = 3 (ca - cb) w,  z = 10 cab R_z w^2
+    //   delta = -q [2 + w (ca + cb + 2 cab w)],  m = ca y3 + cb x3
+    const T a2 = a * a, b2 = b * b, s = a2 + b2;
+    const T rho2 = fma_(dx, dx, fma_(dy, dy, Rz * Rz));
     const T q = rsq(rho2);
-    const T qw = q * q;
-    const T q3 = q * qw, q5 = q3 * qw, q7 = q5 * qw, q9 = q7 * qw;
-    const T ca = T(2.0 / 3.0) * a * a, cb = T(2.0 / 3.0) * b * b, cab = ca * b * b;
-    const T Rz2 = Rz * Rz;
+    const T w = q * q;
+    const T q3 = q * w;
+    const T ca = T(2.0 / 3.0) * a2, cb = T(2.0 / 3.0) * b2, cab = ca * b2;
     const T xy = x3 * y3;
-    const T m = ca * y3 + cb * x3;
-    const T P = fma_(s * qw, T(1.0 / 3.0), T(1)) * q;
-    const T Q = fma_(-s, qw, T(1)) * q3;
-    c.al = P + T(2) * xy * q3 - T(3) * m * Rz * q5 + cab * (T(5) * Rz2 * q7 - q5);
-    c.be = Q - T(6) * xy * q5 + T(15) * m * Rz * q7 + cab * (T(5) * q7 - T(35) * Rz2 * q9);
-    const T e = T(3) * (ca - cb) * q5;
-    const T z10 = T(10) * cab * Rz * q7;
-    c.g1 = x3 * (e - T(2) * q3) + z10;
-    c.g2 = y3 * (-e - T(2) * q3) + z10;
-    c.de = -T(2) * q - (ca + cb) * q3 - T(2) * cab * q5;
+    const T mR = fma_(ca, y3, cb * x3) * Rz;
+    const T cz = cab * Rz * w;               // cab R_z w
+    const T cR = cz * Rz;
+    c.al = q * fma_(w, fma_(w, fma_(T(5), cR, fma_(T(-3), mR, -cab)), fma_(T(2), xy, T(1.0 / 3.0) * s)), T(1));
+    c.be = q3 * fma_(w, fma_(w, fma_(T(-35), cR, fma_(T(15), mR, T(5) * cab)), fma_(T(-6), xy, -s)), T(1));
+    const T t = T(3) * (ca - cb) * w;
+    const T z = T(10) * cz * w;
+    c.g1 = q3 * fma_(x3, t - T(2), z);
+    c.g2 = q3 * fma_(y3, -t - T(2), z);
+    c.de = -q * fma_(w, fma_(T(2) * cab, w, ca + cb), T(2));
   } else if (bnd == kRadiiFreeSurface) {
     T I1, I2;
     rpy_radii(dx * dx + dy * dy + Rz * Rz, a, b, inva, invb, I1, I2);
@@ -659,18 +664,38 @@ RMW_HD CoefRadii<T> coef_radii(T dx, T dy, T dz, T Rz, T x3, T y3, T a, T b, T i
   return c;
 }
 
-template <typename T>
-RMW_HD Vec3<T> apply_radii(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz)
+template <typename T, bool ADD = false>
+RMW_HD Vec3<T> apply_radii(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz,
+                           const Vec3<T>& acc = Vec3<T>{})
 {
-  const T p = dx * vx + dy * vy;
-  const T dv = p + dz * vz;
-  const T Rv = p - Rz * vz;               // R . D v
-  const T h = c.be * Rv - c.g1 * vz;      // coefficient of R
+  const T p = fma_(dx, vx, dy * vy);
+  const T dv = fma_(dz, vz, p);
+  const T Rv = fma_(-Rz, vz, p);          // R . D v
+  const T h = fma_(c.be, Rv, -c.g1 * vz);   // coefficient of -R
   const T q = c.C2 * dv;
+  const T k = c.C1 - c.al, e = q - h;
   Vec3<T> u;
-  u.x = (c.C1 - c.al) * vx + (q - h) * dx;
-  u.y = (c.C1 - c.al) * vy + (q - h) * dy;
-  u.z = (c.C1 + c.al) * vz + q * dz - h * Rz - (c.g2 * Rv - c.de * vz);
+  u.x = fma_(k, vx, fma_or_mul<ADD>(e, dx, acc.x));
+  u.y = fma_(k, vy, fma_or_mul<ADD>(e, dy, acc.y));
+  u.z = fma_(c.C1 + c.al + c.de, vz, fma_(q, dz, fma_(-h, Rz, fma_or_mul<ADD>(-c.g2, Rv, acc.z))));
+  return u;
+}
+
+// M_ij^T v (the coefficients as computed for the ordered pair (i, j)).
+template <typename T, bool ADD = false>
+RMW_HD Vec3<T> apply_radii_t(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz,
+                             const Vec3<T>& acc = Vec3<T>{})
+{
+  const T p = fma_(dx, vx, dy * vy);
+  const T dv = fma_(dz, vz, p);
+  const T Rv = fma_(Rz, vz, p);           // R . v
+  const T h = fma_(c.be, Rv, c.g2 * vz);    // coefficient of -D R
+  const T q = c.C2 * dv;
+  const T k = c.C1 - c.al, e = q - h;
+  Vec3<T> u;
+  u.x = fma_(k, vx, fma_or_mul<ADD>(e, dx, acc.x));
+  u.y = fma_(k, vy, fma_or_mul<ADD>(e, dy, acc.y));
+  u.z = fma_(c.C1 + c.al + c.de, vz, fma_(q, dz, fma_(h, Rz, fma_or_mul<ADD>(c.g1, Rv, acc.z))));
   return u;
 }
 

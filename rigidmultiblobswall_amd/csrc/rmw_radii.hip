@@ -175,28 +175,63 @@ __global__ void radii_zero_kernel(double* __restrict__ out, int64_t n)
   if (i < n) out[i] = 0.0;
 }
 
+// Rules of the launches without a shape in the tuning; wall, one MI355X, us:
+//  - one direct launch up to kRDirectPairs source-target pairs (before: the
+//    ordered kernel with chunks of 256 sources, 97 at all of these), unless
+//    few workgroups would walk many sources or hold few of them each:
+//    1000 x 5000 20 in FP32 (direct) against 33 (ordered), FP64 29 / 43;
+//    256 x 20000 26 / 32, FP64 38 / 41; but 20000 x 260 99 / 84, FP64
+//    105 / 99, and 10 x 20000 22 / 16, FP64 31 / 16.
+//  - sources = targets, no images: direct up to kRDirectSelf^2 pairs, then the
+//    symmetric kernel on 64-blob blocks up to kRBlockBlobs, then on 256-blob
+//    tiles.  direct / blocks at 1280 blobs 12 / 14, 1600 15 / 16, 2304
+//    25 / 20 (FP64 16 / 16, 20 / 20, 37 / 26); blocks / tiles at 2304 blobs
+//    20 / 113, 6000 66 / 126, 10007 152 / 192, 18000 422 / 430, 20480
+//    527 / 535, 32768 1311 / 1287 (FP64 10007 246 / 311, 18000 744 / 748).
+//  - ordered chunks of at least 64 sources (256 before: 97 at 1000 x 5000),
+//    256 beyond 65536 sources, whose partial sums the reduce would walk for
+//    longer than the pairs take (1000000 x 5: 2511 against 1025).
+constexpr int kRDT = 4;      // targets of a workgroup of the direct kernel
+constexpr double kRDirectPairs = 2304.0 * 2304.0, kRDirectSelf = 1600.0 * 1600.0;
+constexpr int64_t kRDirectSources = 8192, kRDirectTargets = 256;   // targets per source
+constexpr int64_t kRBlockBlobs = 18432;
+
+static bool shaped(const rmw_tuning* t)
+{
+  return t && (t->chunk_len > 0 || t->max_wgs > 0 || t->symmetric != 0);
+}
+
 struct RadiiPlan {
+  bool direct = false;
   int64_t chunk_len = 0, n_chunks = 0, n_tt = 0, total_items = 0;
   size_t bytes = 0;
 };
 
-static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* tuning)
+static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* tuning,
+                            double direct_pairs = kRDirectPairs)
 {
   RMW_REQUIRE(prec == RMW_PREC_F32_F64ACC || prec == RMW_PREC_F32_KAHAN || prec == RMW_PREC_F64 ||
                   prec == RMW_PREC_F32_BLOCKED,
               "unknown precision mode");
   RMW_REQUIRE(ns >= 0 && nt >= 0, "sizes must be >= 0");
   RadiiPlan pl;
+  pl.n_tt = (nt + kRBlock - 1) / kRBlock;
+  if (!shaped(tuning) && (double)ns * (double)nt <= direct_pairs && ns <= kRDirectSources &&
+      nt <= kRDirectTargets * ns) {
+    pl.direct = true;
+    pl.total_items = (nt + kRDT - 1) / kRDT;
+    pl.bytes = align_up((size_t)nt * 3 * sizeof(double));   // the output of a product in place
+    return pl;
+  }
   int64_t chunk = tuning && tuning->chunk_len > 0 ? tuning->chunk_len : 0;
   if (chunk <= 0) {
     const double c = (double)ns * (double)nt / (16.0 * std::max(device_props().cu_count, 1) * kRBlock);
-    chunk = std::max<int64_t>(kRBlock, (int64_t)std::ceil(c / 64.0) * 64);
+    chunk = std::max<int64_t>(ns <= 65536 ? 64 : kRBlock, (int64_t)std::ceil(c / 64.0) * 64);
   }
   chunk = std::max<int64_t>(64, (chunk + 63) / 64 * 64);
   if (ns > 0) chunk = std::min<int64_t>(chunk, (ns + 63) / 64 * 64);
   pl.chunk_len = chunk;
   pl.n_chunks = ns > 0 ? (ns + chunk - 1) / chunk : 0;
-  pl.n_tt = (nt + kRBlock - 1) / kRBlock;
   pl.total_items = pl.n_tt * pl.n_chunks;
   pl.bytes = align_up((size_t)pl.n_chunks * nt * 3 * sizeof(double));
   return pl;
@@ -210,22 +245,6 @@ static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* 
 // swaps g1 and g2, which the free surface does not have), so each unordered
 // pair is evaluated once and applied to both blobs.
 // ---------------------------------------------------------------------------
-
-// M_ij^T v (the coefficients as computed for the ordered pair (i, j)).
-template <typename T>
-__device__ __forceinline__ Vec3<T> apply_radii_t(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz)
-{
-  const T p = dx * vx + dy * vy;
-  const T dv = p + dz * vz;
-  const T Rv = p + Rz * vz;               // R . v
-  const T h = c.be * Rv + c.g2 * vz;      // coefficient of -D R
-  const T q = c.C2 * dv;
-  Vec3<T> u;
-  u.x = (c.C1 - c.al) * vx + (q - h) * dx;
-  u.y = (c.C1 - c.al) * vy + (q - h) * dy;
-  u.z = (c.C1 + c.al) * vz + q * dz + h * Rz + c.g1 * Rv + c.de * vz;
-  return u;
-}
 
 struct RadiiMutParams {
   const double* r;
@@ -317,7 +336,11 @@ __global__ __launch_bounds__(kRBlock) void radii_mutual_kernel(RadiiMutParams p)
           const T zj = s_zr[jl];
           const T Rz = zir + zj;
           const CoefRadii<T> c = coef_radii<T>(dx, dy, dz, Rz, zir, zj, ar, s_b[jl], inva, s_ib[jl], BND);
-          const Vec3<T> vi = apply_radii<T>(dx, dy, dz, Rz, c, s_f[0][jl], s_f[1][jl], s_f[2][jl]);
+          // unmasked, the target side's product is seeded with the running sum
+          // where the accumulator allows
+          constexpr bool C = Acc<ACC>::kChain && !MASKED;
+          const Vec3<T> seed{chain_seed<C, T>(u[0]), chain_seed<C, T>(u[1]), chain_seed<C, T>(u[2])};
+          const Vec3<T> vi = apply_radii<T, C>(dx, dy, dz, Rz, c, s_f[0][jl], s_f[1][jl], s_f[2][jl], seed);
           const Vec3<T> vj = apply_radii_t<T>(dx, dy, dz, Rz, c, fi[0], fi[1], fi[2]);
           if constexpr (MASKED) {
             u[0].add(on ? vi.x : T(0));
@@ -327,9 +350,9 @@ __global__ __launch_bounds__(kRBlock) void radii_mutual_kernel(RadiiMutParams p)
             ja[1] = rol1(ja[1]) + (on_j ? (JT)vj.y : JT(0));
             ja[2] = rol1(ja[2]) + (on_j ? (JT)vj.z : JT(0));
           } else {
-            u[0].add(vi.x);
-            u[1].add(vi.y);
-            u[2].add(vi.z);
+            chain_take<C>(u[0], vi.x);
+            chain_take<C>(u[1], vi.y);
+            chain_take<C>(u[2], vi.z);
             ja[0] = rol1(ja[0]) + (JT)vj.x;
             ja[1] = rol1(ja[1]) + (JT)vj.y;
             ja[2] = rol1(ja[2]) + (JT)vj.z;
@@ -372,10 +395,197 @@ __global__ __launch_bounds__(kRBlock) void radii_mutual_kernel(RadiiMutParams p)
   }
 }
 
+// Symmetric kernel on pairs of 64-blob blocks for the middle sizes: work item =
+// (target block I, run of source blocks J >= I); the four waves hold the same
+// 64 targets and share the 64 steps of a block pair (wave v takes 16 v ..
+// 16 v + 15, lane l meeting source (l + s) mod 64 at step s), and their sums
+// of both sides are added through LDS in a fixed order.  A diagonal block
+// takes steps 1..32 (32 for the lower lanes only: s and 64 - s are the same
+// pairs) and wave 0 the self pairs.  The tile kernel's items, 256 x 256 pairs,
+// are too few below some twenty thousand blobs: 820 at 10007 blobs for 256 CUs
+// (203 us there before, 152 with these; FP64 311 and 246).  Bound by the issue
+// of the pair's instructions.
+constexpr int kRB = 64;
+template <int ACC, typename T, int BND>
+__global__ __launch_bounds__(kRBlock) void radii_block_kernel(RadiiMutParams p)
+{
+  using JT = typename std::conditional<ACC == RMW_PREC_F32_BLOCKED, float, double>::type;
+  // each source twice: the rotated read of step s, entry lane + s, needs no wrap
+  __shared__ double s_x[2 * kRB], s_y[2 * kRB], s_z[2 * kRB];
+  __shared__ T s_zr[2 * kRB], s_b[2 * kRB], s_ib[2 * kRB];
+  __shared__ T s_f[3][2 * kRB];
+  __shared__ double s_sum[kRBlock / 64][3][kRB];   // the waves' sums of one side
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  auto write_sums = [&](double* out, int cnt) {
+    const int e = threadIdx.x, l = e / 3, c = e - 3 * l;
+    if (e < 3 * kRB && l < cnt) out[e] = ((s_sum[0][c][l] + s_sum[1][c][l]) + s_sum[2][c][l]) + s_sum[3][c][l];
+  };
+
+  for (int64_t item = blockIdx.x; item < p.total_items; item += gridDim.x) {
+    const int64_t I = pair_target_tile(item, p.n_t, p.chunk_tiles);
+    const int64_t J0 = I + (item - items_before(I, p.n_t, p.chunk_tiles)) * p.chunk_tiles;
+    const int64_t J1 = J0 + p.chunk_tiles < p.n_t ? J0 + p.chunk_tiles : p.n_t;
+    const int icnt = (int)(p.n - I * kRB < kRB ? p.n - I * kRB : kRB);
+    const bool valid = lane < icnt;
+    const int64_t gi = I * kRB + (valid ? lane : 0);
+    const double xi = p.r[3 * gi], yi = p.r[3 * gi + 1];
+    const double a = p.rad[gi];
+    double zi, Bi;
+    wall_shift(p.r[3 * gi + 2], a, BND, zi, Bi);
+    const T ar = (T)a, inva = (T)(1.0 / a), zir = (T)zi;
+    T fi[3];
+    {
+      const double c = valid ? p.norm * Bi : 0.0;
+      fi[0] = (T)(c * p.f[3 * gi]); fi[1] = (T)(c * p.f[3 * gi + 1]); fi[2] = (T)(c * p.f[3 * gi + 2]);
+    }
+    Acc<ACC> u[3];
+
+    for (int64_t J = J0; J < J1; ++J) {
+      const int cnt = (int)(p.n - J * kRB < kRB ? p.n - J * kRB : kRB);
+      __syncthreads();   // the previous block (or item) has been consumed
+      if (wv < 2) {      // both halves of the doubled arrays
+        const bool in = lane < cnt;
+        const int64_t j = J * kRB + (in ? lane : 0);
+        const double b = p.rad[j];
+        double zj, Bj;
+        wall_shift(p.r[3 * j + 2], b, BND, zj, Bj);
+        const double c = p.norm * Bj;
+        const int e = threadIdx.x;
+        // finite stand-ins beyond the system: masked below
+        s_x[e] = in ? p.r[3 * j] : 0.0; s_y[e] = in ? p.r[3 * j + 1] : 0.0; s_z[e] = in ? zj : 1.0;
+        s_zr[e] = in ? (T)zj : T(1); s_b[e] = in ? (T)b : T(1); s_ib[e] = in ? (T)(1.0 / b) : T(1);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) s_f[q][e] = in ? (T)(c * p.f[3 * j + q]) : T(0);
+      }
+      __syncthreads();
+      const bool diag = J == I;
+      const bool full = !diag && cnt == kRB && icnt == kRB;
+      const int st0 = diag ? 1 + 8 * wv : 16 * wv, st1 = st0 + (diag ? 8 : 16);
+      JT ja[3] = {JT(0), JT(0), JT(0)};
+      // on, on_j: the pair is taken on the target side, on the source side
+      auto pair = [&](auto masked_c, int jr, bool on, bool on_j) {
+        constexpr bool MASKED = decltype(masked_c)::value, C = Acc<ACC>::kChain && !MASKED;
+        const T dx = (T)(xi - s_x[jr]), dy = (T)(yi - s_y[jr]), dz = (T)(zi - s_z[jr]);
+        const T zj = s_zr[jr];
+        const T Rz = zir + zj;
+        const CoefRadii<T> c = coef_radii<T>(dx, dy, dz, Rz, zir, zj, ar, s_b[jr], inva, s_ib[jr], BND);
+        const Vec3<T> seed{chain_seed<C, T>(u[0]), chain_seed<C, T>(u[1]), chain_seed<C, T>(u[2])};
+        const Vec3<T> vi = apply_radii<T, C>(dx, dy, dz, Rz, c, s_f[0][jr], s_f[1][jr], s_f[2][jr], seed);
+        const Vec3<T> vj = apply_radii_t<T>(dx, dy, dz, Rz, c, fi[0], fi[1], fi[2]);
+        chain_take<C>(u[0], on ? vi.x : T(0));
+        chain_take<C>(u[1], on ? vi.y : T(0));
+        chain_take<C>(u[2], on ? vi.z : T(0));
+        ja[0] = rol1(ja[0]) + (on_j ? (JT)vj.x : JT(0));
+        ja[1] = rol1(ja[1]) + (on_j ? (JT)vj.y : JT(0));
+        ja[2] = rol1(ja[2]) + (on_j ? (JT)vj.z : JT(0));
+      };
+      if (full) {
+        for (int st = st0; st < st1; ++st) pair(std::false_type{}, lane + st, true, true);
+      } else {
+        if (diag && wv == 0) pair(std::true_type{}, lane, valid, false);   // the self pairs
+        for (int st = st0; st < st1; ++st) {
+          const int jr = lane + st;
+          const bool on = valid && (jr & 63) < cnt && !(diag && st == 32 && lane >= 32);
+          pair(std::true_type{}, jr, on, on);
+        }
+      }
+      u[0].flush(); u[1].flush(); u[2].flush();   // at most kSub + 1 sources since the last fold
+      const int jw = (lane + st1 - 1) & 63;       // the source whose sum this lane holds
+#pragma unroll
+      for (int k = 0; k < 3; ++k) s_sum[wv][k][jw] = (double)ja[k];
+      __syncthreads();
+      write_sums(p.part_j + tri_index(J, I) * kRB * 3, cnt);
+    }
+    __syncthreads();   // the last block's source-side sums have been written out
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s_sum[wv][k][lane] = u[k].get();
+    __syncthreads();
+    write_sums(p.part_i + item * kRB * 3, icnt);
+  }
+}
+
+// Few blobs, one launch (400 blobs: 11 us, the ordered kernel and its reduce
+// 96, one workgroup of which walked 256 sources; bound by launch and latency): a workgroup owns kRDT targets, its 256 threads share
+// the sources (thread t takes t, t + 256, ...), and the 256 partial sums per
+// component are added through LDS in a fixed order and damped.
+template <int ACC, typename T, int BND>
+__global__ __launch_bounds__(kRBlock) void radii_direct_kernel(RadiiParams p, double* __restrict__ out)
+{
+  constexpr int V = 3 * kRDT, kRow = kRBlock + 16;
+  __shared__ double s_part[V][kRow];
+  const int64_t t0 = (int64_t)blockIdx.x * kRDT;
+  double xi[kRDT], yi[kRDT], zi[kRDT], Bi[kRDT];
+  T ar[kRDT], inva[kRDT], zir[kRDT];
+  Acc<ACC> u[kRDT][3];
+#pragma unroll
+  for (int q = 0; q < kRDT; ++q) {
+    const int64_t i = t0 + q < p.nt ? t0 + q : p.nt - 1;
+    const double a = p.rt[i];
+    xi[q] = p.trg[3 * i]; yi[q] = p.trg[3 * i + 1];
+    wall_shift(p.trg[3 * i + 2], a, BND, zi[q], Bi[q]);
+    ar[q] = (T)a; inva[q] = (T)(1.0 / a); zir[q] = (T)zi[q];
+  }
+  int pbox[3];
+  for (int d = 0; d < 3; ++d) pbox[d] = (p.periodic >> d) & 1;
+  int taken = 0;
+  for (int64_t j = threadIdx.x; j < p.ns; j += kRBlock) {
+    const double b = p.rs[j], x = p.src[3 * j], y = p.src[3 * j + 1];
+    double zj, Bj;
+    wall_shift(p.src[3 * j + 2], b, BND, zj, Bj);
+    const double cj = p.norm * Bj;
+    const T br = (T)b, invb = (T)(1.0 / b), zjr = (T)zj;
+    const T f0 = (T)(cj * p.f[3 * j]), f1 = (T)(cj * p.f[3 * j + 1]), f2 = (T)(cj * p.f[3 * j + 2]);
+    ++taken;
+#pragma unroll
+    for (int q = 0; q < kRDT; ++q) {
+      const T Rz = zir[q] + zjr;
+      auto add = [&](T dx, T dy, T dz) {
+        const CoefRadii<T> c = coef_radii<T>(dx, dy, dz, Rz, zir[q], zjr, ar[q], br, inva[q], invb, BND);
+        const Vec3<T> v = apply_radii<T>(dx, dy, dz, Rz, c, f0, f1, f2);
+        u[q][0].add(v.x); u[q][1].add(v.y); u[q][2].add(v.z);
+      };
+      double ddx = xi[q] - x, ddy = yi[q] - y, ddz = zi[q] - zj;
+      if (!p.periodic) {
+        add((T)ddx, (T)ddy, (T)ddz);
+      } else {
+        // as radii_kernel: R_z is not shifted
+        if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
+        if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
+        if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
+        for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
+          for (int by = -pbox[1]; by <= pbox[1]; ++by)
+            for (int bz = -pbox[2]; bz <= pbox[2]; ++bz)
+              add((T)(ddx + bx * p.L[0]), (T)(ddy + by * p.L[1]), (T)(ddz + bz * p.L[2]));
+      }
+    }
+    if (p.periodic || (taken & (kSub - 1)) == 0) {
+#pragma unroll
+      for (int q = 0; q < kRDT; ++q) { u[q][0].flush(); u[q][1].flush(); u[q][2].flush(); }
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < V; ++o) s_part[o][threadIdx.x] = u[o / 3][o % 3].get();
+  __syncthreads();
+  const int o = threadIdx.x >> 4, sub = threadIdx.x & 15;
+  if (o < V) {
+    double s = 0.0;
+#pragma unroll
+    for (int m = 0; m < kRBlock / 16; ++m) s += s_part[o][sub + 16 * m];
+#pragma unroll
+    for (int m = 8; m >= 1; m >>= 1) s += __shfl_xor(s, m, 16);
+    if (sub == 0 && t0 + o / 3 < p.nt) {
+      const int q = o / 3;
+      const double B = q == 0 ? Bi[0] : (q == 1 ? Bi[1] : (q == 2 ? Bi[2] : Bi[3]));
+      out[3 * t0 + o] = B * s;
+    }
+  }
+}
+
 // Blob i of tile X: the target-side sums of the items of tile X and the
 // source-side sums (X, T) for T = 0..X, split over kRRedGroups threads per
 // output whose sums are added in a fixed order; then the damping.
 constexpr int kRRedGroups = 8, kRRedOut = 256 / kRRedGroups;
+template <int BS>   // blobs per tile of the pair kernel: 256 or 64
 __global__ __launch_bounds__(256) void radii_mutual_reduce_kernel(const double* __restrict__ part_i,
                                                                   const double* __restrict__ part_j,
                                                                   const double* __restrict__ r,
@@ -391,11 +601,11 @@ __global__ __launch_bounds__(256) void radii_mutual_reduce_kernel(const double* 
   if (valid) {
     const int64_t i = tid / 3;
     const int c = (int)(tid - 3 * i);
-    const int64_t X = i / kRBlock, l = i - X * kRBlock;
+    const int64_t X = i / BS, l = i - X * BS;
     const int64_t it0 = items_before(X, n_t, chunk_tiles), it1 = items_before(X + 1, n_t, chunk_tiles);
-    const int64_t step = (int64_t)kRBlock * 3;
-    s = group_strided_sum<kRRedGroups>(part_i + (it0 * kRBlock + l) * 3 + c, it1 - it0, step, g) +
-        group_strided_sum<kRRedGroups>(part_j + (tri_index(X, 0) * kRBlock + l) * 3 + c, X + 1, step, g);
+    const int64_t step = (int64_t)BS * 3;
+    s = group_strided_sum<kRRedGroups>(part_i + (it0 * BS + l) * 3 + c, it1 - it0, step, g) +
+        group_strided_sum<kRRedGroups>(part_j + (tri_index(X, 0) * BS + l) * 3 + c, X + 1, step, g);
   }
   part[g][ol] = s;
   __syncthreads();
@@ -413,7 +623,7 @@ __global__ __launch_bounds__(256) void radii_mutual_reduce_kernel(const double* 
 constexpr size_t kRMutAutoBytes = size_t(2) << 30;
 
 struct RadiiSelfPlan {
-  bool mutual = false;
+  bool mutual = false, blocks = false;
   int64_t n_t = 0, chunk_tiles = 0, total_items = 0;
   size_t off_pj = 0, bytes = 0;
   RadiiPlan ordered;
@@ -425,21 +635,25 @@ struct RadiiSelfPlan {
 static RadiiSelfPlan radii_self_plan(int prec, int64_t n, bool periodic, const rmw_tuning* tuning)
 {
   RadiiSelfPlan pl;
-  pl.ordered = radii_plan(prec, n, n, tuning);
+  pl.ordered = radii_plan(prec, n, n, tuning, periodic ? kRDirectPairs : kRDirectSelf);
   const int sym = tuning ? tuning->symmetric : 0;
   const int cu = std::max(device_props().cu_count, 1);
-  pl.n_t = (n + kRBlock - 1) / kRBlock;
+  pl.blocks = !shaped(tuning) && !pl.ordered.direct && !periodic && n <= kRBlockBlobs;
+  const int64_t bs = pl.blocks ? kRB : kRBlock;
+  pl.n_t = (n + bs - 1) / bs;
   const int64_t tile_pairs = pl.n_t * (pl.n_t + 1) / 2;
   RMW_REQUIRE(!(sym > 0 && periodic), "the symmetric radii kernel has no periodic form");
-  pl.mutual = n > 0 && !periodic && sym >= 0 && (sym > 0 || tile_pairs >= cu);
+  pl.mutual = n > 0 && !periodic && sym >= 0 && !pl.ordered.direct && (sym > 0 || pl.blocks || tile_pairs >= cu);
   if (pl.mutual) {
-    if (tuning && tuning->chunk_len > 0)
+    if (pl.blocks)
+      pl.chunk_tiles = tile_pairs <= 12 * (int64_t)cu ? 1 : (tile_pairs <= 144 * (int64_t)cu ? 2 : 4);
+    else if (tuning && tuning->chunk_len > 0)
       pl.chunk_tiles = std::max<int64_t>(1, (tuning->chunk_len + kRBlock - 1) / kRBlock);
     else
       pl.chunk_tiles = std::max<int64_t>(1, tile_pairs / (16 * (int64_t)cu));
     pl.total_items = items_before(pl.n_t, pl.n_t, pl.chunk_tiles);
-    pl.off_pj = align_up((size_t)pl.total_items * kRBlock * 3 * sizeof(double));
-    pl.bytes = pl.off_pj + align_up((size_t)tile_pairs * kRBlock * 3 * sizeof(double));
+    pl.off_pj = align_up((size_t)pl.total_items * bs * 3 * sizeof(double));
+    pl.bytes = pl.off_pj + align_up((size_t)tile_pairs * bs * 3 * sizeof(double));
     if (sym == 0 && pl.bytes > kRMutAutoBytes) pl.mutual = false;
   }
   if (!pl.mutual) pl.bytes = pl.ordered.bytes;
@@ -478,7 +692,25 @@ static void launch_radii_mutual(int prec, dim3 g, dim3 b, hipStream_t st, const 
   else hipLaunchKernelGGL((radii_mutual_kernel<RMW_PREC_F64, double, BND>), g, b, 0, st, q);
 }
 
-// The ordered pair kernel and its reduce, source -> target.
+template <int BND>
+static void launch_radii_block(int prec, dim3 g, dim3 b, hipStream_t st, const RadiiMutParams& q)
+{
+  if (prec == RMW_PREC_F32_F64ACC) hipLaunchKernelGGL((radii_block_kernel<RMW_PREC_F32_F64ACC, float, BND>), g, b, 0, st, q);
+  else if (prec == RMW_PREC_F32_BLOCKED) hipLaunchKernelGGL((radii_block_kernel<RMW_PREC_F32_BLOCKED, float, BND>), g, b, 0, st, q);
+  else if (prec == RMW_PREC_F32_KAHAN) hipLaunchKernelGGL((radii_block_kernel<RMW_PREC_F32_KAHAN, float, BND>), g, b, 0, st, q);
+  else hipLaunchKernelGGL((radii_block_kernel<RMW_PREC_F64, double, BND>), g, b, 0, st, q);
+}
+
+template <int BND>
+static void launch_radii_direct(int prec, dim3 g, dim3 b, hipStream_t st, const RadiiParams& q, double* out)
+{
+  if (prec == RMW_PREC_F32_F64ACC) hipLaunchKernelGGL((radii_direct_kernel<RMW_PREC_F32_F64ACC, float, BND>), g, b, 0, st, q, out);
+  else if (prec == RMW_PREC_F32_BLOCKED) hipLaunchKernelGGL((radii_direct_kernel<RMW_PREC_F32_BLOCKED, float, BND>), g, b, 0, st, q, out);
+  else if (prec == RMW_PREC_F32_KAHAN) hipLaunchKernelGGL((radii_direct_kernel<RMW_PREC_F32_KAHAN, float, BND>), g, b, 0, st, q, out);
+  else hipLaunchKernelGGL((radii_direct_kernel<RMW_PREC_F64, double, BND>), g, b, 0, st, q, out);
+}
+
+// The direct kernel, or the ordered pair kernel and its reduce, source -> target.
 static void radii_ordered(const RadiiPlan& pl, int prec, int bnd, const double* source, const double* target,
                           const double* force, const double* radius_source, const double* radius_target,
                           double* velocity, int64_t ns, int64_t nt, double eta, const double* L,
@@ -504,6 +736,19 @@ static void radii_ordered(const RadiiPlan& pl, int prec, int bnd, const double* 
   ProfRec rec{};
   bool prof = false;
   prof_begin(rec, prof, st, 1);
+  if (pl.direct) {
+    auto over = [&](const double* in, int64_t len) { return overlap(velocity, 3 * nt, in, len); };
+    const bool in_place = over(source, 3 * ns) || over(target, 3 * nt) || over(force, 3 * ns) ||
+                          over(radius_source, ns) || over(radius_target, nt);
+    double* const out = in_place ? (double*)workspace : velocity;
+    if (bnd == kRadiiWall) launch_radii_direct<kRadiiWall>(prec, g, b, st, q, out);
+    else if (bnd == kRadiiFreeSurface) launch_radii_direct<kRadiiFreeSurface>(prec, g, b, st, q, out);
+    else launch_radii_direct<kRadiiUnbounded>(prec, g, b, st, q, out);
+    RMW_CHECK_HIP(hipGetLastError());
+    prof_end(rec, prof, st);
+    if (in_place) launch_copy_rows(out, 3 * nt, velocity, 3 * nt, 3 * nt, 1, st);
+    return;
+  }
   if (bnd == kRadiiWall) launch_radii<kRadiiWall>(prec, g, b, st, q);
   else if (bnd == kRadiiFreeSurface) launch_radii<kRadiiFreeSurface>(prec, g, b, st, q);
   else launch_radii<kRadiiUnbounded>(prec, g, b, st, q);
@@ -601,13 +846,22 @@ extern "C" int rmw_radii_self_apply(int prec, int boundary, const double* r, con
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st, 1);
-    if (boundary == kRadiiWall) launch_radii_mutual<kRadiiWall>(prec, g, b, st, q);
+    if (pl.blocks) {
+      if (boundary == kRadiiWall) launch_radii_block<kRadiiWall>(prec, g, b, st, q);
+      else if (boundary == kRadiiFreeSurface) launch_radii_block<kRadiiFreeSurface>(prec, g, b, st, q);
+      else launch_radii_block<kRadiiUnbounded>(prec, g, b, st, q);
+    } else if (boundary == kRadiiWall) launch_radii_mutual<kRadiiWall>(prec, g, b, st, q);
     else if (boundary == kRadiiFreeSurface) launch_radii_mutual<kRadiiFreeSurface>(prec, g, b, st, q);
     else launch_radii_mutual<kRadiiUnbounded>(prec, g, b, st, q);
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
-    hipLaunchKernelGGL(radii_mutual_reduce_kernel, dim3((unsigned)((n * 3 + kRRedOut - 1) / kRRedOut)), dim3(256), 0,
-                       st, q.part_i, q.part_j, r, radius, q.bnd, n, pl.n_t, pl.chunk_tiles, velocity);
+    const dim3 rg((unsigned)((n * 3 + kRRedOut - 1) / kRRedOut));
+    if (pl.blocks)
+      hipLaunchKernelGGL(radii_mutual_reduce_kernel<kRB>, rg, dim3(256), 0, st, q.part_i, q.part_j, r, radius, q.bnd, n,
+                         pl.n_t, pl.chunk_tiles, velocity);
+    else
+      hipLaunchKernelGGL(radii_mutual_reduce_kernel<kRBlock>, rg, dim3(256), 0, st, q.part_i, q.part_j, r, radius, q.bnd,
+                         n, pl.n_t, pl.chunk_tiles, velocity);
     RMW_CHECK_HIP(hipGetLastError());
   });
 }
