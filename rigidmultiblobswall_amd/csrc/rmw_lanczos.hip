@@ -5,23 +5,32 @@
 // (i+1) x (i+1) tridiagonal h every iteration, takes numpy.linalg.eigh,
 // replaces negative eigenvalues by 0 and evaluates
 //   noise = V^T Q (|z| factor sqrt(lambda) * Q^T e_1).
-// Here the eigen-decomposition is the implicit QL method with Wilkinson
-// shifts (Bowdler, Martin, Reinsch & Wilkinson, Numer. Math. 11 (1968) 293,
-// the algorithm behind EISPACK tql2), run by one wavefront per right-hand
-// side: the scalar recurrence is evaluated redundantly by all 64 lanes, each
-// plane rotation is applied to the eigenvector columns with the lanes spread
-// over rows.  The kernel is one dependent chain, so it is bound by the latency
-// of a rotation.  Up to 64 steps the tridiagonal lives in the lanes'
-// registers, the search for a negligible off-diagonal is one ballot, the
-// eigenvectors are in LDS with their next column read ahead, and
-// 1/sqrt(f^2 + g^2) is the refined hardware estimate of the pair terms (with
-// all of it in memory, a correctly rounded hypot and two divisions the launch
-// took 35 us on average over 11 Lanczos steps, with d and e in LDS 24, now 20).
+// Here sqrt(T) e_1 is a quadrature: sqrt(l) = (2/pi) int l / (l + t^2) dt over
+// t > 0, and with t = sqrt(M) e^x (M >= every eigenvalue) the trapezoidal rule
+// of step h is off by 2 exp(-pi^2 / h) of sqrt(l) for every l >= 0, plus
+// sqrt(M) e^-37 from |x| > 37: 320 nodes reach the last bits of a double
+// whatever the condition of T.  The nodes are independent tridiagonal solves
+// (T + t^2) x = e_1, one per thread: 2 m short steps instead of the ~m^2
+// dependent plane rotations of a QL sweep.  l / (l + s) is taken as
+// 1 - s / (l + s) for s < M and as T (T + s)^-1 beyond, so that no term loses
+// digits.  Error of c in units of |c| against 50 digits, this / eigh: 11 steps
+// at condition 1e4 4e-16 / 5e-15, 25 at 1e6 3e-16 / 1e-14, 40 at 1e13
+// 1e-14 / 3e-12.  One T of
+// 11 steps takes 6 us, of 60 14, of 100 47, of 400 141 (the QL sweeps, bound by
+// the latency of their rotations, took 20 us on average over 11 steps with T in
+// registers, 8.0 ms at 100 steps and 254 ms at 400 with T in memory).
+// A T with an eigenvalue <= 0 (a negative pivot in a solve) or not finite takes
+// the eigen-decomposition instead: implicit QL with Wilkinson shifts (Bowdler,
+// Martin, Reinsch & Wilkinson, Numer. Math. 11 (1968) 293, the algorithm
+// behind EISPACK tql2) by the first wavefront, the scalar recurrence evaluated
+// redundantly by all 64 lanes and the rotations applied to the eigenvector
+// columns with the lanes spread over rows.
 // The kernel returns the coefficient vector c (noise = V c), not the noise
 // itself.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <algorithm>
 #include <cmath>
 
 #include "rmw_internal.h"
@@ -171,53 +180,139 @@ __device__ int tridiag_ql(int m, double* d, double* e, double* __restrict__ Z)
   return 0;
 }
 
+// 1 / d for positive d of ordinary size
+__device__ __forceinline__ double reciprocal(double d)
+{
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return fma(y, fma(-d, y, 1.0), y);
+}
+
+constexpr int kQuadNodes = 320, kQuadWaves = kQuadNodes / 64;
+constexpr double kQuadRange = 37.0;
+constexpr double kQuadLow = 0.635203471872816;   // the weights of the first half's nodes, over sqrt(M)
+// Nodes taken at a time by `waves` wavefronts, and the row length in which
+// their solutions are kept (padded: rows start in different LDS banks).
+__host__ __device__ constexpr int quad_row(int waves) { return 64 * waves + 8; }
+
 // H of right-hand side r starts at H + r * h_rhs_stride; Lanczos step i wrote
 // alpha_i = H[i * ldh + i] and beta_i = H[i * ldh + i + 1].  test (may be
 // null): |c - c_prev|, |c_prev| and the status of every right-hand side, with
-// c_prev the m - 1 coefficients that c_out held before.  LANES: m <= 64, the
-// eigenvectors in LDS.
-template <bool LANES>
-__global__ __launch_bounds__(64) void tridiag_sqrt_e1_kernel(const double* __restrict__ H, int64_t h_rhs_stride,
-                                                             int64_t ldh, int m, const double* __restrict__ scale,
+// c_prev the m - 1 coefficients that c_out held before.  LDS (dynamic): a, b,
+// the sums P and Q (m each), then the solutions x_0 .. x_(m-1) of 64 * waves
+// nodes, which with MEM are in the scratch array instead (it holds m^2).
+template <bool MEM>
+__global__ __launch_bounds__(kQuadNodes) void sqrt_e1_kernel(const double* __restrict__ H, int64_t h_rhs_stride,
+                                                             int64_t ldh, int m, int waves,
+                                                             const double* __restrict__ scale,
                                                              double* __restrict__ c_out, int64_t c_stride,
                                                              double* __restrict__ zscratch, int* __restrict__ status,
                                                              double* __restrict__ test)
 {
-  extern __shared__ double s_z[];
-  __shared__ double d[LANES ? 64 : kMaxLanczos], e[LANES ? 1 : kMaxLanczos];
-  const int r = blockIdx.x;
-  const int lane = threadIdx.x;
+  extern __shared__ double sm[];
+  __shared__ double s_max[kQuadWaves], s_red[2][kQuadWaves];
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  double *const a = sm, *const b = a + m, *const P = b + m, *const Q = P + m;
+  double* const Z = MEM ? zscratch + (int64_t)r * m * m : Q + m;
   const double* Hr = H + r * h_rhs_stride;
-  double* Z = LANES ? s_z : zscratch + (int64_t)r * m * m;
-  for (int idx = lane; idx < m * m; idx += 64) Z[idx] = (idx % (m + 1) == 0) ? 1.0 : 0.0;
-  int fail;
-  if constexpr (LANES) {
-    double dv = lane < m ? Hr[(int64_t)lane * ldh + lane] : 0.0;
-    double ev = lane + 1 < m ? Hr[(int64_t)lane * ldh + lane + 1] : 0.0;
-    __syncthreads();
-    fail = tridiag_ql_lanes(m, dv, ev, Z);
-    d[lane] = dv;
-  } else {
-    for (int i = lane; i < m; i += 64) {
-      d[i] = Hr[(int64_t)i * ldh + i];
-      e[i] = (i + 1 < m) ? Hr[(int64_t)i * ldh + i + 1] : 0.0;
+  double top = 0.0;   // Gershgorin
+  bool ok = true;
+  for (int i = tid; i < m; i += kQuadNodes) {
+    const double* row = Hr + (int64_t)i * ldh + i;
+    const double ai = row[0], bi = i + 1 < m ? row[1] : 0.0, bp = i > 0 ? row[-ldh] : 0.0;
+    a[i] = ai;
+    b[i] = bi;
+    P[i] = 0.0;
+    Q[i] = 0.0;
+    const double g = fabs(ai) + fabs(bi) + fabs(bp);
+    ok = ok && g < 1e140;
+    top = fmax(top, g);
+  }
+  for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
+  if (lane == 0) s_max[wv] = top;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kQuadWaves; ++w) top = fmax(top, s_max[w]);
+  ok = ok && top > 1e-140;   // (b^2 and M e^74 stay ordinary numbers)
+
+  constexpr double h = 2.0 * kQuadRange / kQuadNodes;
+  const int ns = quad_row(waves);
+  for (int n0 = 0; n0 < kQuadNodes; n0 += 64 * waves) {
+    const int node = n0 + tid;
+    if (wv < waves && node < kQuadNodes) {
+      const double t = sqrt(top) * exp((node - 0.5 * (kQuadNodes - 1)) * h);
+      const double s = t * t, w = (2.0 / M_PI) * h * t;
+      const bool low = node < kQuadNodes / 2;
+      double* x = Z + tid;
+      // pivots from the last row up, then the solution from the first down
+      double inv = 0.0, bi = 0.0;
+#pragma unroll 4
+      for (int i = m - 1; i >= 0; --i) {
+        const double d = fma(-bi * bi, inv, a[i] + s);
+        ok = ok && d > 0.0;
+        inv = reciprocal(d);
+        x[(int64_t)i * ns] = inv;
+        bi = i > 0 ? b[i - 1] : 0.0;
+      }
+      double xi = low ? w * s * inv : w * inv;
+      x[0] = xi;
+#pragma unroll 4
+      for (int i = 1; i < m; ++i) {
+        xi = -b[i - 1] * xi * x[(int64_t)i * ns];
+        x[(int64_t)i * ns] = xi;
+      }
     }
     __syncthreads();
-    fail = tridiag_ql(m, d, e, Z);
-  }
-  // sqrt+(lambda) times the first components, which lane 0's row holds
-  __syncthreads();
-  for (int k = lane; k < m; k += 64) {
-    const double lam = d[k];
-    d[k] = (lam > 0.0 ? sqrt(lam) : 0.0) * Z[(int64_t)k * m];
-  }
-  __syncthreads();
-  const double sc = scale[r];
-  double diff = 0.0, prev = 0.0;
-  for (int j = lane; j < m; j += 64) {
-    double acc = 0.0;
+    // sums over the nodes of each half, eight threads each
+    const int n1 = n0 + 64 * waves < kQuadNodes ? n0 + 64 * waves : kQuadNodes;
+    for (int task = tid >> 3; task < 2 * m; task += kQuadNodes / 8) {
+      const int i = task >> 1, half = task & 1;
+      const int lo = half ? (n0 > kQuadNodes / 2 ? n0 : kQuadNodes / 2) : n0;
+      const int hi = half ? n1 : (n1 < kQuadNodes / 2 ? n1 : kQuadNodes / 2);
+      const double* x = Z + (int64_t)i * ns - n0;
+      double sum = 0.0;
 #pragma unroll 4
-    for (int k = 0; k < m; ++k) acc += Z[(int64_t)k * m + j] * d[k];
+      for (int q = lo + (tid & 7); q < hi; q += 8) sum += x[q];
+      for (int o = 4; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 8);
+      if ((tid & 7) == 0) (half ? Q : P)[i] += sum;
+    }
+    __syncthreads();
+  }
+  int fail = 0;
+  const bool quad = __syncthreads_and(ok);
+  double* const E = m <= 64 && !MEM ? Z : zscratch + (int64_t)r * m * m;   // eigenvectors
+  if (!quad) {
+    double *d = P, *e = Q;
+    for (int idx = tid; idx < m * m; idx += kQuadNodes) E[idx] = (idx % (m + 1) == 0) ? 1.0 : 0.0;
+    for (int i = tid; i < m; i += kQuadNodes) { d[i] = a[i]; e[i] = b[i]; }
+    __syncthreads();
+    if (wv == 0) {
+      if (m <= 64 && !MEM) {
+        double dv = lane < m ? d[lane] : 0.0, ev = lane < m ? e[lane] : 0.0;
+        fail = tridiag_ql_lanes(m, dv, ev, E);
+        if (lane < m) d[lane] = dv;
+      } else {
+        fail = tridiag_ql(m, d, e, E);
+      }
+    }
+    __syncthreads();
+    // sqrt+(lambda) times the first components, which row 0 holds
+    for (int k = tid; k < m; k += kQuadNodes) d[k] = (d[k] > 0.0 ? sqrt(d[k]) : 0.0) * E[(int64_t)k * m];
+    __syncthreads();
+  }
+  const double sc = scale[r], first = kQuadLow * sqrt(top);
+  double diff = 0.0, prev = 0.0;
+  for (int j = tid; j < m; j += kQuadNodes) {
+    double acc;
+    if (quad) {   // e_1 sum(w) - sum(w s x) over s < M, + T sum(w x) over s >= M
+      acc = fma(a[j], Q[j], (j == 0 ? first : 0.0) - P[j]);
+      if (j > 0) acc = fma(b[j - 1], Q[j - 1], acc);
+      if (j + 1 < m) acc = fma(b[j], Q[j + 1], acc);
+    } else {
+      acc = 0.0;
+#pragma unroll 4
+      for (int k = 0; k < m; ++k) acc += E[(int64_t)k * m + j] * P[k];
+    }
     const double now = sc * acc;
     if (test) {
       const double old = j < m - 1 ? c_out[r * c_stride + j] : 0.0;
@@ -231,28 +326,45 @@ __global__ __launch_bounds__(64) void tridiag_sqrt_e1_kernel(const double* __res
       diff += __shfl_xor(diff, o, 64);
       prev += __shfl_xor(prev, o, 64);
     }
-    if (lane == 0) {
-      test[3 * r] = sqrt(diff);
-      test[3 * r + 1] = sqrt(prev);
-      test[3 * r + 2] = (double)fail;
+    if (lane == 0) { s_red[0][wv] = diff; s_red[1][wv] = prev; }
+    __syncthreads();
+    if (tid < 2) {
+      double v = s_red[tid][0];
+#pragma unroll
+      for (int w = 1; w < kQuadWaves; ++w) v += s_red[tid][w];
+      test[3 * r + tid] = sqrt(v);
     }
+    if (tid == 0) test[3 * r + 2] = (double)fail;
   }
-  if (lane == 0 && status) status[r] = fail;
+  if (tid == 0 && status) status[r] = fail;
 }
 
-static void launch_tridiag(const double* H, int64_t h_rhs_stride, int64_t ldh, int m, int k, const double* scale,
+static void launch_sqrt_e1(const double* H, int64_t h_rhs_stride, int64_t ldh, int m, int k, const double* scale,
                            double* c_out, int64_t c_stride, double* scratch, size_t scratch_doubles, int* status,
                            double* test, hipStream_t st)
 {
   RMW_REQUIRE(m >= 1 && m <= kMaxLanczos && k >= 1, "bad sizes");
   RMW_REQUIRE(ldh >= m + 1 && c_stride >= m, "bad strides");
   RMW_REQUIRE(scratch && scratch_doubles >= (size_t)k * m * m, "scratch too small");
-  if (m <= 64)
-    hipLaunchKernelGGL(tridiag_sqrt_e1_kernel<true>, dim3(k), dim3(64), (size_t)m * m * sizeof(double), st, H,
-                       h_rhs_stride, ldh, m, scale, c_out, c_stride, scratch, status, test);
-  else
-    hipLaunchKernelGGL(tridiag_sqrt_e1_kernel<false>, dim3(k), dim3(64), 0, st, H, h_rhs_stride, ldh, m, scale, c_out,
-                       c_stride, scratch, status, test);
+  // as many nodes at a time as their solutions fit into LDS (all up to 60
+  // steps, 64 up to 266), then into the scratch array's m doubles per row
+  constexpr int kLdsDoubles = 159 * 1024 / 8;
+  int waves = kQuadWaves;
+  while (waves > 0 && (4 + quad_row(waves)) * m > kLdsDoubles) --waves;
+  const bool mem = waves == 0;
+  if (mem) waves = std::min(kQuadWaves, (m - 8) / 64);
+  const size_t lds = sizeof(double) * (size_t)m * (4 + (mem ? 0 : quad_row(waves)));
+  const dim3 g(k), bl(kQuadNodes);
+  if (mem) {
+    hipLaunchKernelGGL(sqrt_e1_kernel<true>, g, bl, lds, st, H, h_rhs_stride, ldh, m, waves, scale, c_out, c_stride,
+                       scratch, status, test);
+  } else {
+    if (lds > 64 * 1024)
+      RMW_CHECK_HIP(hipFuncSetAttribute((const void*)sqrt_e1_kernel<false>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsDoubles * 8));
+    hipLaunchKernelGGL(sqrt_e1_kernel<false>, g, bl, lds, st, H, h_rhs_stride, ldh, m, waves, scale, c_out, c_stride,
+                       scratch, status, test);
+  }
   RMW_CHECK_HIP(hipGetLastError());
 }
 
@@ -275,7 +387,7 @@ extern "C" int rmw_lanczos_sqrt_coeffs(const double* H, int64_t h_rhs_stride, in
                                        size_t scratch_doubles, int* status, void* stream)
 {
   return guarded([&] {
-    launch_tridiag(H, h_rhs_stride, ldh, m, k, scale, c_out, c_stride, scratch, scratch_doubles, status, nullptr,
+    launch_sqrt_e1(H, h_rhs_stride, ldh, m, k, scale, c_out, c_stride, scratch, scratch_doubles, status, nullptr,
                    (hipStream_t)stream);
   });
 }
@@ -289,7 +401,7 @@ extern "C" int rmw_lanczos_step_coeffs(const double* H, int64_t h_rhs_stride, in
 {
   return guarded([&] {
     RMW_REQUIRE(test != nullptr, "test is null");
-    launch_tridiag(H, h_rhs_stride, ldh, m, k, scale, c_out, c_stride, scratch, scratch_doubles, nullptr, test,
+    launch_sqrt_e1(H, h_rhs_stride, ldh, m, k, scale, c_out, c_stride, scratch, scratch_doubles, nullptr, test,
                    (hipStream_t)stream);
   });
 }

@@ -135,3 +135,33 @@ def test_preconditioner_of_bodies_of_every_block_size(gpu, sizes):
         assert np.abs(ys[3 * off:3 * off + n] - lam).max() <= 1e-9 * np.abs(Mi @ s).max()
         off += nb
         moff += n * n
+
+
+@pytest.mark.parametrize("m", [1, 59, 60, 61, 78, 79, 156, 157, 267, 268, 269, 327, 328, 400])
+def test_square_root_storage_edges(gpu, m):
+    """Sizes at which fewer nodes fit into LDS at a time, or none, for a
+    positive definite T and one with a negative eigenvalue."""
+    print(f"case square root m={m}", flush=True)
+    lib = _lib.load()
+    rng = np.random.default_rng(m)
+    k = 2
+    a, b = rng.uniform(2.5, 30.0, (k, m)), rng.uniform(0.0, 1.2, (k, m))
+    a[1, m // 2] = -4.0
+    H = torch.zeros((k, m, m + 1), dtype=torch.float64)
+    want = []
+    for r in range(k):
+        T = np.diag(a[r]) + np.diag(b[r, :-1], 1) + np.diag(b[r, :-1], -1)
+        lam, Q = np.linalg.eigh(T)
+        want.append(Q @ (np.sqrt(np.maximum(lam, 0)) * Q[0]))
+        H[r, np.arange(m), np.arange(m)] = torch.from_numpy(a[r])
+        H[r, np.arange(m), np.arange(m) + 1] = torch.from_numpy(b[r])
+    H = H.to(gpu)
+    C = torch.zeros((k, m), dtype=torch.float64, device=gpu)
+    sc = torch.ones(k, dtype=torch.float64, device=gpu)
+    status = torch.full((k,), 7, dtype=torch.int32, device=gpu)
+    scr = torch.empty(k * m * m, dtype=torch.float64, device=gpu)
+    _lib.check(lib.rmw_lanczos_sqrt_coeffs(H.data_ptr(), H.stride(0), H.stride(1), m, k, sc.data_ptr(), C.data_ptr(), m,
+                                           scr.data_ptr(), scr.numel(), status.data_ptr(), _stream()))
+    assert status.tolist() == [0, 0]
+    for r in range(k):
+        assert np.linalg.norm(C[r].cpu().numpy() - want[r]) <= 1e-13 * max(np.linalg.norm(want[r]), 1.0)
