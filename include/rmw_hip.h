@@ -165,6 +165,19 @@ int rmw_mobility_apply(int domain, int mask, int prec, const double* r_vectors, 
                        size_t workspace_bytes, void* stream);
 
 /*
+ * One product between pinned host buffers (hipHostMalloc), returning when the
+ * outputs are there: in = r, then force and torque as the mask takes them,
+ * out = velocity and omega as it gives them, 3 n doubles each.  The workspace
+ * (device memory) holds the product's own and a copy of in;
+ * rmw_mobility_host_workspace_size gives its size.
+ */
+int rmw_mobility_host_workspace_size(int domain, int mask, int prec, int64_t n, const rmw_tuning* tuning,
+                                     size_t* bytes);
+int rmw_mobility_apply_host(int domain, int mask, int prec, const double* in, double* out, int64_t n, double eta,
+                            double a, const double* L, const rmw_tuning* tuning, void* workspace,
+                            size_t workspace_bytes, void* stream);
+
+/*
  * The launch plan rmw_wall_rpy_apply would use for these sizes (periodic:
  * whether L has a positive entry): which kernel, the right-hand sides per
  * pass, the source chunk and the number of work items.  No reference
@@ -470,6 +483,10 @@ int rmw_axpby(double alpha, const double* x, double beta, double* y, int64_t n, 
  * h[0..j] = coefficients, h[j+1] = ||w||, V[j+1] = w / ||w||. */
 int rmw_arnoldi_cgs2(double* V, int64_t ldv, int j, double* w, int64_t n, double* h,
                      double* hscratch, void* workspace, size_t workspace_bytes, void* stream);
+/* The same, h[0..j+1] also written to pinned host memory, where it may be
+ * read after a wait for the stream. */
+int rmw_arnoldi_cgs2_host(double* V, int64_t ldv, int j, double* w, int64_t n, double* h, double* h_host,
+                          double* hscratch, void* workspace, size_t workspace_bytes, void* stream);
 /* The same step for k bases in the same launches: basis r at V + r * v_rhs,
  * its candidate at w + r * w_rhs, its coefficients at h + r * h_rhs. */
 int rmw_arnoldi_cgs2_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, double* w, int64_t w_rhs,

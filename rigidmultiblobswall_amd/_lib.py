@@ -97,6 +97,9 @@ PROTOTYPES = {
     "rmw_mobility_apply": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _dp, _dp, _dp, _dp, _dp, _i64,
                                           ctypes.c_int, _i64, ctypes.c_double, ctypes.c_double, _hdp, _tp, _vp, _sz,
                                           _vp]),
+    "rmw_mobility_host_workspace_size": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _i64, _tp, _szp]),
+    "rmw_mobility_apply_host": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _dp, _dp, _i64,
+                                               ctypes.c_double, ctypes.c_double, _hdp, _tp, _vp, _sz, _vp]),
     "rmw_rigid_force_torque": (ctypes.c_int, [_dp, _i64p, ctypes.c_int, _dp, _dp, _vp, _sz, _vp]),
     "rmw_bodies_advance": (ctypes.c_int, [_dp, _dp, _dp, _dp, ctypes.c_int, ctypes.c_double, ctypes.c_double,
                                           ctypes.c_double, _dp, _dp, _vp]),
@@ -144,6 +147,7 @@ PROTOTYPES = {
     "rmw_combination": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _dp, _i64, ctypes.c_int, _vp]),
     "rmw_axpby": (ctypes.c_int, [ctypes.c_double, _dp, ctypes.c_double, _dp, _i64, _dp, _vp]),
     "rmw_arnoldi_cgs2": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _i64, _dp, _dp, _vp, _sz, _vp]),
+    "rmw_arnoldi_cgs2_host": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _i64, _dp, _dp, _dp, _vp, _sz, _vp]),
     # segmented (ragged-batch) Krylov kernels
     "rmw_seg_workspace_size": (ctypes.c_int, [_sgp, ctypes.c_int, _szp]),
     "rmw_seg_dot_many": (ctypes.c_int, [_dp, _i64, ctypes.c_int, _dp, _sgp, _dp, _i64, ctypes.c_int, _vp, _sz, _vp]),

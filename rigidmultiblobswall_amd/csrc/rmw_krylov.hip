@@ -171,6 +171,7 @@ struct ArnoldiParams {
   int64_t w_rhs, n;
   double* h;            // coefficients r at h + r * h_rhs
   int64_t h_rhs;
+  double* h_host;       // pinned host copy of h of basis 0, or null
   double* part;         // per basis: part1 [m][G], part2 [m][G], part3 [G]
   int64_t part_rhs;
   int m;                // vectors in the basis
@@ -247,7 +248,10 @@ __global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
   } else if constexpr (PASS == 3) {
     block_coefs(part3, G, 1, coef);
     const double norm = sqrt(coef[0]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) h[p.m] = norm;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      h[p.m] = norm;
+      if (p.h_host) p.h_host[p.m] = norm;
+    }
     const double al = norm > 0.0 ? 1.0 / norm : 0.0;
     double* v = V + (int64_t)p.m * p.ldv;
 #pragma unroll
@@ -258,7 +262,11 @@ __global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
   } else {
     block_coefs(PASS == 1 ? part1 : part2, G, p.m, coef);
     if (blockIdx.x == 0)
-      for (int j = threadIdx.x; j < p.m; j += kKBlock) h[j] = PASS == 1 ? coef[j] : h[j] + coef[j];
+      for (int j = threadIdx.x; j < p.m; j += kKBlock) {
+        const double v = PASS == 1 ? coef[j] : h[j] + coef[j];
+        h[j] = v;
+        if (PASS == 2 && p.h_host) p.h_host[j] = v;
+      }
 #pragma unroll 4
     for (int j = 0; j < p.m; ++j) {
       const double* v = V + (int64_t)j * p.ldv;
@@ -442,7 +450,7 @@ static void arnoldi_separate(const DotLaunch& L, hipStream_t st, double* V, int6
 
 static void arnoldi_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, double* w, int64_t w_rhs, int64_t n,
                           double* h, int64_t h_rhs, double* hscratch, void* workspace, size_t workspace_bytes,
-                          hipStream_t st)
+                          hipStream_t st, double* h_host = nullptr)
 {
   const int m = j + 1;
   RMW_REQUIRE(m >= 1 && m + 1 <= kMaxVec, "bad Arnoldi index");
@@ -455,7 +463,7 @@ static void arnoldi_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, d
     const int fit = (int)std::min<int64_t>(k, (int64_t)(workspace_bytes / sizeof(double)) / per);
     for (int r0 = 0; r0 < k; r0 += fit) {
       ArnoldiParams p{V + r0 * v_rhs, ldv, v_rhs, w + r0 * w_rhs, w_rhs, n, h + r0 * h_rhs, h_rhs,
-                      (double*)workspace, per, m};
+                      h_host, (double*)workspace, per, m};
       const int kk = std::min(fit, k - r0);
       switch (L.E) {
         case 1: launch_arnoldi<1>(p, L.G, kk, st); break;
@@ -467,6 +475,7 @@ static void arnoldi_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, d
   } else {
     for (int r = 0; r < k; ++r)
       arnoldi_separate(L, st, V + r * v_rhs, ldv, m, w + r * w_rhs, n, h + r * h_rhs, hscratch, (double*)workspace);
+    if (h_host) RMW_CHECK_HIP(hipMemcpyAsync(h_host, h, (m + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
   }
   RMW_CHECK_HIP(hipGetLastError());
 }
@@ -480,6 +489,17 @@ extern "C" int rmw_arnoldi_cgs2(double* V, int64_t ldv, int j, double* w, int64_
 {
   return guarded([&] {
     arnoldi_batch(V, ldv, 0, j, 1, w, 0, n, h, 0, hscratch, workspace, workspace_bytes, (hipStream_t)stream);
+  });
+}
+
+// rmw_arnoldi_cgs2, also leaving h[0..j+1] in pinned host memory, where it may
+// be read once the stream has been waited for: no copy behind the kernels.
+extern "C" int rmw_arnoldi_cgs2_host(double* V, int64_t ldv, int j, double* w, int64_t n, double* h, double* h_host,
+                                     double* hscratch, void* workspace, size_t workspace_bytes, void* stream)
+{
+  return guarded([&] {
+    RMW_REQUIRE(h_host != nullptr, "h_host is null");
+    arnoldi_batch(V, ldv, 0, j, 1, w, 0, n, h, 0, hscratch, workspace, workspace_bytes, (hipStream_t)stream, h_host);
   });
 }
 

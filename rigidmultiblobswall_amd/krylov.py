@@ -91,6 +91,14 @@ class KrylovOps:
         _lib.check(self.lib.rmw_arnoldi_cgs2(V.data_ptr(), V.stride(0), j, w.data_ptr(), self.n, h.data_ptr(),
                                              hs.data_ptr(), self.ws.data_ptr(), self.ws.numel(), _stream()))
 
+    def arnoldi_host(self, V: torch.Tensor, j: int, w: torch.Tensor, h: torch.Tensor, h_host: torch.Tensor,
+                     hs: torch.Tensor):
+        """arnoldi(), the column also written to the pinned h_host (to be
+        read after a wait for the stream)."""
+        _lib.check(self.lib.rmw_arnoldi_cgs2_host(V.data_ptr(), V.stride(0), j, w.data_ptr(), self.n, h.data_ptr(),
+                                                  h_host.data_ptr(), hs.data_ptr(), self.ws.data_ptr(),
+                                                  self.ws.numel(), _stream()))
+
 
 def gmres(A: Callable[[torch.Tensor, torch.Tensor], None], b: torch.Tensor,
           Pinv: Optional[Callable[[torch.Tensor, torch.Tensor], None]] = None,
@@ -116,8 +124,8 @@ def gmres(A: Callable[[torch.Tensor, torch.Tensor], None], b: torch.Tensor,
     h = torch.empty(m + 2, dtype=torch.float64, device=device)
     hs = torch.empty(m + 2, dtype=torch.float64, device=device)
     ycoef = torch.empty(m + 1, dtype=torch.float64, device=device)
-    # pinned host copy of the Arnoldi column: one short copy and a stream
-    # synchronisation per step
+    # pinned host copy of the Arnoldi column, which the step's kernels write:
+    # one stream synchronisation per step
     stream = torch.cuda.current_stream(device)
     h_host = _pinned_column(m + 2, stream.cuda_stream)
     x = torch.zeros(n, dtype=torch.float64, device=device) if x0 is None else x0.clone()
@@ -160,8 +168,7 @@ def gmres(A: Callable[[torch.Tensor, torch.Tensor], None], b: torch.Tensor,
                 Pinv(V[j], z)
                 A(z, w)
             res.matvecs += 1
-            ops.arnoldi(V, j, w, h, hs)
-            h_host[: j + 2].copy_(h[: j + 2], non_blocking=True)
+            ops.arnoldi_host(V, j, w, h, h_host, hs)
             stream.synchronize()
             col = h_host[: j + 2].tolist()
             hnext = col[j + 1]

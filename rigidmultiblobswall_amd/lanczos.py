@@ -94,9 +94,8 @@ def lanczos_block(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torch
     scale = znorm * factor
     nscr = ctypes.c_size_t()
     # scratch of the tridiagonal solve (k m^2 doubles), grown geometrically,
-    # and the stop test's numbers with a pinned host copy
+    # and the stop test's numbers, which the kernel writes to pinned memory
     zscr = None
-    test = torch.empty((k, 3), dtype=torch.float64, device=dev)
     t_host = torch.empty((k, 3), dtype=torch.float64, pin_memory=True)
     t_np = t_host.numpy()
     eps = np.finfo(float).eps
@@ -123,9 +122,8 @@ def lanczos_block(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torch
             zscr = torch.empty(nscr.value, dtype=torch.float64, device=dev)
         _lib.check(lib.rmw_lanczos_step_coeffs(H.data_ptr(), H.stride(0), H.stride(1), m, k, scale.data_ptr(),
                                                C.data_ptr(), C.stride(0), zscr.data_ptr(), zscr.numel(),
-                                               test.data_ptr(), _stream()))
-        # one read-back per step: the change of the coefficients and the QL status
-        t_host.copy_(test, non_blocking=True)
+                                               t_host.data_ptr(), _stream()))
+        # one wait per step: the change of the coefficients and the status
         stream.synchronize()
         if t_np[:, 2].any():
             raise RuntimeError("tridiagonal eigen-solve did not converge")

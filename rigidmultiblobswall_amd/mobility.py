@@ -66,34 +66,42 @@ def _host(t):
     return t.reshape(-1).cpu().numpy()
 
 
+def _product(domain, mask, r_vectors, force, torque, eta, a, kwargs):
+    """The product as one host array (velocity, then omega)."""
+    opts = _apply_opts(kwargs)
+    if not opts["check_finite"]:
+        out = wall_rpy.apply_host(mask, r_vectors, force, torque, eta, a, opts["periodic_length"], opts["precision"],
+                                  opts["tuning"], domain)
+        if out is not None:
+            return out
+    outs = wall_rpy.apply(mask, r_vectors, force=force, torque=torque, eta=eta, a=a, domain=domain, **opts)
+    outs = [_host(t) for t in outs if t is not None]
+    return outs[0] if len(outs) == 1 else np.concatenate(outs)
+
+
 def single_wall_mobility_trans_times_force_hip(r_vectors, force, eta, a, *args, **kwargs):
     """u = B M_UF(z_eff) B f; drop-in for mobility.py:1132-1163."""
-    u, _ = wall_rpy.apply(RMW_UF, r_vectors, force=force, eta=eta, a=a, **_apply_opts(kwargs))
-    return _host(u)
+    return _product("single_wall", RMW_UF, r_vectors, force, None, eta, a, kwargs)
 
 
 def single_wall_mobility_trans_times_torque_hip(r_vectors, torque, eta, a, *args, **kwargs):
     """u = B M_UT(z_eff) B t; drop-in for mobility.py:1213-1232."""
-    u, _ = wall_rpy.apply(RMW_UT, r_vectors, torque=torque, eta=eta, a=a, **_apply_opts(kwargs))
-    return _host(u)
+    return _product("single_wall", RMW_UT, r_vectors, None, torque, eta, a, kwargs)
 
 
 def single_wall_mobility_rot_times_force_hip(r_vectors, force, eta, a, *args, **kwargs):
     """w = B M_WF(z_eff) B f; drop-in for mobility.py:1273-1298."""
-    _, w = wall_rpy.apply(RMW_WF, r_vectors, force=force, eta=eta, a=a, **_apply_opts(kwargs))
-    return _host(w)
+    return _product("single_wall", RMW_WF, r_vectors, force, None, eta, a, kwargs)
 
 
 def single_wall_mobility_rot_times_torque_hip(r_vectors, torque, eta, a, *args, **kwargs):
     """w = B M_WT(z_eff) B t; drop-in for mobility.py:1316-1342."""
-    _, w = wall_rpy.apply(RMW_WT, r_vectors, torque=torque, eta=eta, a=a, **_apply_opts(kwargs))
-    return _host(w)
+    return _product("single_wall", RMW_WT, r_vectors, None, torque, eta, a, kwargs)
 
 
 def single_wall_mobility_trans_times_force_torque_hip(r_vectors, force, torque, eta, a, *args, **kwargs):
     """u = M_UF f + M_UT t in one pass; drop-in for mobility.py:384-410."""
-    u, _ = wall_rpy.apply(RMW_UF | RMW_UT, r_vectors, force=force, torque=torque, eta=eta, a=a, **_apply_opts(kwargs))
-    return _host(u)
+    return _product("single_wall", RMW_UF | RMW_UT, r_vectors, force, torque, eta, a, kwargs)
 
 
 def single_wall_grand_mobility_hip(r_vectors, force_torque, eta, a, *args, **kwargs):
@@ -103,15 +111,7 @@ def single_wall_grand_mobility_hip(r_vectors, force_torque, eta, a, *args, **kwa
     ft = np.asarray(force_torque, dtype=np.float64).reshape(-1) if not torch.is_tensor(force_torque) \
         else force_torque.reshape(-1)
     half = ft.shape[0] // 2
-    u, w = wall_rpy.apply(RMW_UF | RMW_UT | RMW_WF | RMW_WT, r_vectors, force=ft[:half], torque=ft[half:],
-                          eta=eta, a=a, **_apply_opts(kwargs))
-    return np.concatenate([_host(u), _host(w)])
-
-
-def _product(domain, mask, r_vectors, force, torque, eta, a, kwargs, out="u"):
-    u, w = wall_rpy.apply(mask, r_vectors, force=force, torque=torque, eta=eta, a=a, domain=domain,
-                          **_apply_opts(kwargs))
-    return _host(u if out == "u" else w)
+    return _product("single_wall", RMW_UF | RMW_UT | RMW_WF | RMW_WT, r_vectors, ft[:half], ft[half:], eta, a, kwargs)
 
 
 def no_wall_mobility_trans_times_force_hip(r_vectors, force, eta, a, *args, **kwargs):
@@ -126,12 +126,12 @@ def no_wall_mobility_trans_times_torque_hip(r_vectors, torque, eta, a, *args, **
 
 def no_wall_mobility_rot_times_force_hip(r_vectors, force, eta, a, *args, **kwargs):
     """Unbounded w = M_WF f; drop-in for mobility.py:1258-1270."""
-    return _product("no_wall", RMW_WF, r_vectors, force, None, eta, a, kwargs, out="w")
+    return _product("no_wall", RMW_WF, r_vectors, force, None, eta, a, kwargs)
 
 
 def no_wall_mobility_rot_times_torque_hip(r_vectors, torque, eta, a, *args, **kwargs):
     """Unbounded w = M_WT t; drop-in for mobility.py:1301-1313."""
-    return _product("no_wall", RMW_WT, r_vectors, None, torque, eta, a, kwargs, out="w")
+    return _product("no_wall", RMW_WT, r_vectors, None, torque, eta, a, kwargs)
 
 
 def no_wall_mobility_trans_times_force_torque_hip(r_vectors, force, torque, eta, a, *args, **kwargs):

@@ -172,6 +172,66 @@ def apply(mask: int, r_vectors, force=None, torque=None, eta: float = 1.0, a: fl
     return u, w
 
 
+# Pinned host buffers of apply_host: taken by one call at a time, at most
+# _STAGES kept (list.pop and list.append are atomic; a call has waited for its
+# stream before it gives its buffer back).
+_STAGE_DOUBLES, _STAGES = 1 << 17, 8
+_stages: list = []
+_F64 = np.dtype(np.float64)
+
+
+def apply_host(mask: int, r_vectors, force=None, torque=None, eta: float = 1.0, a: float = 1.0,
+               periodic_length=None, precision="fp32", tuning=None, domain: str = "single_wall"):
+    """apply() for numpy inputs and one right-hand side, the outputs as one
+    new float64 array (velocity, then omega, as the mask gives them): inputs
+    and outputs go through one pinned buffer and the stream is waited for
+    once.  Returns None for what it does not take -- anything but contiguous
+    native float64 arrays of matching sizes that fit the buffer -- and leaves
+    that, errors included, to apply()."""
+    ins = [r_vectors]
+    if mask & (RMW_UF | RMW_WF):
+        ins.append(force)
+    if mask & (RMW_UT | RMW_WT):
+        ins.append(torque)
+    for x in ins:
+        if type(x) is not np.ndarray or x.dtype != _F64 or not x.flags.c_contiguous:
+            return None
+    n3 = ins[0].size
+    nout = n3 * (bool(mask & (RMW_UF | RMW_UT)) + bool(mask & (RMW_WF | RMW_WT)))
+    if n3 == 0 or n3 % 3 or len(ins) * n3 + nout > _STAGE_DOUBLES or any(x.size != n3 for x in ins) or \
+            domain not in DOMAINS:
+        return None
+    lib = _lib.load()
+    device = _device()
+    n, dom = n3 // 3, DOMAINS[domain]
+    prec = _lib.precision_code(precision)
+    if dom == 0:
+        tun = _tuning_for(tuning, mask, precision, 1, float(n) * n, False, _periodic(periodic_length))
+    else:
+        tun = None if tuning is None or isinstance(tuning, str) else tuning
+    tp = _lib.tuning_ptr(tun)
+    nbytes = ctypes.c_size_t()
+    _lib.check(lib.rmw_mobility_host_workspace_size(dom, mask, prec, n, tp, ctypes.byref(nbytes)))
+    ws = workspace(nbytes.value, device)
+    L = _L_array(periodic_length)
+    try:
+        stage = _stages.pop()
+    except IndexError:
+        t = torch.empty(_STAGE_DOUBLES, dtype=torch.float64, pin_memory=True)
+        stage = (t, t.numpy(), t.data_ptr())
+    _, buf, ptr = stage
+    o = 0
+    for x in ins:
+        buf[o:o + n3] = x.reshape(-1)
+        o += n3
+    _lib.check(lib.rmw_mobility_apply_host(dom, mask, prec, ptr, ptr + 8 * o, n, float(eta), float(a), L, tp,
+                                           ws.data_ptr(), ws.numel(), _stream_ptr(device)))
+    out = buf[o:o + nout].copy()
+    if len(_stages) < _STAGES:
+        _stages.append(stage)
+    return out
+
+
 class Product:
     """A prepared product of the blocks of ``mask`` on the positions held by
     ``r`` (a contiguous float64 (N, 3) device tensor, read at every call, so
