@@ -77,4 +77,35 @@ __device__ __forceinline__ double image_count(double d, double L)
   return trunc(d / L + 0.5 * s);
 }
 
+// The same number without the division, iL = 1 / L rounded: d * iL is off by
+// less than 1e-10 up to 1e5 boxes, which the integer part hides unless it is
+// next to an integer; those, larger ones and non-finite ones are divided.
+__device__ __forceinline__ double image_count(double d, double L, double iL)
+{
+  const double v = fma(d, iL, d > 0.0 ? 0.5 : (d < 0.0 ? -0.5 : 0.0));
+  const bool safe = fabs(v - rint(v)) > 1e-9 && fabs(v) < 1e5;
+  return __builtin_expect(safe, 1) ? trunc(v) : image_count(d, L);
+}
+
+// f(dx, dy, dz, central) for the minimum image of d (FP64) and its neighbours
+// in the periodic directions (bits of `periodic`); central: the minimum image.
+template <typename R, typename F>
+__device__ __forceinline__ void each_image(double ddx, double ddy, double ddz, int periodic, const double (&L)[3],
+                                           const double (&iL)[3], F&& f)
+{
+  const int nx = periodic & 1, ny = (periodic >> 1) & 1, nz = (periodic >> 2) & 1;
+  auto shifted = [](double d, int b, double len) { return (R)(d + (b < 0 ? -len : (b > 0 ? len : 0.0))); };
+  if (nx) ddx -= image_count(ddx, L[0], iL[0]) * L[0];
+  if (ny) ddy -= image_count(ddy, L[1], iL[1]) * L[1];
+  if (nz) ddz -= image_count(ddz, L[2], iL[2]) * L[2];
+  for (int bz = -nz; bz <= nz; ++bz) {
+    const R dz = shifted(ddz, bz, L[2]);
+    for (int bx = -nx; bx <= nx; ++bx) {
+      const R dx = shifted(ddx, bx, L[0]);
+      for (int by = -ny; by <= ny; ++by)
+        f(dx, shifted(ddy, by, L[1]), dz, bx == 0 && by == 0 && bz == 0);
+    }
+  }
+}
+
 }  // namespace rmw

@@ -42,7 +42,7 @@ struct RadiiParams {
   double norm;            // 1 / (8 pi eta)
   int bnd;                // kRadiiUnbounded, kRadiiWall or kRadiiFreeSurface
   int periodic;           // bit d set when L_d > 0
-  double L[3];
+  double L[3], iL[3];
   double* partial;        // [chunk][nt][3]
   int64_t n_chunks, chunk_len, total_items;
 };
@@ -66,8 +66,6 @@ __global__ __launch_bounds__(kRBlock) void radii_kernel(RadiiParams p)
   __shared__ double s_x[kRBlock], s_y[kRBlock], s_z[kRBlock];
   __shared__ T s_b[kRBlock], s_ib[kRBlock], s_zr[kRBlock];
   __shared__ T s_f[3][kRBlock];
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = (p.periodic >> d) & 1;
   const int il = threadIdx.x;
 
   for (int64_t item = blockIdx.x; item < p.total_items; item += gridDim.x) {
@@ -123,20 +121,13 @@ __global__ __launch_bounds__(kRBlock) void radii_kernel(RadiiParams p)
           // minimum image of the FP64 difference, then the neighbouring boxes;
           // R_z = z_i + z_j is not shifted, so with L_z > 0 the image term is
           // taken once per z box, as the reference kernels do
-          if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-          if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-          if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-          for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-            for (int by = -pbox[1]; by <= pbox[1]; ++by)
-              for (int bz = -pbox[2]; bz <= pbox[2]; ++bz) {
-                const T dx = (T)(ddx + bx * p.L[0]), dy = (T)(ddy + by * p.L[1]), dz = (T)(ddz + bz * p.L[2]);
-                const CoefRadii<T> c =
-                    coef_radii<T>(dx, dy, dz, Rz, zir, zj, ar, s_b[j], inva, s_ib[j], BND);
-                const Vec3<T> v = apply_radii<T>(dx, dy, dz, Rz, c, s_f[0][j], s_f[1][j], s_f[2][j]);
-                u[0].add(v.x);
-                u[1].add(v.y);
-                u[2].add(v.z);
-              }
+          each_image<T>(ddx, ddy, ddz, p.periodic, p.L, p.iL, [&](T dx, T dy, T dz, bool) {
+            const CoefRadii<T> c = coef_radii<T>(dx, dy, dz, Rz, zir, zj, ar, s_b[j], inva, s_ib[j], BND);
+            const Vec3<T> v = apply_radii<T>(dx, dy, dz, Rz, c, s_f[0][j], s_f[1][j], s_f[2][j]);
+            u[0].add(v.x);
+            u[1].add(v.y);
+            u[2].add(v.z);
+          });
           u[0].flush(); u[1].flush(); u[2].flush();
         }
       }
@@ -525,8 +516,6 @@ __global__ __launch_bounds__(kRBlock) void radii_direct_kernel(RadiiParams p, do
     wall_shift(p.trg[3 * i + 2], a, BND, zi[q], Bi[q]);
     ar[q] = (T)a; inva[q] = (T)(1.0 / a); zir[q] = (T)zi[q];
   }
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = (p.periodic >> d) & 1;
   int taken = 0;
   for (int64_t j = threadIdx.x; j < p.ns; j += kRBlock) {
     const double b = p.rs[j], x = p.src[3 * j], y = p.src[3 * j + 1];
@@ -549,13 +538,7 @@ __global__ __launch_bounds__(kRBlock) void radii_direct_kernel(RadiiParams p, do
         add((T)ddx, (T)ddy, (T)ddz);
       } else {
         // as radii_kernel: R_z is not shifted
-        if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-        if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-        if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-        for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-          for (int by = -pbox[1]; by <= pbox[1]; ++by)
-            for (int bz = -pbox[2]; bz <= pbox[2]; ++bz)
-              add((T)(ddx + bx * p.L[0]), (T)(ddy + by * p.L[1]), (T)(ddz + bz * p.L[2]));
+        each_image<T>(ddx, ddy, ddz, p.periodic, p.L, p.iL, [&](T dx, T dy, T dz, bool) { add(dx, dy, dz); });
       }
     }
     if (p.periodic || (taken & (kSub - 1)) == 0) {
@@ -724,6 +707,7 @@ static void radii_ordered(const RadiiPlan& pl, int prec, int bnd, const double* 
   for (int d = 0; d < 3; ++d) {
     const double Ld = L ? L[d] : 0.0;
     q.L[d] = Ld > 0.0 ? Ld : 0.0;
+    q.iL[d] = Ld > 0.0 ? 1.0 / Ld : 0.0;
     if (Ld > 0.0) q.periodic |= 1 << d;
   }
   q.partial = (double*)workspace;

@@ -35,8 +35,6 @@ __global__ __launch_bounds__(kBlock) void block_kernel(MutParams p)
   __shared__ R s_t[KT][3][2 * kBB];
   __shared__ double s_sum[kBlock / 64][K][OC][kBB];   // the waves' sums of one side
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = PER ? (p.periodic >> d) & 1 : 0;
   constexpr double pz = DOM == kDomInPlane ? 0.0 : 1.0;   // in plane: P v
 
   // out[k][l][c] = the four waves' sums, added in order
@@ -130,27 +128,25 @@ __global__ __launch_bounds__(kBlock) void block_kernel(MutParams p)
           const int jr = lane + st;               // LDS entry of source jr mod 64
           const bool on = !MASKED || (valid && (jr & 63) < cnt && !(diag && st == 32 && lane >= 32));
           const R zj = s_zr[jr];
-          auto apply = [&](R dx, R dy, R dz) {
-            mutual_apply<MASK, K, ACC, R, DOM, MASKED, !PER, JT>(
+          auto apply = [&](auto rot_c, R dx, R dy, R dz, auto& sums) {
+            mutual_apply<MASK, K, ACC, R, DOM, MASKED, decltype(rot_c)::value>(
                 dx, dy, dz, zi, zj, on, fi, ti, [&](int k, int c) { return s_f[BT::NF ? k : 0][c][jr]; },
-                [&](int k, int c) { return s_t[BT::NT ? k : 0][c][jr]; }, u, w, ja);
+                [&](int k, int c) { return s_t[BT::NT ? k : 0][c][jr]; }, u, w, sums);
           };
           if constexpr (!PER) {
-            apply((R)(Xi - s_x[jr]), (R)(Yi - s_y[jr]), (R)(Zi - s_z[jr]));
+            apply(std::true_type{}, (R)(Xi - s_x[jr]), (R)(Yi - s_y[jr]), (R)(Zi - s_z[jr]), ja);
           } else {
+            ImageSum<ACC, R> ji[K][OC];
 #pragma unroll
             for (int k = 0; k < K; ++k)
 #pragma unroll
-              for (int c = 0; c < OC; ++c) ja[k][c] = rol1(ja[k][c]);
-            // minimum image of the FP64 difference, then the neighbouring boxes
-            double ddx = Xi - s_x[jr], ddy = Yi - s_y[jr], ddz = Zi - s_z[jr];
-            if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-            if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-            if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-            for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-              for (int by = -pbox[1]; by <= pbox[1]; ++by)
-                for (int bz = -pbox[2]; bz <= pbox[2]; ++bz)
-                  apply((R)(ddx + bx * p.L[0]), (R)(ddy + by * p.L[1]), (R)(ddz + bz * p.L[2]));
+              for (int c = 0; c < OC; ++c) ji[k][c] = 0;
+            each_image<R>(Xi - s_x[jr], Yi - s_y[jr], Zi - s_z[jr], p.periodic, p.L, p.iL,
+                          [&](R dx, R dy, R dz, bool) { apply(std::false_type{}, dx, dy, dz, ji); });
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+              for (int c = 0; c < OC; ++c) ja[k][c] = rol1(ja[k][c]) + (JT)ji[k][c];
             flush_all<K, ACC>(u, w);
           }
         }

@@ -53,8 +53,6 @@ __global__ __launch_bounds__(kBlock) void direct_kernel(DirectParams p)
     zi[q] = (R)Zi[q];
   }
   Acc<ACC> u[TT][K][3], w[TT][K][3];
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = PER ? (p.periodic >> d) & 1 : 0;
   constexpr double pz = DOM == kDomInPlane ? 0.0 : 1.0;   // in plane: P v
 
   int taken = 0;
@@ -87,16 +85,10 @@ __global__ __launch_bounds__(kBlock) void direct_kernel(DirectParams p)
         pair_eval<MASK, K, ACC, R, DOM>((R)(Xi[q] - X), (R)(Yi[q] - Y), (R)(Zi[q] - Z), zi[q], zj, sf, st, own,
                                         u[q], w[q]);
       } else {
-        // minimum image of the FP64 difference, then the neighbouring boxes
-        double ddx = Xi[q] - X, ddy = Yi[q] - Y, ddz = Zi[q] - Z;
-        if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-        if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-        if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-        for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-          for (int by = -pbox[1]; by <= pbox[1]; ++by)
-            for (int bz = -pbox[2]; bz <= pbox[2]; ++bz)
-              pair_eval<MASK, K, ACC, R, DOM>((R)(ddx + bx * p.L[0]), (R)(ddy + by * p.L[1]), (R)(ddz + bz * p.L[2]),
-                                              zi[q], zj, sf, st, own && bx == 0 && by == 0 && bz == 0, u[q], w[q]);
+        each_image<R>(Xi[q] - X, Yi[q] - Y, Zi[q] - Z, p.periodic, p.L, p.iL,
+                      [&](R dx, R dy, R dz, bool central) {
+                        pair_eval<MASK, K, ACC, R, DOM>(dx, dy, dz, zi[q], zj, sf, st, own && central, u[q], w[q]);
+                      });
       }
     }
     // fold the FP32 sums every kSub sources (every source with the images)

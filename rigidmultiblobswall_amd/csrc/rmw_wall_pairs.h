@@ -137,6 +137,11 @@ struct MutSys {
   int64_t pi0, pj0;     // first target-side / source-side slot
 };
 
+// Source-side sums over one source's images: in the pair's type where the
+// mode sums images so anyway, in FP64 for the FP32 modes that do not.
+template <int ACC, typename R>
+using ImageSum = typename std::conditional<ACC == RMW_PREC_F32_F64ACC || ACC == RMW_PREC_F32_KAHAN, double, R>::type;
+
 struct MutParams {
   const double* r;
   const double* f;          // K right-hand sides rhs_stride apart, or null
@@ -150,7 +155,7 @@ struct MutParams {
   int nsys;
   int64_t n_items, chunk_blocks;   // work item: a run of chunk_blocks 64-source blocks
   int periodic;             // bit d set when L_d > 0 (the PER instantiations)
-  double L[3];              // periodic lengths / a
+  double L[3], iL[3];       // periodic lengths / a and their inverses (0: none)
 };
 
 __device__ __forceinline__ MutSys mut_sys_of_item(const MutParams& p, int64_t item)
@@ -183,6 +188,8 @@ __device__ __forceinline__ void mutual_apply(R dx, R dy, R dz, R zi, R zj, bool 
   auto acc_j = [](JT& a, JT x) {
     if constexpr (ROT) a = rol1(a) + x; else a = a + x;
   };
+  // sums that stay where they are, in the pair's type: they seed the products
+  constexpr bool CJ = !ROT && std::is_same<JT, R>::value;
   // a pair not taken contributes exact zeros (make_geom_on)
   const Geom<R> g = MASKED ? make_geom_on(dx, dy, dz, zi, zj, on) : make_geom(dx, dy, dz, zi, zj);
   CoefUF<R> cuf;
@@ -216,31 +223,33 @@ __device__ __forceinline__ void mutual_apply(R dx, R dy, R dz, R zi, R zj, bool 
         if constexpr (BT::HU) {
           R x = R(0), y = R(0);
           if constexpr (kChain) x = u[k][r].run();
+          if constexpr (CJ) y = ja[k][r];
           if constexpr (UF) {
             x = fma_(Mu.m[r][0], fj[0], fma_(Mu.m[r][1], fj[1], kChain ? fma_(Mu.m[r][2], fj[2], x) : Mu.m[r][2] * fj[2]));
-            y = fma_(Mu.m[0][r], fi[k][0], fma_(Mu.m[1][r], fi[k][1], Mu.m[2][r] * fi[k][2]));
+            y = fma_(Mu.m[0][r], fi[k][0], fma_(Mu.m[1][r], fi[k][1], CJ ? fma_(Mu.m[2][r], fi[k][2], y) : Mu.m[2][r] * fi[k][2]));
           }
           if constexpr (UT)
             x = fma_(Mc.m[r][0], tj[0], fma_(Mc.m[r][1], tj[1], r == 2 ? x : fma_(Mc.m[r][2], tj[2], x)));
           if constexpr (WF)
             y = fma_(Md.m[0][r], ti[k][0], fma_(Md.m[1][r], ti[k][1], r == 2 ? y : fma_(Md.m[2][r], ti[k][2], y)));
           if constexpr (kChain) u[k][r].run() = x; else u[k][r].add(x);
-          acc_j(ja[k][r], (JT)y);
+          if constexpr (CJ) ja[k][r] = y; else acc_j(ja[k][r], (JT)y);
         }
         if constexpr (BT::HW) {
           constexpr int o = BT::HU ? 3 : 0;
           R x = R(0), y = R(0);
           if constexpr (kChain) x = w[k][r].run();
+          if constexpr (CJ) y = ja[k][o + r];
           if constexpr (WT) {
             x = fma_(Mw.m[r][0], tj[0], fma_(Mw.m[r][1], tj[1], kChain ? fma_(Mw.m[r][2], tj[2], x) : Mw.m[r][2] * tj[2]));
-            y = fma_(Mw.m[0][r], ti[k][0], fma_(Mw.m[1][r], ti[k][1], Mw.m[2][r] * ti[k][2]));
+            y = fma_(Mw.m[0][r], ti[k][0], fma_(Mw.m[1][r], ti[k][1], CJ ? fma_(Mw.m[2][r], ti[k][2], y) : Mw.m[2][r] * ti[k][2]));
           }
           if constexpr (WF)
             x = fma_(Md.m[r][0], fj[0], fma_(Md.m[r][1], fj[1], r == 2 ? x : fma_(Md.m[r][2], fj[2], x)));
           if constexpr (UT)
             y = fma_(Mc.m[0][r], fi[k][0], fma_(Mc.m[1][r], fi[k][1], r == 2 ? y : fma_(Mc.m[2][r], fi[k][2], y)));
           if constexpr (kChain) w[k][r].run() = x; else w[k][r].add(x);
-          acc_j(ja[k][o + r], (JT)y);
+          if constexpr (CJ) ja[k][o + r] = y; else acc_j(ja[k][o + r], (JT)y);
         }
       }
     }
@@ -255,22 +264,34 @@ __device__ __forceinline__ void mutual_apply(R dx, R dy, R dz, R zi, R zj, bool 
       Vec3<R> ui{}, wi{}, uj{}, wj{};
       if constexpr (C && BT::HU) ui = Vec3<R>{u[k][0].run(), u[k][1].run(), u[k][2].run()};
       if constexpr (C && BT::HW) wi = Vec3<R>{w[k][0].run(), w[k][1].run(), w[k][2].run()};
+      if constexpr (CJ && BT::HU) uj = Vec3<R>{ja[k][0], ja[k][1], ja[k][2]};
+      if constexpr (CJ && BT::HW) {
+        constexpr int o = BT::HU ? 3 : 0;
+        wj = Vec3<R>{ja[k][o], ja[k][o + 1], ja[k][o + 2]};
+      }
       if constexpr (UF) {
         ui = apply_uf<C>(g, cuf, sf(k, 0), sf(k, 1), sf(k, 2), ui);
-        uj = apply_uf_t(g, cuf, fi[k][0], fi[k][1], fi[k][2]);
+        uj = apply_uf_t<CJ>(g, cuf, fi[k][0], fi[k][1], fi[k][2], uj);
       }
       if constexpr (UT) {
         ui = apply_ut<C || UF>(g, cut, st(k, 0), st(k, 1), st(k, 2), ui);
-        uj = apply_wf_t<UF>(g, cwf, ti[k][0], ti[k][1], ti[k][2], uj);
+        uj = apply_wf_t<CJ || UF>(g, cwf, ti[k][0], ti[k][1], ti[k][2], uj);
       }
       if constexpr (WF) {
         wi = apply_wf<C>(g, cwf, sf(k, 0), sf(k, 1), sf(k, 2), wi);
-        wj = apply_ut_t(g, cut, fi[k][0], fi[k][1], fi[k][2]);
+        wj = apply_ut_t<CJ>(g, cut, fi[k][0], fi[k][1], fi[k][2], wj);
       }
       if constexpr (WT) {
         wi = apply_wt<C || WF>(g, cwt, st(k, 0), st(k, 1), st(k, 2), wi);
-        wj = apply_wt_t<WF>(g, cwt, ti[k][0], ti[k][1], ti[k][2], wj);
+        wj = apply_wt_t<CJ || WF>(g, cwt, ti[k][0], ti[k][1], ti[k][2], wj);
       }
+      auto put_j = [&](JT* a, const Vec3<R>& v) {
+        if constexpr (CJ) {
+          a[0] = v.x; a[1] = v.y; a[2] = v.z;
+        } else {
+          acc_j(a[0], (JT)v.x); acc_j(a[1], (JT)v.y); acc_j(a[2], (JT)v.z);
+        }
+      };
       auto put = [](Acc<ACC> (&s)[3], const Vec3<R>& v) {
         if constexpr (C) {
           s[0].run() = v.x; s[1].run() = v.y; s[2].run() = v.z;
@@ -280,16 +301,12 @@ __device__ __forceinline__ void mutual_apply(R dx, R dy, R dz, R zi, R zj, bool 
       };
       if constexpr (BT::HU) {
         put(u[k], ui);
-        acc_j(ja[k][0], (JT)uj.x);
-        acc_j(ja[k][1], (JT)uj.y);
-        acc_j(ja[k][2], (JT)uj.z);
+        put_j(&ja[k][0], uj);
       }
       if constexpr (BT::HW) {
         constexpr int o = BT::HU ? 3 : 0;
         put(w[k], wi);
-        acc_j(ja[k][o], (JT)wj.x);
-        acc_j(ja[k][o + 1], (JT)wj.y);
-        acc_j(ja[k][o + 2], (JT)wj.z);
+        put_j(&ja[k][o], wj);
       }
     }
   }
@@ -387,7 +404,7 @@ struct DirectParams {
   DirectSys single;
   int nsys;
   int periodic;             // bit d set when L_d > 0
-  double L[3];              // periodic lengths / a
+  double L[3], iL[3];       // periodic lengths / a and their inverses (0: none)
 };
 
 // Targets per workgroup of the direct kernel for these blocks and

@@ -90,7 +90,7 @@ struct PairParams {
   int64_t ntot;
   int64_t total_items;
   int periodic;           // bit d set when L_d > 0
-  double L[3];            // periodic lengths / a
+  double L[3], iL[3];     // periodic lengths / a and their inverses (0: none)
   int domain;             // kDomWall, kDomNoWall, kDomInPlane, kDomFreeSurface
 };
 
@@ -195,8 +195,6 @@ __global__ __launch_bounds__(kBlock, (pair_min_waves<MASK, K>())) void pair_kern
   __shared__ SrcF32 s_pos[kBlock];
   __shared__ float4 s_f[BT::NF ? K * kBlock : 1];
   __shared__ float4 s_t[BT::NT ? K * kBlock : 1];
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = (p.periodic >> d) & 1;
 
   for (int64_t item = blockIdx.x; item < p.total_items; item += gridDim.x) {
     const SysInfo S = find_sys_item(p, item);
@@ -257,21 +255,11 @@ __global__ __launch_bounds__(kBlock, (pair_min_waves<MASK, K>())) void pair_kern
       } else {
         for (int j = 0; j < cnt; ++j) {
           const SrcF32 sp = s_pos[j];
-          // minimum image of the FP64 difference, then every box shift in FP64
-          double ddx = Xi - sp.x, ddy = Yi - sp.y, ddz = Zi - sp.z;
-          if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-          if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-          if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-          for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-            for (int by = -pbox[1]; by <= pbox[1]; ++by)
-              for (int bz = -pbox[2]; bz <= pbox[2]; ++bz) {
-                const float dx = (float)(ddx + bx * p.L[0]);
-                const float dy = (float)(ddy + by * p.L[1]);
-                const float dz = (float)(ddz + bz * p.L[2]);
-                const bool central = (bx == 0) && (by == 0) && (bz == 0);
-                pair_eval<MASK, K, ACC, float, DOM>(dx, dy, dz, zi, sp.zf, lds(s_f, j), lds(s_t, j),
-                                                    diag && central && (j == self_j), u, w);
-              }
+          each_image<float>(Xi - sp.x, Yi - sp.y, Zi - sp.z, p.periodic, p.L, p.iL,
+                            [&](float dx, float dy, float dz, bool central) {
+                              pair_eval<MASK, K, ACC, float, DOM>(dx, dy, dz, zi, sp.zf, lds(s_f, j), lds(s_t, j),
+                                                                  diag && central && (j == self_j), u, w);
+                            });
           flush_all<K, ACC>(u, w);
         }
       }
@@ -287,8 +275,6 @@ __global__ __launch_bounds__(kBlock) void pair_kernel_f64(PairParams p)
   __shared__ double4 s_pos[kBlock];
   __shared__ double4 s_f[BT::NF ? K * kBlock : 1];
   __shared__ double4 s_t[BT::NT ? K * kBlock : 1];
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = (p.periodic >> d) & 1;
 
   for (int64_t item = blockIdx.x; item < p.total_items; item += gridDim.x) {
     const SysInfo S = find_sys_item(p, item);
@@ -324,17 +310,10 @@ __global__ __launch_bounds__(kBlock) void pair_kernel_f64(PairParams p)
           pair_eval<MASK, K, RMW_PREC_F64, double, DOM>(rx, ry, rz, Zi, pj.z, lds(s_f, j), lds(s_t, j),
                                                         diag && j == self_j, u, w);
         } else {
-          if (pbox[0]) rx -= image_count(rx, p.L[0]) * p.L[0];
-          if (pbox[1]) ry -= image_count(ry, p.L[1]) * p.L[1];
-          if (pbox[2]) rz -= image_count(rz, p.L[2]) * p.L[2];
-          for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-            for (int by = -pbox[1]; by <= pbox[1]; ++by)
-              for (int bz = -pbox[2]; bz <= pbox[2]; ++bz) {
-                const bool central = (bx == 0) && (by == 0) && (bz == 0);
-                pair_eval<MASK, K, RMW_PREC_F64, double, DOM>(rx + bx * p.L[0], ry + by * p.L[1],
-                                                              rz + bz * p.L[2], Zi, pj.z, lds(s_f, j),
-                                                              lds(s_t, j), diag && central && (j == self_j), u, w);
-              }
+          each_image<double>(rx, ry, rz, p.periodic, p.L, p.iL, [&](double dx, double dy, double dz, bool central) {
+            pair_eval<MASK, K, RMW_PREC_F64, double, DOM>(dx, dy, dz, Zi, pj.z, lds(s_f, j), lds(s_t, j),
+                                                          diag && central && (j == self_j), u, w);
+          });
         }
       }
     }
@@ -377,7 +356,7 @@ __global__ __launch_bounds__(kBlock) void mutual_kernel(MutParams p)
   using BT = BlockTraits<MASK>;
   constexpr bool UF = (MASK & kUF) != 0, UT = (MASK & kUT) != 0, WF = (MASK & kWF) != 0, WT = (MASK & kWT) != 0;
   constexpr int OC = BT::OC;
-  constexpr bool kFoldJ = ACC == RMW_PREC_F32_BLOCKED;
+  constexpr bool kFoldJ = ACC == RMW_PREC_F32_BLOCKED && !PER;
   // several right-hand sides: form each pair's blocks once as 3x3 matrices
   constexpr bool kMat = K >= 2;
   using JT = typename std::conditional<kFoldJ, float, double>::type;
@@ -396,8 +375,6 @@ __global__ __launch_bounds__(kBlock) void mutual_kernel(MutParams p)
   const int il = threadIdx.x;
   // fold the FP32 sums every kSub sources (every source with the images)
   constexpr int kFold = PER ? 0 : kSub - 1;
-  int pbox[3];
-  for (int d = 0; d < 3; ++d) pbox[d] = PER ? (p.periodic >> d) & 1 : 0;
 
   for (int64_t item = blockIdx.x; item < p.n_items; item += gridDim.x) {
     const MutSys Sy = mut_sys_of_item(p, item);
@@ -529,12 +506,13 @@ __global__ __launch_bounds__(kBlock) void mutual_kernel(MutParams p)
           // one image d = (dx, dy, dz) of the pair, applied on both sides; the
           // source-side sums move one lane per step (fused into the add; with
           // images, once per step before them)
-          auto pair_apply = [&](R dx, R dy, R dz) {
-            mutual_apply<MASK, K, ACC, R, DOM, MASKED, !PER, JT>(
+          auto image = [&](auto rot_c, R dx, R dy, R dz, auto& sums) {
+            mutual_apply<MASK, K, ACC, R, DOM, MASKED, decltype(rot_c)::value>(
                 dx, dy, dz, zi, zj, on, fi, ti,
                 [&](int k, int c) { return kEarly ? fje[kEarly ? k : 0][c] : s_f[k][c][jr]; },
-                [&](int k, int c) { return kEarly ? tje[kEarly ? k : 0][c] : s_t[k][c][jr]; }, u, w, ja);
+                [&](int k, int c) { return kEarly ? tje[kEarly ? k : 0][c] : s_t[k][c][jr]; }, u, w, sums);
           };
+          auto pair_apply = [&](R dx, R dy, R dz) { image(std::true_type{}, dx, dy, dz, ja); };
           if constexpr (kEarly) {
             if constexpr (sizeof(R) == 4)
               pair_apply((R)(Xi - xje), (R)(Yi - yje), (R)(Zi - zje));
@@ -546,19 +524,17 @@ __global__ __launch_bounds__(kBlock) void mutual_kernel(MutParams p)
             else
               pair_apply(Xi - s_x[jr], Yi - s_y[jr], Zi - s_z[jr]);
           } else {
+            ImageSum<ACC, R> ji[K][OC];
 #pragma unroll
             for (int k = 0; k < K; ++k)
 #pragma unroll
-              for (int c = 0; c < OC; ++c) ja[k][c] = rol1(ja[k][c]);
-            // minimum image of the FP64 difference, then the neighbouring boxes
-            double ddx = Xi - s_x[jr], ddy = Yi - s_y[jr], ddz = Zi - s_z[jr];
-            if (pbox[0]) ddx -= image_count(ddx, p.L[0]) * p.L[0];
-            if (pbox[1]) ddy -= image_count(ddy, p.L[1]) * p.L[1];
-            if (pbox[2]) ddz -= image_count(ddz, p.L[2]) * p.L[2];
-            for (int bx = -pbox[0]; bx <= pbox[0]; ++bx)
-              for (int by = -pbox[1]; by <= pbox[1]; ++by)
-                for (int bz = -pbox[2]; bz <= pbox[2]; ++bz)
-                  pair_apply((R)(ddx + bx * p.L[0]), (R)(ddy + by * p.L[1]), (R)(ddz + bz * p.L[2]));
+              for (int c = 0; c < OC; ++c) ji[k][c] = 0;
+            each_image<R>(Xi - s_x[jr], Yi - s_y[jr], Zi - s_z[jr], p.periodic, p.L, p.iL,
+                          [&](R dx, R dy, R dz, bool) { image(std::false_type{}, dx, dy, dz, ji); });
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+              for (int c = 0; c < OC; ++c) ja[k][c] = rol1(ja[k][c]) + (JT)ji[k][c];
           }
           if ((st & kFold) == kFold) {
             flush_all<K, ACC>(u, w);
@@ -1489,7 +1465,7 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     q.n_items = pl.mut_items;
     q.chunk_blocks = pl.chunk_blocks;
     q.periodic = periodic;
-    for (int d = 0; d < 3; ++d) q.L[d] = Lp[d];
+    for (int d = 0; d < 3; ++d) { q.L[d] = Lp[d]; q.iL[d] = Lp[d] > 0.0 ? 1.0 / Lp[d] : 0.0; }
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st);
@@ -1574,7 +1550,7 @@ static void run_direct(const Plan& pl, const double* r, const double* f, const d
     q.single = table[0];
     q.nsys = (int)table.size();
     q.periodic = periodic;
-    for (int d = 0; d < 3; ++d) q.L[d] = Lp[d];
+    for (int d = 0; d < 3; ++d) { q.L[d] = Lp[d]; q.iL[d] = Lp[d] > 0.0 ? 1.0 / Lp[d] : 0.0; }
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st);
@@ -1715,7 +1691,7 @@ static void run_plan(const Plan& pl, const double* r, const double* f, const dou
     q.ntot = pl.ntot;
     q.total_items = pl.total_items;
     q.periodic = periodic;
-    for (int d = 0; d < 3; ++d) q.L[d] = Lp[d];
+    for (int d = 0; d < 3; ++d) { q.L[d] = Lp[d]; q.iL[d] = Lp[d] > 0.0 ? 1.0 / Lp[d] : 0.0; }
     q.domain = pl.domain;
     // The partial layout was planned for kmax RHS; a smaller trailing group
     // reuses it with its own K (items only touch their own slots).

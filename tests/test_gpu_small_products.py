@@ -123,3 +123,22 @@ def test_coincident_blobs_stay_non_finite(gpu, n, prec):
     u, _ = wall_rpy.apply(RMW_UF, r, f, eta=ETA, a=A, precision=prec, tuning="heuristic")
     bad = ~torch.isfinite(u).all(dim=1)
     assert bool(bad[3]) and bool(bad[n - 1]) and int(bad.sum()) == 2
+
+
+@pytest.mark.parametrize("n", [90, 2433])
+def test_minimum_images_at_ties(gpu, n):
+    """Blobs on a lattice of half the box, many boxes apart: d / L + 1/2 is a
+    whole number, where the count of boxes must be that of the division."""
+    rng = np.random.default_rng(n)
+    L = np.array([16.0, 24.0, 0.0])
+    boxes = rng.integers(-3, 4, (n, 2)) * np.where(rng.random((n, 1)) < 0.2, 1e5, 1.0)
+    r = np.column_stack([rng.integers(0, 2, (n, 2)) * (L[:2] / 2) + boxes * L[:2], 0.75 * np.arange(1, n + 1)])
+    f, t = rng.standard_normal((1, n, 3)), rng.standard_normal((1, n, 3))
+    rows = (0, 90)
+    want = [O.block_apply(blk, r, v[0], ETA, 0.5, L, rows=rows).reshape(n, 3)[:90] for blk, v in ((O.UF, f), (O.UT, t))]
+    for prec in ("fp64", "fp32_blocked"):
+        for tuning in ("heuristic", ORDERED, _lib.Tuning(256, 0, 0, 1, 0)):
+            u, _ = wall_rpy.apply(RMW_UF | RMW_UT, r, force=f, torque=t, eta=ETA, a=0.5, precision=prec,
+                                  periodic_length=L, tuning=tuning)
+            ref = torch.as_tensor(want[0] + want[1]).to(u)
+            assert rel(u.reshape(n, 3)[:90], ref) <= TOL[prec], (prec, tuning)
