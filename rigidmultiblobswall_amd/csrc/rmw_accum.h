@@ -108,4 +108,27 @@ __device__ __forceinline__ void each_image(double ddx, double ddy, double ddz, i
   }
 }
 
+// Sum over the 64 lanes, in every lane: within the rows of 16 by DPP moves
+// (a shuffle through LDS takes some 60 cycles per step and half of a double).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v)
+{
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double v)   // over rows of 16 lanes
+{
+  v = dpp_add<0xB1>(v);    // quad_perm 1 0 3 2
+  v = dpp_add<0x4E>(v);    // quad_perm 2 3 0 1
+  v = dpp_add<0x141>(v);   // row_half_mirror
+  return dpp_add<0x140>(v);   // row_mirror
+}
+__device__ __forceinline__ double wave_sum(double v)
+{
+  v = row_sum(v);
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
 }  // namespace rmw

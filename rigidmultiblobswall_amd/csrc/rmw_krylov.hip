@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "rmw_accum.h"
 #include "rmw_internal.h"
 
 namespace rmw {
@@ -162,7 +163,9 @@ __global__ void axpby_kernel(double alpha, const double* __restrict__ x, double 
 // no launch in between turns partial sums into coefficients.  The chain of
 // small launches, not the vectors, was the time of the step: ten launches
 // took 35 us at n = 15000 with 11 vectors (13 MB read, 2.7 us at the rate of
-// a copy), these take 17.
+// a copy), these 17, and 16 with the first vectors loaded before anything is
+// waited for and the sums taken by DPP moves (13200 elements, 8 vectors on
+// average: 19.6 before, 16).
 // ---------------------------------------------------------------------------
 struct ArnoldiParams {
   double* V;            // basis r at V + r * v_rhs, vectors ldv apart
@@ -177,39 +180,59 @@ struct ArnoldiParams {
   int m;                // vectors in the basis
 };
 
-// coef[j] = sum_g part[j * G + g], j < m: one wave per j at a time.
+// coef[j] = sum_g part[j * G + g], j < m: sixteen threads per j.
 __device__ __forceinline__ void block_coefs(const double* __restrict__ part, int G, int m, double* coef)
 {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int j = wv; j < m; j += kKBlock / 64) {
+  const int sub = threadIdx.x & 15;
+  for (int j = threadIdx.x >> 4; j < m; j += kKBlock / 16) {
     double s = 0.0;
-    for (int g = lane; g < G; g += 64) s += part[(int64_t)j * G + g];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if (lane == 0) coef[j] = s;
+#pragma unroll 4
+    for (int g = sub; g < G; g += 16) s += part[(int64_t)j * G + g];
+    s = row_sum(s);
+    if (sub == 0) coef[j] = s;
   }
   __syncthreads();
 }
 
-// part[j * G + block] = V_j . w over this block's slice, w in registers.
+// part[j * G + block] = V_j . w over this block's slice, w in registers; the
+// first held_vectors(E) vectors' slices are in registers too (v).
+constexpr int held_vectors(int E) { return 16 / E; }   // 32 registers' worth
 template <int E>
 __device__ __forceinline__ void block_dots(const double* __restrict__ V, int64_t ldv, int m, const double (&wr)[E],
-                                           int64_t base, int64_t n, double* __restrict__ part, int G)
+                                           const double (&v)[held_vectors(E)][E], int64_t base, int64_t n,
+                                           double* __restrict__ part, int G)
 {
+  constexpr int kHeld = held_vectors(E);
   __shared__ double red[kDotGroup][kKBlock / 64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  auto put = [&](int jj, double acc) {
+    acc = wave_sum(acc);
+    if (lane == 0) red[jj][wv] = acc;
+  };
   for (int j0 = 0; j0 < m; j0 += kDotGroup) {
     const int jn = m - j0 < kDotGroup ? m - j0 : kDotGroup;
+    int jj = 0;
+    if (j0 == 0) {
+#pragma unroll
+      for (int q = 0; q < kHeld; ++q)
+        if (q < jn) {
+          double acc = 0.0;
+#pragma unroll
+          for (int e = 0; e < E; ++e) acc = fma(v[q][e], wr[e], acc);
+          put(q, acc);
+        }
+      jj = kHeld;
+    }
 #pragma unroll 4
-    for (int jj = 0; jj < jn; ++jj) {
-      const double* v = V + (int64_t)(j0 + jj) * ldv;
+    for (; jj < jn; ++jj) {
+      const double* vj = V + (int64_t)(j0 + jj) * ldv;
       double acc = 0.0;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const int64_t i = base + (int64_t)e * kKBlock;
-        if (i < n) acc = fma(v[i], wr[e], acc);
+        if (i < n) acc = fma(vj[i], wr[e], acc);
       }
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-      if (lane == 0) red[jj][wv] = acc;
+      put(jj, acc);
     }
     __syncthreads();
     if ((int)threadIdx.x < jn) {
@@ -243,11 +266,25 @@ __global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
     const int64_t i = base + (int64_t)e * kKBlock;
     wr[e] = i < p.n ? w[i] : 0.0;
   }
+  // the slices of the first vectors, loaded before anything has to be waited for
+  constexpr int kHeld = held_vectors(E);
+  double held[PASS < 3 ? kHeld : 1][E];
+  if constexpr (PASS < 3) {
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int64_t i = base + (int64_t)e * kKBlock;
+        held[j][e] = j < p.m && i < p.n ? V[(int64_t)j * p.ldv + i] : 0.0;
+      }
+  }
   if constexpr (PASS == 0) {
-    block_dots<E>(V, p.ldv, p.m, wr, base, p.n, part1, G);
+    block_dots<E>(V, p.ldv, p.m, wr, held, base, p.n, part1, G);
   } else if constexpr (PASS == 3) {
-    block_coefs(part3, G, 1, coef);
-    const double norm = sqrt(coef[0]);
+    // (every wave by itself, one load each up to 64 blocks)
+    double sq = 0.0;
+    for (int g = threadIdx.x & 63; g < G; g += 64) sq += part3[g];
+    const double norm = sqrt(wave_sum(sq));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       h[p.m] = norm;
       if (p.h_host) p.h_host[p.m] = norm;
@@ -267,8 +304,14 @@ __global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
         h[j] = v;
         if (PASS == 2 && p.h_host) p.h_host[j] = v;
       }
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+      if (j < p.m) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) wr[e] -= coef[j] * held[j][e];
+      }
 #pragma unroll 4
-    for (int j = 0; j < p.m; ++j) {
+    for (int j = kHeld; j < p.m; ++j) {
       const double* v = V + (int64_t)j * p.ldv;
 #pragma unroll
       for (int e = 0; e < E; ++e) {
@@ -282,13 +325,13 @@ __global__ __launch_bounds__(kKBlock) void arnoldi_pass(ArnoldiParams p)
       if (i < p.n) w[i] = wr[e];
     }
     if constexpr (PASS == 1) {
-      block_dots<E>(V, p.ldv, p.m, wr, base, p.n, part2, G);
+      block_dots<E>(V, p.ldv, p.m, wr, held, base, p.n, part2, G);
     } else {
       __shared__ double red[kKBlock / 64];
       double acc = 0.0;
 #pragma unroll
       for (int e = 0; e < E; ++e) acc = fma(wr[e], wr[e], acc);
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+      acc = wave_sum(acc);
       if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
       __syncthreads();
       if (threadIdx.x == 0) part3[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];

@@ -28,6 +28,7 @@
 #include <cstring>
 #include <vector>
 
+#include "rmw_accum.h"
 #include "rmw_internal.h"
 #include "rmw_pair_terms.h"
 
@@ -101,15 +102,17 @@ __global__ __launch_bounds__(kRigidBlock) void rigid_post_kernel(const double* _
     acc[4] += rz * lx - rx * lz;
     acc[5] += rx * ly - ry * lx;
   }
-  __shared__ double red[6][kRigidBlock];
-  for (int c = 0; c < 6; ++c) red[c][threadIdx.x] = acc[c];
-  __syncthreads();
-  for (int s = kRigidBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s)
-      for (int c = 0; c < 6; ++c) red[c][threadIdx.x] += red[c][threadIdx.x + s];
-    __syncthreads();
+  __shared__ double red[6][kRigidBlock / 64];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    acc[c] = wave_sum(acc[c]);
+    if ((threadIdx.x & 63) == 0) red[c][threadIdx.x >> 6] = acc[c];
   }
-  if (threadIdx.x < 6) y[3 * nblobs + 6 * (int64_t)b + threadIdx.x] = -red[threadIdx.x][0];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const double* q = red[threadIdx.x];
+    y[3 * nblobs + 6 * (int64_t)b + threadIdx.x] = -(((q[0] + q[1]) + q[2]) + q[3]);
+  }
 }
 
 // Body force-torque from blob forces: F_b = sum f_i, T_b = sum r_i x f_i
@@ -759,6 +762,22 @@ __global__ __launch_bounds__(kRigidBlock) void pc_apply_kernel(const int64_t* __
   __shared__ double red[6][kRigidBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const double* MK = minvk + 3 * i0 * 6;
+  // this wave's four rows of M^-1 (rows beyond n repeat the last and are
+  // dropped): the first kAhead columns of each lane before anything else
+  constexpr int kAhead = 2;
+  const double* M = minv + moff[b];
+  const int r0 = row0 + 4 * wv;
+  const double* Mr[4];
+  double ahead[4][kAhead];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    Mr[q] = M + (int64_t)(r0 + q < n ? r0 + q : n - 1) * n;
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int j = lane + 64 * k;
+      ahead[q][k] = j < n ? Mr[q][j] : 0.0;
+    }
+  }
   double acc[6] = {0, 0, 0, 0, 0, 0};
   for (int i = tid; i < n; i += kRigidBlock) {
     const double v = x[3 * i0 + i];
@@ -768,7 +787,7 @@ __global__ __launch_bounds__(kRigidBlock) void pc_apply_kernel(const int64_t* __
   }
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
-    for (int o = 32; o > 0; o >>= 1) acc[c] += __shfl_down(acc[c], o, 64);
+    acc[c] = wave_sum(acc[c]);
     if (lane == 0) red[c][wv] = acc[c];
   }
   __syncthreads();
@@ -790,22 +809,22 @@ __global__ __launch_bounds__(kRigidBlock) void pc_apply_kernel(const int64_t* __
     for (int c = 1; c < 6; ++c) v = tid == c ? Y[c] : v;
     y[3 * nblobs + 6 * (int64_t)b + tid] = v;
   }
-  // rows r0 .. r0 + 3 of M^-1 s (rows beyond n repeat the last and are dropped)
-  const double* M = minv + moff[b];
-  const int r0 = row0 + 4 * wv;
   if (r0 >= n) return;
   double a[4] = {0, 0, 0, 0};
-  const double* Mr[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) Mr[q] = M + (int64_t)(r0 + q < n ? r0 + q : n - 1) * n;
-  for (int j = lane; j < n; j += 64) {
+  for (int k = 0; k < kAhead; ++k) {
+    const int j = lane + 64 * k;
+    const double v = j < n ? s[j] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = fma(ahead[q][k], v, a[q]);
+  }
+  for (int j = lane + 64 * kAhead; j < n; j += 64) {
     const double v = s[j];
 #pragma unroll
     for (int q = 0; q < 4; ++q) a[q] = fma(Mr[q][j], v, a[q]);
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    for (int o = 32; o > 0; o >>= 1) a[q] += __shfl_xor(a[q], o, 64);
+  for (int q = 0; q < 4; ++q) a[q] = wave_sum(a[q]);
   if (lane < 4 && r0 + lane < n) {
     const int i = r0 + lane;
     double v = lane == 0 ? a[0] : (lane == 1 ? a[1] : (lane == 2 ? a[2] : a[3]));
