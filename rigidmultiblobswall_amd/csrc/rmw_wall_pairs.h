@@ -135,6 +135,7 @@ struct MutSys {
   int64_t b0, n, n_t;   // first blob, blobs, tiles of kBlock
   int64_t item0;        // first work item
   int64_t pi0, pj0;     // first target-side / source-side slot
+  int64_t t0;           // tiles of the systems before
 };
 
 // Source-side sums over one source's images: in the pair's type where the

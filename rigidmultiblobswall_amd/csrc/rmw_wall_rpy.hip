@@ -687,7 +687,7 @@ struct MutReduceParams {
   int nsys;
   int mask;
   int K;
-  int64_t ntot, chunk_blocks;
+  int64_t chunk_blocks;
   int64_t rhs_stride;
   double a, inva, c1, c2;
   int domain;
@@ -697,9 +697,12 @@ struct MutReduceParams {
 
 // Output o (component c of blob gi, RHS k) sums the target-side slots of the
 // work items of its tile and the source-side slots (X, T), T <= X.  Eight
-// groups of 32 threads share a block's 32 outputs: group g takes slots
+// groups of 32 threads share a workgroup's 32 outputs: group g takes slots
 // g, g + 8, ... of both lists (consecutive threads read consecutive
 // outputs of one slot), then group 0 adds the eight partial sums in order.
+// The 32 outputs lie in one tile and right-hand side, which the workgroup's
+// number gives: the search for the system and the divisions are scalar work
+// (64 systems of 128 to 4096 blobs: 106 us with both per thread, in 64 bits, 76).
 constexpr int kRedGroups = 8, kRedOut = 256 / kRedGroups;
 
 // PER: pseudo-periodic calls, which add the self pair's outer images; the
@@ -716,36 +719,33 @@ __global__ __launch_bounds__(256) void mutual_reduce_kernel(MutReduceParams p)
   const bool HW = (p.mask & (kWF | kWT)) != 0;
   const int OC = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
   const int g = threadIdx.x / kRedOut, ol = threadIdx.x - g * kRedOut;
-  const int64_t tid = (int64_t)blockIdx.x * kRedOut + ol;
-  const int64_t per_k = p.ntot * OC;
-  const bool valid = tid < per_k * p.K;
-  double sum = 0.0;
-  int k = 0;
-  int64_t gi = 0;
-  int c = 0;
-  if (valid) {
-    k = (int)(tid / per_k);
-    const int64_t rem = tid - (int64_t)k * per_k;
-    gi = rem / OC;
-    c = (int)(rem - gi * OC);
-    MutSys Sy = p.single;
-    if (p.table) {
-      int lo = 0, hi = p.nsys - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (p.table[mid].b0 <= gi) lo = mid; else hi = mid - 1;
-      }
-      Sy = p.table[lo];
+  constexpr int R3 = BS * 3 / kRedOut, R6 = BS * 6 / kRedOut;   // workgroups of one tile
+  const int k = blockIdx.y;
+  const int Xg = OC == 3 ? blockIdx.x / R3 : blockIdx.x / R6;   // the tile, among all systems'
+  const int run = (int)blockIdx.x - Xg * (OC == 3 ? R3 : R6);
+  MutSys Sy = p.single;
+  if (p.table) {
+    int lo = 0, hi = p.nsys - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (p.table[mid].t0 <= Xg) lo = mid; else hi = mid - 1;
     }
-    const int64_t il = gi - Sy.b0;
-    const int64_t X = il / BS, l = il - X * BS;
+    Sy = p.table[lo];
+  }
+  const int64_t X = Xg - Sy.t0;
+  const int e = run * kRedOut + ol;   // output within the tile
+  const int l = OC == 3 ? e / 3 : e / 6, c = e - l * OC;
+  const bool valid = X * BS + l < Sy.n;
+  const int64_t gi = Sy.b0 + X * BS + l;
+  double sum = 0.0;
+  if (valid) {
     auto before = [&](int64_t x) {
       return BS == kBlock ? items_before_blocks(x, Sy.n_t, p.chunk_blocks) : items_before(x, Sy.n_t, p.chunk_blocks);
     };
     const int64_t it0 = before(X), it1 = before(X + 1);
     const int64_t step = (int64_t)p.K * BS * OC;
-    const double* Pi = p.part_i + (((Sy.pi0 + it0) * p.K + k) * BS + l) * OC + c;
-    const double* Pj = p.part_j + (((Sy.pj0 + tri_index(X, 0)) * p.K + k) * BS + l) * OC + c;
+    const double* Pi = p.part_i + ((Sy.pi0 + it0) * p.K + k) * (BS * OC) + e;
+    const double* Pj = p.part_j + ((Sy.pj0 + tri_index(X, 0)) * p.K + k) * (BS * OC) + e;
     // four loads in flight per thread (the loop is latency-bound: one
     // dependent load per slot took ~2x longer at 32768 blobs)
     auto strided_sum = [&](const double* P, int64_t cnt) {
@@ -863,7 +863,7 @@ struct Plan {
   size_t off_partial = 0, off_table = 0, total = 0;
   // symmetric paths
   int kmax_mut = 1;
-  int64_t mut_items = 0, chunk_blocks = 4;   // symmetric work item: chunk_blocks 64-source blocks
+  int64_t mut_items = 0, mut_tiles = 0, chunk_blocks = 4;   // symmetric work item: chunk_blocks 64-source blocks
   SmallVec<MutSys> msys;     // non-empty systems only
   size_t off_pi = 0, off_pj = 0, off_mtable = 0;
   // direct path
@@ -1130,7 +1130,7 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
                         : tile_pairs <= 36 * (int64_t)cu ? 2
                                                          : 4 * std::max<int64_t>(1, tile_pairs / (48 * (int64_t)cu));
     }
-    int64_t item = 0, pj = 0;
+    int64_t item = 0, pj = 0, tiles = 0;
     for (int s = 0; s < nsys; ++s) {
       MutSys M;
       M.b0 = offsets[s];
@@ -1140,12 +1140,15 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
       M.item0 = item;
       M.pi0 = item;
       M.pj0 = pj;
+      M.t0 = tiles;
+      tiles += M.n_t;
       item += blk ? items_before(M.n_t, M.n_t, pl.chunk_blocks)
                   : items_before_blocks(M.n_t, M.n_t, pl.chunk_blocks);
       pj += M.n_t * (M.n_t + 1) / 2;
       pl.msys.push_back(M);
     }
     pl.mut_items = item;
+    pl.mut_tiles = tiles;
     const size_t slot = (size_t)bs * ((mask & (kWF | kWT)) && (mask & (kUF | kUT)) ? 6 : 3) * sizeof(double);
     if (rc <= 0 && pl.kmax_mut > 2 && (size_t)(item + pj) * pl.kmax_mut * slot > kMutAutoBytes)
       pl.kmax_mut = group_k(k, 2);   // partial sums of 4 RHS too large: 2 per pass
@@ -1487,7 +1490,6 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     rp.nsys = q.nsys;
     rp.mask = pl.mask;
     rp.K = K;
-    rp.ntot = pl.ntot;
     rp.chunk_blocks = pl.chunk_blocks;
     rp.rhs_stride = stride;
     rp.a = a; rp.inva = inva; rp.c1 = c1; rp.c2 = c2;
@@ -1495,8 +1497,8 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     rp.periodic = periodic;
     for (int d = 0; d < 3; ++d) rp.L[d] = Lp[d];
     const int OC = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
-    const int64_t nout = pl.ntot * K * OC;
-    const dim3 rgrid((unsigned)((nout + kRedOut - 1) / kRedOut));
+    const int64_t tile_out = (pl.path == kBlocksPath ? 64 : kBlock) * OC;
+    const dim3 rgrid((unsigned)(pl.mut_tiles * (tile_out / kRedOut)), K);
     const dim3 rb(256);
     if (pl.path == kBlocksPath) {
       if (periodic) hipLaunchKernelGGL((mutual_reduce_kernel<true, 64>), rgrid, rb, 0, st, rp);
