@@ -116,8 +116,9 @@ int rmw_wall_rpy_apply(int mask, int prec, const double* r_vectors, const double
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as rmw_wall_rpy_apply; when the launch shape
  * rmw_wall_rpy_apply would choose needs more partial-sum space than the
- * array holds, the ordered kernel runs with longer source chunks (and
- * fewer right-hand sides per pass) so that it fits; sizes for which even
+ * array holds, the 256-blob tiles (fewer partial sums than 64-blob blocks)
+ * or the ordered kernel with longer source chunks (and fewer right-hand
+ * sides per pass) run so that it fits; sizes for which even
  * that does not fit (about 2.7 million blobs per right-hand side and
  * output block) return RMW_E_LIMIT before any launch.  Every call on one
  * device shares that device's array: calls that overlap in time on one
@@ -539,8 +540,9 @@ int rmw_seg_arnoldi_cgs2(double* V, int64_t ldv, int j, double* w, const rmw_seg
  * H_r[i*ldh + i + 1], H_r = H + r*h_rhs_stride), writes
  *   c_out[r*c_stride + j] = scale[r] * (sqrt+(T_r) e_1)_j,   j < m,
  * sqrt+ taking the square root of the non-negative eigenvalues (negative
- * ones -> 0) of an implicit-QL eigen-decomposition; status[r] = 1 when QL
- * did not converge.  This is the eigh step of stochastic_forcing_lanczos,
+ * ones -> 0): a quadrature of tridiagonal solves for a positive definite
+ * T_r, an implicit-QL eigen-decomposition otherwise; status[r] = 1 when QL
+ * did not converge.  scratch holds k m^2 doubles.  This is the eigh step of stochastic_forcing_lanczos,
  * stochastic_forcing/stochastic_forcing.py:208-227 (noise = V c).
  * ---------------------------------------------------------------------- */
 int rmw_lanczos_scratch_doubles(int m, int k, size_t* doubles);

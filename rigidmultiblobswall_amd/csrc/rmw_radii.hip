@@ -12,7 +12,9 @@
 // the 'radii*' implementations of set_mobility_vector_prod
 // (multi_bodies/multi_bodies.py:266-287).
 //
-// Two launches: the pair kernel (256 targets per workgroup in registers,
+// Small products take one launch (radii_direct_kernel), sources = targets the
+// symmetric kernels on 64-blob blocks or 256-blob tiles, the rest two launches:
+// the pair kernel (256 targets per workgroup in registers,
 // sources streamed through LDS as structure-of-arrays, each work item one
 // chunk of sources, FP64 partial sums per (chunk, target)) and a reduce
 // (fixed-order chunk sum, target damping).  The self pair needs no special

@@ -2,7 +2,12 @@
 //
 // One call evaluates any subset of the grand mobility blocks
 // [[UF, UT], [WF, WT]] for k right-hand sides on one suspension, or on a
-// ragged batch of independent suspensions, in two launches:
+// ragged batch of independent suspensions.  Few blobs take one launch
+// (rmw_wall_direct.hip), up to some thousand the symmetric kernel on 64-blob
+// blocks (rmw_wall_blocks.hip), larger suspensions the symmetric kernel on
+// 256-blob tiles below (section 3b), each followed by one reduce; what those
+// do not serve, or a tuning that asks for it, runs the ordered kernels in two
+// launches:
 //
 //   1. pair   : all-pairs sums; each workgroup owns 256 targets (one per
 //               lane, in registers) and one chunk of sources that it

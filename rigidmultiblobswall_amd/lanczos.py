@@ -10,7 +10,7 @@ that is one fused UF+UT+WF+WT launch).  Per right-hand side and step:
   w = M v_i;  full re-orthogonalisation of w against v_0..v_i (classical
   Gram-Schmidt twice, FP64 kernels) gives alpha_i = h_i and beta_i = ||w||,
   v_{i+1} = w / beta_i (e_0 if beta_i = 0, as the reference);
-  c_i = |z| factor sqrt+(T_i) e_1 from the GPU tridiagonal QL kernel.
+  c_i = |z| factor sqrt+(T_i) e_1 from the GPU square-root kernel.
 
 The reference forms noise_i = V_i c_i every step and stops when
 ||noise_i - noise_{i-1}|| / max(||noise_{i-1}||, eps) < tol.  With an
@@ -243,7 +243,7 @@ def lanczos_ragged(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torc
     c_prev = None
     i_last = 0
     zscr = None
-    C = torch.empty((R, mmax + 1), dtype=torch.float64, device=dev)       # last column: QL status
+    C = torch.empty((R, mmax + 1), dtype=torch.float64, device=dev)       # last column: status
     c_host = torch.empty((R, mmax + 1), dtype=torch.float64, pin_memory=True)
     for i in range(max_iter + 1):
         if i + 2 > mcap:                      # grow the basis and H geometrically
@@ -266,7 +266,7 @@ def lanczos_ragged(matvec: Callable[[torch.Tensor, torch.Tensor], None], Z: torc
         _lib.check(lib.rmw_lanczos_sqrt_coeffs(H.data_ptr(), H.stride(1), H.stride(2), m, R, scale.data_ptr(),
                                                C.data_ptr(), C.stride(0), zscr.data_ptr(), zscr.numel(),
                                                status.data_ptr(), _stream()))
-        # one read-back per step: the coefficients and the QL status together
+        # one read-back per step: the coefficients and the status together
         C[:, mmax] = status.to(torch.float64)
         c_host[:, :m].copy_(C[:, :m], non_blocking=True)
         c_host[:, mmax].copy_(C[:, mmax], non_blocking=True)

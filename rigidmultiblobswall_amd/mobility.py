@@ -16,7 +16,8 @@ Extra keyword arguments understood here:
              (mobility/mobility_numba.py:88).  Off by default, as there.
 
 The computation always runs on the GPU through librmw_hip; inputs given as
-numpy arrays are copied to the device and results copied back.  Inputs
+numpy arrays go to the device and results back (contiguous float64 arrays
+of up to 1 MiB through one pinned buffer, wall_rpy.apply_host).  Inputs
 given as torch device tensors stay on the device (the copy back to the
 host is the only transfer).
 """

@@ -177,6 +177,9 @@ def apply(mask: int, r_vectors, force=None, torque=None, eta: float = 1.0, a: fl
 # stream before it gives its buffer back).
 _STAGE_DOUBLES, _STAGES = 1 << 17, 8
 _stages: list = []
+# One call at a time per (device, stream): its inputs lie in that stream's
+# scratch between two of its launches.
+_host_locks: dict = {}
 _F64 = np.dtype(np.float64)
 
 
@@ -212,8 +215,9 @@ def apply_host(mask: int, r_vectors, force=None, torque=None, eta: float = 1.0, 
     tp = _lib.tuning_ptr(tun)
     nbytes = ctypes.c_size_t()
     _lib.check(lib.rmw_mobility_host_workspace_size(dom, mask, prec, n, tp, ctypes.byref(nbytes)))
-    ws = workspace(nbytes.value, device)
     L = _L_array(periodic_length)
+    st = _stream_ptr(device)
+    key = (device.index, st, "host")
     try:
         stage = _stages.pop()
     except IndexError:
@@ -224,8 +228,10 @@ def apply_host(mask: int, r_vectors, force=None, torque=None, eta: float = 1.0, 
     for x in ins:
         buf[o:o + n3] = x.reshape(-1)
         o += n3
-    _lib.check(lib.rmw_mobility_apply_host(dom, mask, prec, ptr, ptr + 8 * o, n, float(eta), float(a), L, tp,
-                                           ws.data_ptr(), ws.numel(), _stream_ptr(device)))
+    with _host_locks.setdefault(key, threading.Lock()):
+        ws = _workspace_of(key, nbytes.value, device)
+        _lib.check(lib.rmw_mobility_apply_host(dom, mask, prec, ptr, ptr + 8 * o, n, float(eta), float(a), L, tp,
+                                               ws.data_ptr(), ws.numel(), st))
     out = buf[o:o + nout].copy()
     if len(_stages) < _STAGES:
         _stages.append(stage)

@@ -70,13 +70,14 @@ def test_inputs_of_other_forms(gpu):
     assert np.array_equal(UF(r, f, 0.9, 0.4), want)
 
 
-def test_threads_and_streams(gpu):
-    systems = [_system(n) for n in (50, 300, 900, 1500)]
+@pytest.mark.parametrize("own_stream", [True, False])
+def test_threads_and_streams(gpu, own_stream):
+    systems = [_system(n) for n in (50, 300, 2500, 1500)]
     want = [UF(r, f, 0.9, 0.4) for r, f, _ in systems]
     wrong = []
 
     def work(q):
-        with torch.cuda.stream(torch.cuda.Stream()):
+        with torch.cuda.stream(torch.cuda.Stream() if own_stream else torch.cuda.default_stream()):
             for _ in range(20):
                 if not np.array_equal(UF(*systems[q][:2], 0.9, 0.4), want[q]):
                     wrong.append(q)
