@@ -742,7 +742,8 @@ __global__ __launch_bounds__(kPfBlock) void point_field_kernel(const double* __r
 // a workgroup has Y = N_b (-F - (M^-1 K)^T s) after reading the body's n x 6
 // block and needs no other rows than its own: one workgroup per body, in
 // three dependent phases, took 28.9 us for 100 bodies of 42 blobs (12.7 MB of
-// M^-1, 2.6 us at the rate of a copy), 9.5 now.  Four rows per wave at a time,
+// M^-1, 2.6 us at the rate of a copy), 9.5 in slices, 6.7 with
+// the first columns loaded ahead.  Four rows per wave at a time,
 // lanes across the columns.
 constexpr int kPcRows = 16;
 __global__ __launch_bounds__(kRigidBlock) void pc_apply_kernel(const int64_t* __restrict__ offs,

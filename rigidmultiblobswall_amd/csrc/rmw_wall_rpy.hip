@@ -989,8 +989,8 @@ constexpr double kDirectPairs = 2304.0 * 2304.0;
 // against tiles with 64-source items, us): UF fp32_blocked 36 / 39 at 4200,
 // 55.2 / 54.2 at 6000, 133 / 129 at 10752; FP64 45 / 52, 77 / 81, 212 / 217;
 // all four blocks 59 / 71, 105 / 108, 279 / 281; four right-hand sides of
-// them 150 / 169 at 4200, 463 / 451 at 8192; UF + UT with images 478 / 574 at
-// 6151, 800 / 850 at 8192.
+// them 150 / 169 at 4200, 463 / 451 at 8192; UF + UT with images 470 / 548 at
+// 6151, 753 / 819 at 8192.
 static double block_kernel_blobs(int mask, int prec, int K, bool periodic)
 {
   const bool light = K > 1 || (mask == kUF && prec != RMW_PREC_F64 && !periodic);
@@ -1116,7 +1116,8 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
       // runs of one source block while that leaves a CU fewer than 12 work
       // items, then two (fewer target-side sums: UF fp32_blocked 141.6 ->
       // 132.5 us at 10752 blobs), four for large batches; with images one
-      // up to twice that (478 against 501 us at 6151)
+      // up to three times that (478 against 501 us at 6151 before the divisions
+      // for the images went)
       const int64_t fine = (periodic ? 36 : 12) * (int64_t)cu;
       pl.chunk_blocks = block_pairs <= fine ? 1 : (block_pairs <= 144 * (int64_t)cu ? 2 : 4);
     } else if (tuning && tuning->chunk_len > 0) {
