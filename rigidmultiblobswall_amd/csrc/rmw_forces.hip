@@ -353,12 +353,16 @@ __global__ __launch_bounds__(kFBlock) void force_direct_kernel(ForceParams p, do
 //          arrive;
 //   place  first entry of every bucket (one atomic per workgroup: where a
 //          bucket lies does not matter);
-//   list   the blobs of every bucket, in order of arrival;
+//   list   the blobs of every bucket, in order of arrival, and an estimate of
+//          the pairs the cells will visit, from one blob of every sixteen
+//          (the lookups of the 27 cells by one lane for every bucket, in the
+//          sort, took 9 us; sixteen lanes to a sampled blob 2: 49 -> 43 us for
+//          32768 blobs, 35 -> 28 for 9001 in FP64 in a box);
 //   sort   blobs of a bucket by index (the order of arrival differs from run
-//          to run, the sums must not), positions gathered, and the number
-//          of pairs the cells will visit;
+//          to run, the sums must not), positions gathered;
 //   cells  every blob's force, sixteen lanes to a blob.
-// If more than a quarter of all ordered pairs would be visited, or a blob
+// If more than a quarter of all ordered pairs would be visited (by the
+// estimate, which depends on the blobs and their order alone), or a blob
 // does not fit the cell arithmetic, the last launch evaluates all pairs
 // instead: as the direct kernel does up to kDirectFallback blobs, by the
 // symmetric (or the ordered) kernel, whose reduce follows, beyond.
@@ -483,37 +487,19 @@ __global__ __launch_bounds__(256) void cells_place_kernel(CellParams c)
 __global__ __launch_bounds__(256) void cells_list_kernel(ForceParams p, CellParams c)
 {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n) return;
-  c.list[c.start[bucket_of(c.cell[i], c.mask)] + c.slot[i]] = (unsigned int)i;
-}
-
-template <bool F64>
-__global__ __launch_bounds__(256) void cells_sort_kernel(ForceParams p, CellParams c)
-{
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < p.n) c.list[c.start[bucket_of(c.cell[i], c.mask)] + c.slot[i]] = (unsigned int)i;
+  // sixteen lanes look up the 27 cells around one of their sixteen blobs
   unsigned long long visits = 0;
-  if (i < p.n && c.totals->unfit == 0) {
-    const unsigned long long cell = c.cell[i];
-    const unsigned int h = bucket_of(cell, c.mask), s = c.start[h], cnt = c.count[h];
-    unsigned int rank = 0;
-    for (unsigned int m = 0; m < cnt; m += 8) {   // eight loads in flight
-#pragma unroll
-      for (unsigned int u = 0; u < 8; ++u) {
-        const unsigned int k = m + u < cnt ? m + u : cnt - 1;
-        rank += c.list[s + k] < (unsigned int)i && m + u < cnt ? 1u : 0u;
-      }
+  const int64_t g0 = i & ~(int64_t)15;
+  if (g0 < p.n && c.totals->unfit == 0) {
+    const int group = p.n - g0 < 16 ? (int)(p.n - g0) : 16;
+    const int pick = (int)(((unsigned int)(g0 >> 4) * 2654435761u) >> 28);
+    const unsigned long long cell = c.cell[g0 + (pick < group ? pick : 0)];
+    for (int q = (int)(i & 15); q < 27; q += 16) {
+      unsigned long long nb;
+      if (neighbour(c, cell, q, nb)) visits += c.count[bucket_of(nb, c.mask)];
     }
-    c.index[s + rank] = (unsigned int)i;
-    c.scell[s + rank] = cell;
-    c.pos[s + rank] = make_double4(p.r[3 * i], p.r[3 * i + 1], p.r[3 * i + 2], radius_term<F64>(p, i));
-    if (rank == 0) {   // the bucket's first blob speaks for all of them
-#pragma unroll
-      for (int q = 0; q < 27; ++q) {
-        unsigned long long nb;
-        if (neighbour(c, cell, q, nb)) visits += c.count[bucket_of(nb, c.mask)];
-      }
-      visits *= cnt;
-    }
+    visits *= group;
   }
   // one atomic per workgroup: they go to one address, one after the other
   __shared__ unsigned long long s_visits[4];
@@ -521,6 +507,27 @@ __global__ __launch_bounds__(256) void cells_sort_kernel(ForceParams p, CellPara
   if ((threadIdx.x & 63) == 0) s_visits[threadIdx.x >> 6] = visits;
   __syncthreads();
   if (threadIdx.x == 0) atomicAdd(&c.totals->pairs, s_visits[0] + s_visits[1] + s_visits[2] + s_visits[3]);
+}
+
+template <bool F64>
+__global__ __launch_bounds__(256) void cells_sort_kernel(ForceParams p, CellParams c)
+{
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.n || c.totals->unfit != 0) return;
+  const unsigned long long cell = c.cell[i];
+  const double x = p.r[3 * i], y = p.r[3 * i + 1], z = p.r[3 * i + 2], rad = radius_term<F64>(p, i);
+  const unsigned int h = bucket_of(cell, c.mask), s = c.start[h], cnt = c.count[h];
+  unsigned int rank = 0;
+  for (unsigned int m = 0; m < cnt; m += 8) {   // eight loads in flight
+#pragma unroll
+    for (unsigned int u = 0; u < 8; ++u) {
+      const unsigned int k = m + u < cnt ? m + u : cnt - 1;
+      rank += c.list[s + k] < (unsigned int)i && m + u < cnt ? 1u : 0u;
+    }
+  }
+  c.index[s + rank] = (unsigned int)i;
+  c.scell[s + rank] = cell;
+  c.pos[s + rank] = make_double4(x, y, z, rad);
 }
 
 __device__ __forceinline__ bool cells_pay(const CellParams& c)
@@ -685,7 +692,8 @@ __global__ __launch_bounds__(256) void force_mutual_reduce_kernel(const double* 
 
 // Up to direct_blobs blobs one launch over all pairs, beyond it the cells
 // (unless the tuning names a launch shape: then the kernel it was made for).
-// The cells cost about 30 us whatever the size.  Measured on the rollers strip
+// The cells cost some 25 us whatever the size (30 when these were measured, the
+// lines lie a little high for it).  Measured on the rollers strip
 // at 4096 blobs, direct / cells (us): fp32 21 / 36 open, 43 / 39 periodic;
 // FP64 38 / 31 open and 61 / 33 periodic with the cutoff; without it the FP64
 // range (746 Debye lengths) holds most of so small a suspension and the
