@@ -90,8 +90,10 @@ RMW_HD double rcp(double x) { return 1.0 / x; }
 RMW_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 RMW_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// The smaller of x and a constant; a NaN x gives the constant (the pairs
-// concerned keep an unclamped factor that carries the NaN).
+// The smaller of x and a constant; a NaN x gives the constant.  Blobs at one
+// point and non-finite positions (|d| = NaN) must still give non-finite
+// results: every coefficient keeps a factor of 1/|d| or a term in |d| that is
+// not clamped.
 RMW_HD float min_(float x, float c) { return __builtin_fminf(x, c); }
 RMW_HD double min_(double x, double c) { return __builtin_fmin(x, c); }
 
@@ -291,7 +293,9 @@ template <typename T> struct CoefRot {
   T F4;   // F4
 };
 
-// RPY: c = 1/r^3 far, (1 - 3r/8)/2 overlapping: ic^3 + (3/8 - 3 rm/16).
+// RPY: c = 1/r^3 far, (1 - 3r/8)/2 overlapping: ic^3 + (3/8 - 3 rm/16).  The
+// term 0 r is NaN where r is (no other factor here is), and costs the FMA that
+// adds it (a clamp that keeps a NaN: a compare and a select).
 // Wall, for h = h_hat R_z, with q = 1/|R|, w = q^2, b = R_z w:
 //   F1 = w,  F4 = -2 w q (h - b),  F3 = -2 w q B,  F2 = 2 w^2 (1 + 2 R_z B),
 //   B = 3 h - 5 b   (h_hat e_z^2 = h b and h_hat e_z = h q: no division).
@@ -299,7 +303,7 @@ template <typename T>
 RMW_HD CoefRot<T> coef_rot(const Geom<T>& g, T hnum, int dom = kDomWall)
 {
   CoefRot<T> c;
-  c.c = fma_(g.ic * g.ic, g.ic, fma_(T(-0.1875), g.rm, T(0.375)));
+  c.c = fma_(g.ic * g.ic, g.ic, fma_(T(-0.1875), g.rm, fma_(T(0), g.r, T(0.375))));
   if (!dom_has_wall(dom)) {
     c.F1r = T(0); c.F2r = T(0); c.F3r2 = T(0); c.F4 = T(0);
     return c;

@@ -240,6 +240,37 @@ def test_masked_geometry_gives_exact_zeros():
                 assert np.all(np.isfinite(on)) and np.abs(on).max() > 0.0
 
 
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("what", ["one point", "nan x", "nan y", "nan z", "inf x", "-inf y", "inf z"])
+def test_pairs_at_one_point_and_non_finite_positions_stay_non_finite(what, prec):
+    """Two blobs at one point, or a blob whose position is not finite: every
+    component of every block, its transpose and its explicit matrix's rows
+    and columns is non-finite in every boundary that has the block (the
+    products promise it, and their finite check reports it)."""
+    lib = ctypes.CDLL(os.path.join(REPO, "tests", "helpers", "libpair_terms_host.so"))
+    dp = ctypes.POINTER(ctypes.c_double)
+    P = lambda x: x.ctypes.data_as(dp)   # noqa: E731
+    fn = getattr(lib, "pt_masked_blocks_" + prec)
+    fn.argtypes = [dp, dp, ctypes.c_int, dp]
+    for swap in (False, True):
+        ri, rj = np.array([0.3, 0.1, 1.4]), np.array([0.3, 0.1, 1.4])
+        if what != "one point":
+            rj = np.array([-0.7, 0.9, 1.1])
+            val, axis = what.split()
+            ri["xyz".index(axis)] = float(val)
+        if swap:
+            ri, rj = rj, ri
+        m = np.empty(324)
+        assert fn(P(ri), P(rj), 1, P(m)) == 324
+        bad = ~np.isfinite(m)
+        # [domain][unit vector][block form][component]; the free surface has the UF block only
+        blocks = bad[:288].reshape(4, 3, 8, 3).any(axis=1)
+        assert blocks[:3].all(), (what, swap, np.argwhere(~blocks[:3]))
+        assert blocks[3, :2].all(), (what, swap)
+        mats = bad[288:].reshape(4, 3, 3)
+        assert mats.any(axis=1).all() and mats.any(axis=2).all(), (what, swap)
+
+
 def test_work_item_schedule_covers_every_tile_pair_once():
     """The work-item decode of the symmetric kernels (rmw_tile_pairs.h,
     host build): items of C 64-source blocks (C = 1, 2 or a multiple of 4)

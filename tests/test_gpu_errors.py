@@ -53,6 +53,32 @@ def test_grand_mobility_coincident_blobs_reported(gpu):
     assert ei.value.code == _lib.RMW_E_NOTFINITE
 
 
+ORDERED = dict(symmetric=-1)
+
+
+@pytest.mark.parametrize("mask", [2, 3, 4, 5, 8, 10, 12, 15])
+@pytest.mark.parametrize("n,tuning", [(500, None), (3000, None), (10240, None), (700, ORDERED)],
+                         ids=["direct", "blocks", "tiles", "ordered"])
+def test_coincident_blobs_reported_by_every_block(gpu, mask, n, tuning):
+    """The two blobs at one point get non-finite rows in every output of
+    every mask, on every route, with one right-hand side and with two (which
+    several routes evaluate through the blocks' matrices)."""
+    r = _suspension(n, 11)
+    rng = np.random.default_rng(12)
+    f, t = rng.standard_normal((2, n, 3)), rng.standard_normal((2, n, 3))
+    for domain, prec, k in (("single_wall", "fp32_blocked", 1), ("single_wall", "fp32_blocked", 2),
+                            ("single_wall", "fp64", 1), ("no_wall", "fp32_blocked", 1), ("no_wall", "fp64", 1)):
+        print(f"case coincident blobs mask={mask} n={n} {domain} {prec} k={k}", flush=True)
+        kw = dict(force=f[:k], torque=t[:k], eta=1e-3, a=0.656, k=k, precision=prec, domain=domain, tuning=tuning)
+        for out in wall_rpy.apply(mask, r, **kw):
+            if out is not None:
+                bad = ~torch.isfinite(out.reshape(k, n, 3))
+                assert bool(bad[:, [n // 3, n // 2]].all()) and int(bad.sum()) == 6 * k
+        with pytest.raises(_lib.RmwError) as ei:
+            wall_rpy.apply(mask, r, check_finite=True, **kw)
+        assert ei.value.code == _lib.RMW_E_NOTFINITE
+
+
 def test_finite_check_passes_valid_products(gpu):
     """With distinct positions the checked call returns the same product."""
     for n in (500, 8192):
