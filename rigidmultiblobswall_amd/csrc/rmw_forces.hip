@@ -364,12 +364,12 @@ __global__ __launch_bounds__(kFBlock) void force_direct_kernel(ForceParams p, do
 // If more than a quarter of all ordered pairs would be visited (by the
 // estimate, which depends on the blobs and their order alone), or a blob
 // does not fit the cell arithmetic, the last launch evaluates all pairs
-// instead: as the direct kernel does up to kDirectFallback blobs, by the
+// instead: as the direct kernel does up to direct_fallback blobs, by the
 // symmetric (or the ordered) kernel, whose reduce follows, beyond.
 // ---------------------------------------------------------------------------
 struct CellTotals {
   unsigned int cursor;       // entries given out so far
-  unsigned int unfit;        // blobs that do not fit the cell arithmetic
+  unsigned int unfit;        // 1: a blob does not fit the cell arithmetic
   unsigned long long pairs;  // pairs the cells will visit
 };
 
@@ -450,18 +450,45 @@ __global__ __launch_bounds__(256) void cells_zero_kernel(CellParams c)
   if (i == 0) *c.totals = CellTotals{0u, 0u, 0ull};
 }
 
+// Atomics on one counter follow one another at some 12 ns each, which for
+// thousands of blobs in a few cells was the time of the whole call: up to eight
+// buckets of a wave's blobs take their places by one atomic each (30000 blobs in
+// eight cells: 343 us by one atomic per blob, 8 so).
 __global__ __launch_bounds__(256) void cells_count_kernel(ForceParams p, CellParams c)
 {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n) return;
-  int k[3] = {0, 0, 0};
-  bool fits = true;
+  const int lane = threadIdx.x & 63;
+  bool open = i < p.n;   // a blob without a place
+  unsigned int h = 0;
+  if (open) {
+    int k[3] = {0, 0, 0};
+    bool fits = true;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) fits = cell_of(c, d, p.r[3 * i + d], p.L[d], k[d]) && fits;
-  if (!fits) atomicAdd(&c.totals->unfit, 1u);
-  const unsigned long long cell = fits ? pack_cell(k[0], k[1], k[2]) : 0ull;
-  c.cell[i] = cell;
-  c.slot[i] = atomicAdd(&c.count[bucket_of(cell, c.mask)], 1u);
+    for (int d = 0; d < 3; ++d) fits = cell_of(c, d, p.r[3 * i + d], p.L[d], k[d]) && fits;
+    if (!fits) c.totals->unfit = 1u;
+    const unsigned long long cell = fits ? pack_cell(k[0], k[1], k[2]) : 0ull;
+    c.cell[i] = cell;
+    h = bucket_of(cell, c.mask);
+  }
+  unsigned long long mates = 1ull << lane;   // the lanes that share an atomic, its first lane
+  int first = lane;
+  for (int t = 0; t < 8; ++t) {
+    const unsigned long long left = __ballot(open);
+    if (left == 0) break;
+    const int f = __ffsll(left) - 1;
+    const bool with = open && h == (unsigned int)__shfl((int)h, f, 64);
+    const unsigned long long m = __ballot(with);
+    if (with) {
+      mates = m;
+      first = f;
+      open = false;
+    }
+    if (__popcll(m) < 4) break;   // few blobs to a bucket: not worth sharing
+  }
+  unsigned int base = 0;
+  if (i < p.n && lane == first) base = atomicAdd(&c.count[h], (unsigned int)__popcll(mates));
+  base = (unsigned int)__shfl((int)base, first, 64);
+  if (i < p.n) c.slot[i] = base + (unsigned int)__popcll(mates & ((1ull << lane) - 1));
 }
 
 __global__ __launch_bounds__(256) void cells_place_kernel(CellParams c)
@@ -509,11 +536,16 @@ __global__ __launch_bounds__(256) void cells_list_kernel(ForceParams p, CellPara
   if (threadIdx.x == 0) atomicAdd(&c.totals->pairs, s_visits[0] + s_visits[1] + s_visits[2] + s_visits[3]);
 }
 
+__device__ __forceinline__ bool cells_pay(const CellParams& c)
+{
+  return c.totals->unfit == 0 && c.totals->pairs <= c.dense;
+}
+
 template <bool F64>
 __global__ __launch_bounds__(256) void cells_sort_kernel(ForceParams p, CellParams c)
 {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n || c.totals->unfit != 0) return;
+  if (i >= p.n || !cells_pay(c)) return;
   const unsigned long long cell = c.cell[i];
   const double x = p.r[3 * i], y = p.r[3 * i + 1], z = p.r[3 * i + 2], rad = radius_term<F64>(p, i);
   const unsigned int h = bucket_of(cell, c.mask), s = c.start[h], cnt = c.count[h];
@@ -528,11 +560,6 @@ __global__ __launch_bounds__(256) void cells_sort_kernel(ForceParams p, CellPara
   c.index[s + rank] = (unsigned int)i;
   c.scell[s + rank] = cell;
   c.pos[s + rank] = make_double4(x, y, z, rad);
-}
-
-__device__ __forceinline__ bool cells_pay(const CellParams& c)
-{
-  return c.totals->unfit == 0 && c.totals->pairs <= c.dense;
 }
 
 // Force of one blob by the sixteen lanes of its group.  The lanes look up the
@@ -692,21 +719,26 @@ __global__ __launch_bounds__(256) void force_mutual_reduce_kernel(const double* 
 
 // Up to direct_blobs blobs one launch over all pairs, beyond it the cells
 // (unless the tuning names a launch shape: then the kernel it was made for).
-// The cells cost some 25 us whatever the size (30 when these were measured, the
-// lines lie a little high for it).  Measured on the rollers strip
-// at 4096 blobs, direct / cells (us): fp32 21 / 36 open, 43 / 39 periodic;
-// FP64 38 / 31 open and 61 / 33 periodic with the cutoff; without it the FP64
-// range (746 Debye lengths) holds most of so small a suspension and the
-// cells only cost.
+// The cells cost 25 to 31 us whatever the size, seven launches; the direct
+// kernel's time rises in steps of 1024 blobs (a workgroup per CU).  Rollers
+// strip, direct / cells (us): fp32 open 26 / 28 at 5120 blobs, 33 / 28 at 5600,
+// periodic 24 / 27 at 3000, 33 / 26 at 3300; FP64 with the cutoff open 22 / 26
+// at 3000, 29 / 26 at 3300, periodic 25.5 / 26.5 at 2300, 29 / 26 at 2600.
+// Without it the FP64 range (746 Debye lengths) holds most of so small a
+// suspension: open 69 / 78 at 6000, 85 / 79 at 6500, periodic 80 / 94 at 5120,
+// 104 / 95 at 5600.
 static int64_t direct_blobs(bool f64, bool periodic, bool cutoff)
 {
-  if (!f64) return periodic ? 3584 : 5120;
-  if (!cutoff) return periodic ? 4096 : 5120;
-  return periodic ? 2816 : 3584;
+  if (!f64) return periodic ? 3072 : 5120;
+  if (!cutoff) return periodic ? 5120 : 6144;
+  return periodic ? 2304 : 3072;
 }
 // Blobs up to which a suspension that the cells turn out not to suit goes
-// through the direct kernel (39 against 60 us at 4096 in FP64).
-constexpr int64_t kDirectFallback = 8192;
+// through the direct kernel; direct / symmetric kernel and reduce (us): fp32
+// open 35 / 51 at 6000, 46 / 52 at 7000, 60 / 67 at 8192, periodic 82 / 102 at
+// 6000, 110 / 103 at 7000; FP64 open 71 / 87 and 95 / 88, periodic 114 / 136 and
+// 152 / 137.
+static int64_t direct_fallback(bool f64, bool periodic) { return f64 || periodic ? 6400 : 8192; }
 // Beyond these exponents (r - 2a)/b the exponential is exactly 0.
 constexpr double kRangeF64 = 746.0, kRangeF32 = 104.5;
 
@@ -815,7 +847,7 @@ static void launch_force(bool mutual, const ForceParams& q, int grid, hipStream_
 
 template <bool F64, bool CUT>
 static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const CellParams& c, double scale,
-                               double* force, hipStream_t st)
+                               bool small, double* force, hipStream_t st)
 {
   const dim3 b(kFBlock), nb((unsigned)((q.n + 255) / 256)), hb(pl.buckets / 256);
   hipLaunchKernelGGL(cells_zero_kernel, hb, b, 0, st, c);
@@ -823,7 +855,6 @@ static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const 
   hipLaunchKernelGGL(cells_place_kernel, hb, b, 0, st, c);
   hipLaunchKernelGGL(cells_list_kernel, nb, b, 0, st, q, c);
   hipLaunchKernelGGL(cells_sort_kernel<F64>, nb, b, 0, st, q, c);
-  const bool small = q.n <= kDirectFallback;
   const int64_t all = small ? (q.n + kDT - 1) / kDT : pl.total_items;
   const int64_t wgs = (q.n * kCellLanes + kFBlock - 1) / kFBlock;
   const dim3 g((unsigned)std::min<int64_t>(std::max(wgs, all), (int64_t)INT32_MAX));
@@ -838,12 +869,12 @@ static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const 
 
 template <bool F64, bool CUT>
 static void launch_any(const ForcePlan& pl, const ForceParams& q, const CellParams& c, bool direct, bool cells,
-                       double scale, double* force, int grid, hipStream_t st)
+                       bool small, double scale, double* force, int grid, hipStream_t st)
 {
   if (direct)
     hipLaunchKernelGGL((force_direct_kernel<F64, CUT>), dim3((unsigned)((q.n + kDT - 1) / kDT)), dim3(kFBlock), 0, st, q,
                        scale, force);
-  else if (cells) launch_force_cells<F64, CUT>(pl, q, c, scale, force, st);
+  else if (cells) launch_force_cells<F64, CUT>(pl, q, c, scale, small, force, st);
   else launch_force<F64, CUT>(pl.mutual, q, grid, st);
 }
 
@@ -947,19 +978,20 @@ extern "C" int rmw_blob_forces(int prec, const double* r_vectors, const double* 
     }
     // what the cells cannot serve goes the same way as what they turn out not
     // to suit
-    const bool direct = pl.direct || (pl.cells && !cells && !in_place && n <= kDirectFallback);
+    const bool small = n <= direct_fallback(f64, boxed);
+    const bool direct = pl.direct || (pl.cells && !cells && !in_place && small);
     double* const out = direct && in_place ? (double*)workspace : force;
     if (f64) {
-      if (cut) launch_any<true, true>(pl, q, c, direct, cells, scale, out, grid, st);
-      else launch_any<true, false>(pl, q, c, direct, cells, scale, out, grid, st);
+      if (cut) launch_any<true, true>(pl, q, c, direct, cells, small, scale, out, grid, st);
+      else launch_any<true, false>(pl, q, c, direct, cells, small, scale, out, grid, st);
     } else {
-      if (cut) launch_any<false, true>(pl, q, c, direct, cells, scale, out, grid, st);
-      else launch_any<false, false>(pl, q, c, direct, cells, scale, out, grid, st);
+      if (cut) launch_any<false, true>(pl, q, c, direct, cells, small, scale, out, grid, st);
+      else launch_any<false, false>(pl, q, c, direct, cells, small, scale, out, grid, st);
     }
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
     if (out != force) launch_copy_rows(out, 3 * n, force, 3 * n, 3 * n, 1, st);
-    if (direct || (cells && n <= kDirectFallback)) return;
+    if (direct || (cells && small)) return;
     const dim3 rg((unsigned)((n * 3 + 255) / 256)), rb(256);
     if (pl.mutual)
       hipLaunchKernelGGL(force_mutual_reduce_kernel, dim3((unsigned)((n * 3 + kFRedOut - 1) / kFRedOut)), rb, 0, st,
