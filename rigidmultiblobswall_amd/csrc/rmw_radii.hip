@@ -181,9 +181,14 @@ __global__ void radii_zero_kernel(double* __restrict__ out, int64_t n)
 //    25 / 20 (FP64 16 / 16, 20 / 20, 37 / 26); blocks / tiles at 2304 blobs
 //    20 / 113, 6000 66 / 126, 10007 152 / 192, 18000 422 / 430, 20480
 //    527 / 535, 32768 1311 / 1287 (FP64 10007 246 / 311, 18000 744 / 748).
-//  - ordered chunks of at least 64 sources (256 before: 97 at 1000 x 5000),
-//    256 beyond 65536 sources, whose partial sums the reduce would walk for
-//    longer than the pairs take (1000000 x 5: 2511 against 1025).
+//  - ordered chunks of 64 to 256 sources, at most 256 of them (until 256 sources
+//    to a chunk): few sources leave the chip idle in long chunks (1000 x 5000,
+//    chunks of 256: 97), many in short ones give the reduce, one thread to an
+//    output, more partial sums than the pairs take time for.  Chunks of
+//    64 / 128 / 192 / 256: 12000 x 400 59 / 67 / 87 / 108, 20000 x 2000
+//    140 / 125 / 140 / 145, 30000 x 1000 151 / 121 / 125 / 128, 45000 x 600
+//    186 / 150 / 135 / 158, 65536 x 64 182 / 126 / 129 / 136, 65536 x 700
+//    252 / 190 / 193 / 170, 1000000 x 5 2462 / 1510 / 1184 / 1031.
 constexpr int kRDT = 4;      // targets of a workgroup of the direct kernel
 constexpr double kRDirectPairs = 2304.0 * 2304.0, kRDirectSelf = 1600.0 * 1600.0;
 constexpr int64_t kRDirectSources = 8192, kRDirectTargets = 256;   // targets per source
@@ -219,7 +224,8 @@ static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* 
   int64_t chunk = tuning && tuning->chunk_len > 0 ? tuning->chunk_len : 0;
   if (chunk <= 0) {
     const double c = (double)ns * (double)nt / (16.0 * std::max(device_props().cu_count, 1) * kRBlock);
-    chunk = std::max<int64_t>(ns <= 65536 ? 64 : kRBlock, (int64_t)std::ceil(c / 64.0) * 64);
+    const int64_t least = std::min<int64_t>(kRBlock, std::max<int64_t>(64, (ns / 256 + 63) / 64 * 64));
+    chunk = std::max<int64_t>(least, (int64_t)std::ceil(c / 64.0) * 64);
   }
   chunk = std::max<int64_t>(64, (chunk + 63) / 64 * 64);
   if (ns > 0) chunk = std::min<int64_t>(chunk, (ns + 63) / 64 * 64);
