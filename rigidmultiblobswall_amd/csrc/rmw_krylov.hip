@@ -469,6 +469,15 @@ extern "C" int rmw_axpby(double alpha, const double* x, double beta, double* y, 
 // Partial sums that every block adds up by itself, at most: beyond (a basis of
 // many long vectors) turning them into coefficients once is cheaper.
 constexpr int64_t kSelfSums = 32768;
+// m^2 n up to which the four launches are taken for one basis of m vectors: they
+// save some 16 us of launches, but a block's dot products follow one another, so
+// long bases go faster through the separate launches.  Four launches / separate,
+// us: n = 15000 58 / 65 at m = 60, 97 / 98 at 100, 162 / 151 at 150; 60000 58 / 66
+// at 45, 86 / 86 at 60, 124 / 115 at 80; 200000 55 / 69 at 20, 86 / 91 at 30,
+// 131 / 124 at 45; 1000000 59 / 69 at 5, 128 / 122 at 12, 313 / 253 at 30.
+// Several bases share the four launches, and the separate ones are made for each
+// in turn (four bases of 1000000: 654 / 833 at m = 20).
+constexpr double kFusedSize = 1.2e8;
 
 // One CGS2 step of one basis in the launches of the separate operations.
 static void arnoldi_separate(const DotLaunch& L, hipStream_t st, double* V, int64_t ldv, int m, double* w, int64_t n,
@@ -501,9 +510,10 @@ static void arnoldi_batch(double* V, int64_t ldv, int64_t v_rhs, int j, int k, d
   const DotLaunch L = dot_launch(n);
   RMW_REQUIRE(workspace_bytes >= (size_t)L.G * (m + 1) * sizeof(double), "workspace too small");
   const int64_t per = (int64_t)L.G * (2 * m + 1);
-  if (L.E > 0 && (int64_t)L.G * m <= kSelfSums && workspace_bytes >= (size_t)per * sizeof(double)) {
-    // as many bases per launch as the workspace has partial sums for
-    const int fit = (int)std::min<int64_t>(k, (int64_t)(workspace_bytes / sizeof(double)) / per);
+  // as many bases per launch as the workspace has partial sums for
+  const int fit = (int)std::min<int64_t>(k, (int64_t)(workspace_bytes / sizeof(double)) / per);
+  if (L.E > 0 && (int64_t)L.G * m <= kSelfSums && fit > 0 &&
+      (double)m * m * (double)n <= kFusedSize * (double)fit * fit) {
     for (int r0 = 0; r0 < k; r0 += fit) {
       ArnoldiParams p{V + r0 * v_rhs, ldv, v_rhs, w + r0 * w_rhs, w_rhs, n, h + r0 * h_rhs, h_rhs,
                       h_host, (double*)workspace, per, m};
