@@ -1013,10 +1013,12 @@ static SmallVec<DirectSys> direct_table(const int64_t* offsets, int nsys, int tt
 
 // offsets: host array of nsys + 1 blob offsets (offsets[0] = 0).  periodic:
 // the call has pseudo-periodic images (the symmetric wall kernels then take
-// one right-hand side per pass, so their partial sums are sized for one).
+// one right-hand side per pass, so their partial sums are sized for one).  cap:
+// bytes that the partial sums of an automatically chosen symmetric layout may
+// take.
 static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int k,
                       const rmw_tuning* tuning, bool ragged, int domain = kDomWall, bool periodic = false,
-                      bool fine_blocks = true)
+                      size_t cap = kMutAutoBytes)
 {
   RMW_REQUIRE(valid_mask(mask), "mask must be a non-empty subset of UF|UT|WF|WT");
   RMW_REQUIRE(domain >= kDomWall && domain <= kDomFreeSurface, "unknown domain");
@@ -1093,12 +1095,12 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
   }
   const int cu = std::max(device_props().cu_count, 1);
   const int kgroup = periodic || domain != kDomWall || (mask != kUF && mask != 15) ? 1 : group_k(k, 4);
+  const bool tiles_ok = sym_ok && (sym > 0 || (sym == 0 && tile_pairs >= cu));
   if (!shaped && direct_work <= (nsys > 1 ? 0.25 : 1.0) * kDirectPairs)
     pl.path = kDirectPath;
-  else if (!shaped && sym_ok && fine_blocks &&
-           pairs <= block_kernel_blobs(mask, prec, kgroup, periodic) * (double)pl.ntot)
+  else if (!shaped && sym_ok && pairs <= block_kernel_blobs(mask, prec, kgroup, periodic) * (double)pl.ntot)
     pl.path = kBlocksPath;
-  else if (sym_ok && (sym > 0 || (sym == 0 && tile_pairs >= cu)))
+  else if (tiles_ok)
     pl.path = kTilesPath;
 
   size_t o = 0;
@@ -1110,60 +1112,91 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
     pl.kmax_mut = domain == kDomWall && mask != (kUF | kUT) && !single_rot && !periodic
                       ? group_k(k, rc > 0 ? std::min(rc, 4) : 4)
                       : 1;
-    const bool blk = pl.path == kBlocksPath;
-    const int64_t bs = blk ? 64 : kBlock;
-    if (blk) {
+    // Layouts in the order of their speed; the first whose partial sums fit is
+    // taken, with all right-hand sides of a pass before two (the source-side
+    // slots grow as N^2 and with the right-hand sides), and the ordered kernel
+    // where nothing fits.  ms for four right-hand sides of all four blocks:
+    // 96 systems of 4096 blobs, two per pass by blocks 12.9, four by tiles 10.0;
+    // 192, ordered 35.9, tiles 20.6; one of 64000, 26.7 / 23.1 (two / four);
+    // 90000, ordered 60.3, two per pass 53.4.  In the library's own array two
+    // right-hand sides fit only in runs that keep few CUs busy: there the ordered
+    // kernel comes next (10000 blobs: 0.80, two per pass 0.97).
+    const bool fewer = rc <= 0 && cap >= kMutAutoBytes;
+    struct Layout { bool blk; int64_t chunk; };
+    Layout layouts[3];
+    int count = 0;
+    if (pl.path == kBlocksPath) {
       // runs of one source block while that leaves a CU fewer than 12 work
       // items, then two (fewer target-side sums: UF fp32_blocked 141.6 ->
       // 132.5 us at 10752 blobs), four for large batches; with images one
       // up to three times that (478 against 501 us at 6151 before the divisions
       // for the images went)
       const int64_t fine = (periodic ? 36 : 12) * (int64_t)cu;
-      pl.chunk_blocks = block_pairs <= fine ? 1 : (block_pairs <= 144 * (int64_t)cu ? 2 : 4);
-    } else if (tuning && tuning->chunk_len > 0) {
+      layouts[count++] = {true, block_pairs <= fine ? 1 : (block_pairs <= 144 * (int64_t)cu ? 2 : 4)};
+    }
+    if (tuning && tuning->chunk_len > 0) {
       // 64 or 128 sources: a quarter or half of a tile pair per work item
       // (finer work for suspensions of few tiles); else whole source tiles
       const int64_t blocks = (tuning->chunk_len + 63) / 64;
-      pl.chunk_blocks = blocks <= 2 ? blocks : (blocks + 3) / 4 * 4;
-    } else {
+      layouts[count++] = {false, blocks <= 2 ? blocks : (blocks + 3) / 4 * 4};
+    } else if (tiles_ok) {
       // quarter tiles while they balance the CUs better than they cost in
       // partial sums, then half and whole tiles (us at 64 / 128 / 256 sources:
       // UF fp32_blocked 129 / 139 / 152 at 10752 blobs, 618 / 575 / 589 at 24576,
       // 1777 / 1694 / 1676 at 43008; four right-hand sides of all four blocks
-      // 882 / 866 / 967 at 12000, 6271 / 6089 / 6081 at 32768)
+      // 882 / 866 / 967 at 12000, 6271 / 6089 / 6081 at 32768); runs of tiles
+      // with a third of the target-side sums where those do not fit
       const int64_t quarter = (pl.kmax_mut > 1 ? 4 : 8) * (int64_t)cu + 64;
-      pl.chunk_blocks = tile_pairs <= quarter ? 1
-                        : tile_pairs <= 36 * (int64_t)cu ? 2
-                                                         : 4 * std::max<int64_t>(1, tile_pairs / (48 * (int64_t)cu));
+      layouts[count++] = {false, tile_pairs <= quarter ? 1
+                                 : tile_pairs <= 36 * (int64_t)cu
+                                     ? 2
+                                     : 4 * std::max<int64_t>(1, tile_pairs / (48 * (int64_t)cu))};
+      layouts[count++] = {false, 4 * std::max<int64_t>(1, tile_pairs / (16 * (int64_t)cu))};
     }
-    int64_t item = 0, pj = 0, tiles = 0;
-    for (int s = 0; s < nsys; ++s) {
-      MutSys M;
-      M.b0 = offsets[s];
-      M.n = offsets[s + 1] - offsets[s];
-      if (M.n == 0) continue;
-      M.n_t = (M.n + bs - 1) / bs;
-      M.item0 = item;
-      M.pi0 = item;
-      M.pj0 = pj;
-      M.t0 = tiles;
-      tiles += M.n_t;
-      item += blk ? items_before(M.n_t, M.n_t, pl.chunk_blocks)
-                  : items_before_blocks(M.n_t, M.n_t, pl.chunk_blocks);
-      pj += M.n_t * (M.n_t + 1) / 2;
-      pl.msys.push_back(M);
+    const int OCm = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
+    bool fits = false;
+    for (int q = 0; !fits; ++q) {
+      if (q == count) {   // no layout: two right-hand sides per pass, or a required one beyond the limit
+        if (fewer && pl.kmax_mut > 2) {
+          pl.kmax_mut = 2;
+          q = 0;
+        } else {
+          if (sym <= 0) break;
+          fits = true;
+          q = count - 1;
+        }
+      }
+      const bool blk = layouts[q].blk;
+      const int64_t bs = blk ? 64 : kBlock, chunk_blocks = layouts[q].chunk;
+      int64_t item = 0, pj = 0, tiles = 0;
+      pl.msys.clear();
+      for (int s = 0; s < nsys; ++s) {
+        MutSys M;
+        M.b0 = offsets[s];
+        M.n = offsets[s + 1] - offsets[s];
+        if (M.n == 0) continue;
+        M.n_t = (M.n + bs - 1) / bs;
+        M.item0 = item;
+        M.pi0 = item;
+        M.pj0 = pj;
+        M.t0 = tiles;
+        tiles += M.n_t;
+        item += blk ? items_before(M.n_t, M.n_t, chunk_blocks) : items_before_blocks(M.n_t, M.n_t, chunk_blocks);
+        pj += M.n_t * (M.n_t + 1) / 2;
+        pl.msys.push_back(M);
+      }
+      const size_t slot = (size_t)pl.kmax_mut * bs * OCm * sizeof(double);
+      o = 0;
+      pl.off_pi = o; o = align_up(o + (size_t)item * slot);
+      pl.off_pj = o; o = align_up(o + (size_t)pj * slot);
+      if (pl.msys.size() > 1) { pl.off_mtable = o; o = align_up(o + pl.msys.size() * sizeof(MutSys)); }
+      fits = fits || o <= cap;
+      pl.path = blk ? kBlocksPath : kTilesPath;
+      pl.chunk_blocks = chunk_blocks;
+      pl.mut_items = item;
+      pl.mut_tiles = tiles;
     }
-    pl.mut_items = item;
-    pl.mut_tiles = tiles;
-    const size_t slot = (size_t)bs * ((mask & (kWF | kWT)) && (mask & (kUF | kUT)) ? 6 : 3) * sizeof(double);
-    if (rc <= 0 && pl.kmax_mut > 2 && (size_t)(item + pj) * pl.kmax_mut * slot > kMutAutoBytes)
-      pl.kmax_mut = group_k(k, 2);   // partial sums of 4 RHS too large: 2 per pass
-    pl.off_pi = o; o = align_up(o + (size_t)item * pl.kmax_mut * slot);
-    pl.off_pj = o; o = align_up(o + (size_t)pj * pl.kmax_mut * slot);
-    if (pl.msys.size() > 1) { pl.off_mtable = o; o = align_up(o + pl.msys.size() * sizeof(MutSys)); }
-    // the source-side slots grow as N^2: the automatic choice keeps them
-    // within kMutAutoBytes and uses the ordered kernel beyond
-    if (sym == 0 && o > kMutAutoBytes) {
+    if (!fits) {
       pl.path = kOrderedPath;
       pl.msys.clear();
       o = 0;
@@ -1769,12 +1802,8 @@ static void* scratch_address()
 static Plan plan_within(int mask, int prec, int64_t n, int k, const rmw_tuning* tuning, size_t cap, bool periodic)
 {
   const int64_t off[2] = {0, n};
-  Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic);
+  Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, cap);
   if (pl.total <= cap) return pl;
-  if (pl.path == kBlocksPath) {   // the tile kernel writes fewer partial sums
-    pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, false);
-    if (pl.total <= cap) return pl;
-  }
   const bool sym_required = tuning && tuning->symmetric > 0;
   if (!sym_required) {
     const int OC = 3 * (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0));
