@@ -90,12 +90,25 @@ RMW_HD double rcp(double x) { return 1.0 / x; }
 RMW_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 RMW_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// The smaller of x and a constant; a NaN x gives the constant.  Blobs at one
-// point and non-finite positions (|d| = NaN) must still give non-finite
-// results: every coefficient keeps a factor of 1/|d| or a term in |d| that is
-// not clamped.
+// The smaller of x and a constant; a NaN x gives the constant.
 RMW_HD float min_(float x, float c) { return __builtin_fminf(x, c); }
 RMW_HD double min_(double x, double c) { return __builtin_fmin(x, c); }
+
+// min(|d|, 2).  Blobs at one point and non-finite positions (|d| = NaN) must give
+// non-finite results in every block: FP32 keeps the NaN here (gfx950 has such a
+// minimum, at the price of the other), FP64 adds it where no other factor has it
+// (nan_of, an FMA; a minimum that keeps it would be a compare and selects).
+RMW_HD float clamp_2(float r)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_elementwise_minimum(r, 2.0f);
+#else
+  return r > 2.0f ? 2.0f : r;
+#endif
+}
+RMW_HD double clamp_2(double r) { return min_(r, 2.0); }
+RMW_HD float nan_of(float, float c) { return c; }
+RMW_HD double nan_of(double r, double c) { return __builtin_fma(0.0, r, c); }
 
 // ---------------------------------------------------------------------------
 // Shared geometry of one (target, source) pair.
@@ -129,7 +142,7 @@ RMW_HD Geom<T> make_geom(T dx, T dy, T dz, T zi, T zj)
   g.invr = rsq(g.r2);
   g.r = g.r2 * g.invr;
   g.ic = min_(g.invr, T(0.5));
-  g.rm = min_(g.r, T(2));
+  g.rm = clamp_2(g.r);
   T R2 = p2 + g.Rz * g.Rz;
   g.invR = rsq(R2);
   return g;
@@ -152,7 +165,7 @@ RMW_HD Geom<T> make_geom_on(T dx, T dy, T dz, T zi, T zj, bool on)
   g.invr = on ? ir : T(0);
   g.r = on ? g.r2 * ir : T(3);
   g.ic = min_(g.invr, T(0.5));
-  g.rm = min_(g.r, T(2));
+  g.rm = clamp_2(g.r);
   T R2 = p2 + g.Rz * g.Rz;
   const T iR = rsq(R2);
   g.invR = on ? iR : T(0);
@@ -293,9 +306,7 @@ template <typename T> struct CoefRot {
   T F4;   // F4
 };
 
-// RPY: c = 1/r^3 far, (1 - 3r/8)/2 overlapping: ic^3 + (3/8 - 3 rm/16).  The
-// term 0 r is NaN where r is (no other factor here is), and costs the FMA that
-// adds it (a clamp that keeps a NaN: a compare and a select).
+// RPY: c = 1/r^3 far, (1 - 3r/8)/2 overlapping: ic^3 + (3/8 - 3 rm/16).
 // Wall, for h = h_hat R_z, with q = 1/|R|, w = q^2, b = R_z w:
 //   F1 = w,  F4 = -2 w q (h - b),  F3 = -2 w q B,  F2 = 2 w^2 (1 + 2 R_z B),
 //   B = 3 h - 5 b   (h_hat e_z^2 = h b and h_hat e_z = h q: no division).
@@ -303,7 +314,7 @@ template <typename T>
 RMW_HD CoefRot<T> coef_rot(const Geom<T>& g, T hnum, int dom = kDomWall)
 {
   CoefRot<T> c;
-  c.c = fma_(g.ic * g.ic, g.ic, fma_(T(-0.1875), g.rm, fma_(T(0), g.r, T(0.375))));
+  c.c = fma_(g.ic * g.ic, g.ic, fma_(T(-0.1875), g.rm, nan_of(g.r, T(0.375))));
   if (!dom_has_wall(dom)) {
     c.F1r = T(0); c.F2r = T(0); c.F3r2 = T(0); c.F4 = T(0);
     return c;
