@@ -89,6 +89,8 @@ int rmw_wall_rpy_workspace_size(int mask, int prec, int64_t n, int k,
  * or NULL when no block of the mask reads them; velocity/omega likewise
  * (same ld), or NULL when no block writes them.  L[3] are the
  * pseudo-periodic lengths (host array; NULL or entries <= 0 = unbounded).
+ * An output may lie over an input: it is then written to the workspace and
+ * copied when all right-hand sides are done.
  *
  * With tuning->flags & RMW_FLAG_CHECK_FINITE the outputs are scanned and a
  * non-finite entry returns RMW_E_NOTFINITE (the outputs are still written).
@@ -120,7 +122,8 @@ int rmw_wall_rpy_apply(int mask, int prec, const double* r_vectors, const double
  * or the ordered kernel with longer source chunks (and fewer right-hand
  * sides per pass) run so that it fits; sizes for which even
  * that does not fit (about 2.7 million blobs per right-hand side and
- * output block) return RMW_E_LIMIT before any launch.  Every call on one
+ * output block, fewer where the outputs of a call in place need room beside
+ * the sums) return RMW_E_LIMIT before any launch.  Every call on one
  * device shares that device's array: calls that overlap in time on one
  * device (two streams, two threads) race and must be serialised by the
  * caller.  Pair-kernel timing records (rmw_profile_enable) are not taken.

@@ -202,7 +202,7 @@ static bool shaped(const rmw_tuning* t)
 struct RadiiPlan {
   bool direct = false;
   int64_t chunk_len = 0, n_chunks = 0, n_tt = 0, total_items = 0;
-  size_t bytes = 0;
+  size_t off_stage = 0, bytes = 0;   // off_stage: the output of a product in place
 };
 
 static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* tuning,
@@ -218,7 +218,7 @@ static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* 
       nt <= kRDirectTargets * ns) {
     pl.direct = true;
     pl.total_items = (nt + kRDT - 1) / kRDT;
-    pl.bytes = align_up((size_t)nt * 3 * sizeof(double));   // the output of a product in place
+    pl.bytes = align_up((size_t)nt * 3 * sizeof(double));
     return pl;
   }
   int64_t chunk = tuning && tuning->chunk_len > 0 ? tuning->chunk_len : 0;
@@ -232,7 +232,8 @@ static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* 
   pl.chunk_len = chunk;
   pl.n_chunks = ns > 0 ? (ns + chunk - 1) / chunk : 0;
   pl.total_items = pl.n_tt * pl.n_chunks;
-  pl.bytes = align_up((size_t)pl.n_chunks * nt * 3 * sizeof(double));
+  pl.off_stage = align_up((size_t)pl.n_chunks * nt * 3 * sizeof(double));
+  pl.bytes = pl.off_stage + align_up((size_t)nt * 3 * sizeof(double));
   return pl;
 }
 
@@ -623,7 +624,7 @@ constexpr size_t kRMutAutoBytes = size_t(2) << 30;
 struct RadiiSelfPlan {
   bool mutual = false, blocks = false;
   int64_t n_t = 0, chunk_tiles = 0, total_items = 0;
-  size_t off_pj = 0, bytes = 0;
+  size_t off_pj = 0, off_stage = 0, bytes = 0;
   RadiiPlan ordered;
 };
 
@@ -651,8 +652,9 @@ static RadiiSelfPlan radii_self_plan(int prec, int64_t n, bool periodic, const r
       pl.chunk_tiles = std::max<int64_t>(1, tile_pairs / (16 * (int64_t)cu));
     pl.total_items = items_before(pl.n_t, pl.n_t, pl.chunk_tiles);
     pl.off_pj = align_up((size_t)pl.total_items * bs * 3 * sizeof(double));
-    pl.bytes = pl.off_pj + align_up((size_t)tile_pairs * bs * 3 * sizeof(double));
-    if (sym == 0 && pl.bytes > kRMutAutoBytes) pl.mutual = false;
+    pl.off_stage = pl.off_pj + align_up((size_t)tile_pairs * bs * 3 * sizeof(double));
+    pl.bytes = pl.off_stage + align_up((size_t)n * 3 * sizeof(double));
+    if (sym == 0 && pl.off_stage > kRMutAutoBytes) pl.mutual = false;
   }
   if (!pl.mutual) pl.bytes = pl.ordered.bytes;
   return pl;
@@ -735,11 +737,13 @@ static void radii_ordered(const RadiiPlan& pl, int prec, int bnd, const double* 
   ProfRec rec{};
   bool prof = false;
   prof_begin(rec, prof, st, 1);
+  // in place: the launch that writes the output reads inputs of blobs that other
+  // workgroups write (the reduce heights and radii), so it goes to the workspace
+  auto over = [&](const double* in, int64_t len) { return overlap(velocity, 3 * nt, in, len); };
+  const bool in_place = over(source, 3 * ns) || over(target, 3 * nt) || over(force, 3 * ns) ||
+                        over(radius_source, ns) || over(radius_target, nt);
+  double* const out = in_place ? (double*)((char*)workspace + pl.off_stage) : velocity;
   if (pl.direct) {
-    auto over = [&](const double* in, int64_t len) { return overlap(velocity, 3 * nt, in, len); };
-    const bool in_place = over(source, 3 * ns) || over(target, 3 * nt) || over(force, 3 * ns) ||
-                          over(radius_source, ns) || over(radius_target, nt);
-    double* const out = in_place ? (double*)workspace : velocity;
     if (bnd == kRadiiWall) launch_radii_direct<kRadiiWall>(prec, g, b, st, q, out);
     else if (bnd == kRadiiFreeSurface) launch_radii_direct<kRadiiFreeSurface>(prec, g, b, st, q, out);
     else launch_radii_direct<kRadiiUnbounded>(prec, g, b, st, q, out);
@@ -754,8 +758,9 @@ static void radii_ordered(const RadiiPlan& pl, int prec, int bnd, const double* 
   RMW_CHECK_HIP(hipGetLastError());
   prof_end(rec, prof, st);
   hipLaunchKernelGGL(radii_reduce_kernel, dim3((unsigned)((nt * 3 + 255) / 256)), dim3(256), 0, st, q.partial,
-                     pl.n_chunks, nt, target, radius_target, q.bnd, velocity);
+                     pl.n_chunks, nt, target, radius_target, q.bnd, out);
   RMW_CHECK_HIP(hipGetLastError());
+  if (in_place) launch_copy_rows(out, 3 * nt, velocity, 3 * nt, 3 * nt, 1, st);
 }
 
 static bool any_periodic(const double* L)
@@ -854,13 +859,17 @@ extern "C" int rmw_radii_self_apply(int prec, int boundary, const double* r, con
     else launch_radii_mutual<kRadiiUnbounded>(prec, g, b, st, q);
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
+    // the reduce reads heights and radii of blobs that other workgroups write
+    const bool in_place = overlap(velocity, 3 * n, r, 3 * n) || overlap(velocity, 3 * n, radius, n);
+    double* const out = in_place ? (double*)((char*)workspace + pl.off_stage) : velocity;
     const dim3 rg((unsigned)((n * 3 + kRRedOut - 1) / kRRedOut));
     if (pl.blocks)
       hipLaunchKernelGGL(radii_mutual_reduce_kernel<kRB>, rg, dim3(256), 0, st, q.part_i, q.part_j, r, radius, q.bnd, n,
-                         pl.n_t, pl.chunk_tiles, velocity);
+                         pl.n_t, pl.chunk_tiles, out);
     else
       hipLaunchKernelGGL(radii_mutual_reduce_kernel<kRBlock>, rg, dim3(256), 0, st, q.part_i, q.part_j, r, radius, q.bnd,
-                         n, pl.n_t, pl.chunk_tiles, velocity);
+                         n, pl.n_t, pl.chunk_tiles, out);
     RMW_CHECK_HIP(hipGetLastError());
+    if (in_place) launch_copy_rows(out, 3 * n, velocity, 3 * n, 3 * n, 1, st);
   });
 }

@@ -118,11 +118,9 @@ __global__ __launch_bounds__(kBlock) void direct_kernel(DirectParams p)
 #pragma unroll
       for (int m = 8; m >= 1; m >>= 1) s += __shfl_xor(s, m, 16);
       const int q = o / (K * OC), k = (o / OC) % K, c = o % OC;
-      if (sub == 0 && t0 + q < S.n) {
-        const int64_t dk = k * (p.out_stride - p.rhs_stride);   // finish_output counts in rhs_stride
-        finish_output(p.r, p.f, p.t, p.vel ? p.vel + dk : nullptr, p.omg ? p.omg + dk : nullptr, MASK, k,
-                      S.b0 + t0 + q, c, s, p.rhs_stride, p.a, p.inva, p.c1, p.c2, DOM);
-      }
+      if (sub == 0 && t0 + q < S.n)
+        finish_output(p.r, p.f, p.t, p.vel, p.omg, MASK, k, S.b0 + t0 + q, c, s, p.rhs_stride, p.out_stride, p.a,
+                      p.inva, p.c1, p.c2, DOM);
     }
   }
 }

@@ -323,9 +323,9 @@ __device__ __forceinline__ void mutual_apply(R dx, R dy, R dz, R zi, R zj, bool 
 __device__ __forceinline__ void finish_output(const double* __restrict__ r, const double* __restrict__ f,
                                               const double* __restrict__ t, double* __restrict__ vel,
                                               double* __restrict__ omg, int mask, int k, int64_t gi, int c,
-                                              double sum, int64_t rhs_stride, double a, double inva, double c1,
-                                              double c2, int dom, int periodic = 0, double L0 = 0.0,
-                                              double L1 = 0.0, double L2 = 0.0)
+                                              double sum, int64_t rhs_stride, int64_t out_stride, double a,
+                                              double inva, double c1, double c2, int dom, int periodic = 0,
+                                              double L0 = 0.0, double L1 = 0.0, double L2 = 0.0)
 {
   const bool HU = (mask & (kUF | kUT)) != 0;
   const bool HW = (mask & (kWF | kWT)) != 0;
@@ -379,11 +379,11 @@ __device__ __forceinline__ void finish_output(const double* __restrict__ r, cons
   if (!is_w) {
     if (mask & kUF) { Vec3<double> sv = self_uf_dom(dom, h, fv[0], fv[1], fv[2]); self += comp == 0 ? sv.x : (comp == 1 ? sv.y : sv.z); }
     if (mask & kUT) { Vec3<double> sv = self_ut_dom(dom, h, tv[0], tv[1], tv[2]); self += comp == 0 ? sv.x : (comp == 1 ? sv.y : sv.z); }
-    vel[k * rhs_stride + 3 * gi + comp] = (comp == 2 ? pz : 1.0) * B * (sum + self);
+    vel[k * out_stride + 3 * gi + comp] = (comp == 2 ? pz : 1.0) * B * (sum + self);
   } else {
     if (mask & kWF) { Vec3<double> sv = self_wf_dom(dom, h, fv[0], fv[1], fv[2]); self += comp == 0 ? sv.x : (comp == 1 ? sv.y : sv.z); }
     if (mask & kWT) { Vec3<double> sv = self_wt_dom(dom, h, tv[0], tv[1], tv[2]); self += comp == 0 ? sv.x : (comp == 1 ? sv.y : sv.z); }
-    omg[k * rhs_stride + 3 * gi + comp] = B * inva * (sum + self);
+    omg[k * out_stride + 3 * gi + comp] = B * inva * (sum + self);
   }
 }
 

@@ -628,7 +628,7 @@ struct ReduceParams {
   int mask;
   int K;
   int64_t ntot;
-  int64_t rhs_stride;  // doubles between RHS in f/t/vel/omg
+  int64_t rhs_stride, out_stride;  // doubles between RHS in f/t, in vel/omg
   double a, inva, c1, c2;
   int domain;
 };
@@ -672,8 +672,8 @@ __global__ __launch_bounds__(256) void reduce_kernel(ReduceParams p)
   for (; ch < S.n_chunks; ++ch) s0 += P[ch * cstride];
   double sum = (s0 + s1) + (s2 + s3);
 
-  finish_output(p.r, p.f, p.t, p.vel, p.omg, p.mask, k, gi, c, sum, p.rhs_stride, p.a, p.inva, p.c1, p.c2,
-                p.domain);
+  finish_output(p.r, p.f, p.t, p.vel, p.omg, p.mask, k, gi, c, sum, p.rhs_stride, p.out_stride, p.a, p.inva,
+                p.c1, p.c2, p.domain);
 }
 
 // Reduce of the symmetric path: for blob gi of tile X of its system, the
@@ -693,7 +693,7 @@ struct MutReduceParams {
   int mask;
   int K;
   int64_t chunk_blocks;
-  int64_t rhs_stride;
+  int64_t rhs_stride, out_stride;
   double a, inva, c1, c2;
   int domain;
   int periodic;             // bit d set when L_d > 0: add the self pair's outer images
@@ -773,8 +773,8 @@ __global__ __launch_bounds__(256) void mutual_reduce_kernel(MutReduceParams p)
     double s = part[0][ol];
 #pragma unroll
     for (int q = 1; q < kRedGroups; ++q) s += part[q][ol];
-    finish_output(p.r, p.f, p.t, p.vel, p.omg, p.mask, k, gi, c, s, p.rhs_stride, p.a, p.inva, p.c1, p.c2,
-                  p.domain, PER ? p.periodic : 0, p.L[0], p.L[1], p.L[2]);
+    finish_output(p.r, p.f, p.t, p.vel, p.omg, p.mask, k, gi, c, s, p.rhs_stride, p.out_stride, p.a, p.inva,
+                  p.c1, p.c2, p.domain, PER ? p.periodic : 0, p.L[0], p.L[1], p.L[2]);
   }
 }
 
@@ -791,8 +791,9 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(const double* __restrict
 void launch_copy_rows(const double* src, int64_t src_stride, double* dst, int64_t dst_stride, int64_t len, int K,
                       hipStream_t st)
 {
-  hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)((len + 255) / 256), K), dim3(256), 0, st, src, src_stride, dst,
-                     dst_stride, len);
+  for (int k = 0; k < K; k += 65535)
+    hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)((len + 255) / 256), std::min(K - k, 65535)), dim3(256), 0, st,
+                       src + k * src_stride, src_stride, dst + k * dst_stride, dst_stride, len);
   RMW_CHECK_HIP(hipGetLastError());
 }
 
@@ -875,7 +876,9 @@ struct Plan {
   int kmax_direct = 1;
   SmallVec<DirectSys> dsys;  // non-empty systems only
   int64_t direct_wgs = 0;
-  size_t off_dtable = 0, off_stage = 0;   // off_stage: outputs of a product in place
+  size_t off_dtable = 0;
+  // outputs of a product in place: all right-hand sides of the call
+  size_t off_stage = 0, stage_bytes = 0;
   // RMW_FLAG_CHECK_FINITE: a counter of non-finite outputs after the rest
   bool check_finite = false;
   size_t off_status = 0;
@@ -1013,12 +1016,12 @@ static SmallVec<DirectSys> direct_table(const int64_t* offsets, int nsys, int tt
 
 // offsets: host array of nsys + 1 blob offsets (offsets[0] = 0).  periodic:
 // the call has pseudo-periodic images (the symmetric wall kernels then take
-// one right-hand side per pass, so their partial sums are sized for one).  cap:
-// bytes that the partial sums of an automatically chosen symmetric layout may
-// take.
+// one right-hand side per pass, so their partial sums are sized for one).
+// stage: room for the outputs of a product in place.  cap: bytes that the
+// partial sums of an automatically chosen symmetric layout may take.
 static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int k,
                       const rmw_tuning* tuning, bool ragged, int domain = kDomWall, bool periodic = false,
-                      size_t cap = kMutAutoBytes)
+                      bool stage = true, size_t cap = kMutAutoBytes)
 {
   RMW_REQUIRE(valid_mask(mask), "mask must be a non-empty subset of UF|UT|WF|WT");
   RMW_REQUIRE(domain >= kDomWall && domain <= kDomFreeSurface, "unknown domain");
@@ -1153,7 +1156,6 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
                                      : 4 * std::max<int64_t>(1, tile_pairs / (48 * (int64_t)cu))};
       layouts[count++] = {false, 4 * std::max<int64_t>(1, tile_pairs / (16 * (int64_t)cu))};
     }
-    const int OCm = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
     bool fits = false;
     for (int q = 0; !fits; ++q) {
       if (q == count) {   // no layout: two right-hand sides per pass, or a required one beyond the limit
@@ -1185,7 +1187,7 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
         pj += M.n_t * (M.n_t + 1) / 2;
         pl.msys.push_back(M);
       }
-      const size_t slot = (size_t)pl.kmax_mut * bs * OCm * sizeof(double);
+      const size_t slot = (size_t)pl.kmax_mut * bs * OC * sizeof(double);
       o = 0;
       pl.off_pi = o; o = align_up(o + (size_t)item * slot);
       pl.off_pj = o; o = align_up(o + (size_t)pj * slot);
@@ -1206,13 +1208,15 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
     pl.kmax_direct = group_k(k, std::min(direct_max_k(mask, domain), rhs_cap(tuning) > 0 ? rhs_cap(tuning) : 4));
     pl.dsys = direct_table(offsets, nsys, direct_targets(mask, pl.kmax_direct), pl.direct_wgs);
     if (pl.dsys.size() > 1) { pl.off_dtable = o; o = align_up(o + pl.dsys.size() * sizeof(DirectSys)); }
-    pl.off_stage = o;
-    o = align_up(o + (size_t)pl.kmax_direct * 3 * pl.ntot * sizeof(double) *
-                         (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0)));
   }
   if (pl.path == kOrderedPath) {
     pl.off_partial = o; o = align_up(o + pl.partial_doubles * sizeof(double));
     if (ragged) { pl.off_table = o; o = align_up(o + pl.sys.size() * sizeof(SysInfo)); }
+  }
+  if (stage) {
+    pl.off_stage = o;
+    pl.stage_bytes = align_up((size_t)k * pl.ntot * OC * sizeof(double));
+    o += pl.stage_bytes;
   }
   pl.total = o;
   pl.check_finite = tuning && (tuning->flags & RMW_FLAG_CHECK_FINITE) != 0;
@@ -1478,8 +1482,9 @@ void prof_end(const ProfRec& rec, bool on, hipStream_t st)
 }
 
 static void run_mutual(const Plan& pl, const double* r, const double* f, const double* t, double* vel,
-                       double* omg, int k, int64_t stride, double a, double inva, double c1, double c2,
-                       const rmw_tuning* tuning, char* base, hipStream_t st, int periodic, const double* Lp)
+                       double* omg, int k, int64_t stride, int64_t out_stride, double a, double inva, double c1,
+                       double c2, const rmw_tuning* tuning, char* base, hipStream_t st, int periodic,
+                       const double* Lp)
 {
   const bool HU = (pl.mask & (kUF | kUT)) != 0, HW = (pl.mask & (kWF | kWT)) != 0;
   const bool NF = (pl.mask & (kUF | kWF)) != 0, NT = (pl.mask & (kUT | kWT)) != 0;
@@ -1520,8 +1525,8 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     MutReduceParams rp{};
     rp.r = r;
     rp.f = q.f; rp.t = q.t;
-    rp.vel = HU ? vel + (size_t)k0 * stride : nullptr;
-    rp.omg = HW ? omg + (size_t)k0 * stride : nullptr;
+    rp.vel = HU ? vel + (size_t)k0 * out_stride : nullptr;
+    rp.omg = HW ? omg + (size_t)k0 * out_stride : nullptr;
     rp.part_i = q.part_i;
     rp.part_j = q.part_j;
     rp.table = dtable;
@@ -1531,6 +1536,7 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
     rp.K = K;
     rp.chunk_blocks = pl.chunk_blocks;
     rp.rhs_stride = stride;
+    rp.out_stride = out_stride;
     rp.a = a; rp.inva = inva; rp.c1 = c1; rp.c2 = c2;
     rp.domain = pl.domain;
     rp.periodic = periodic;
@@ -1551,8 +1557,8 @@ static void run_mutual(const Plan& pl, const double* r, const double* f, const d
 }
 
 static void run_direct(const Plan& pl, const double* r, const double* f, const double* t, double* vel, double* omg,
-                       int k, int64_t stride, double a, double inva, double c1, double c2, char* base, hipStream_t st,
-                       int periodic, const double* Lp)
+                       int k, int64_t stride, int64_t out_stride, double a, double inva, double c1, double c2,
+                       char* base, hipStream_t st, int periodic, const double* Lp)
 {
   SmallVec<DirectSys> table = pl.dsys;
   int64_t wgs = pl.direct_wgs;
@@ -1582,10 +1588,10 @@ static void run_direct(const Plan& pl, const double* r, const double* f, const d
     q.r = r;
     q.f = f ? f + (size_t)k0 * stride : nullptr;
     q.t = t ? t + (size_t)k0 * stride : nullptr;
-    q.vel = vel ? vel + (size_t)k0 * stride : nullptr;
-    q.omg = omg ? omg + (size_t)k0 * stride : nullptr;
+    q.vel = vel ? vel + (size_t)k0 * out_stride : nullptr;
+    q.omg = omg ? omg + (size_t)k0 * out_stride : nullptr;
     q.rhs_stride = stride;
-    q.out_stride = stride;
+    q.out_stride = out_stride;
     q.a = a; q.inva = inva; q.c1 = c1; q.c2 = c2;
     q.table = dtable;
     q.single = table[0];
@@ -1595,26 +1601,79 @@ static void run_direct(const Plan& pl, const double* r, const double* f, const d
     ProfRec rec{};
     bool prof = false;
     prof_begin(rec, prof, st);
-    // outputs over an input (a product in place): by way of the workspace
-    const int64_t len = 3 * pl.ntot, span = (K - 1) * stride + len;
-    auto over_input = [&](const double* out) {
-      return overlap(out, span, r, len) || overlap(out, span, q.f, span) || overlap(out, span, q.t, span);
-    };
-    double *const vel_k = q.vel, *const omg_k = q.omg;
-    const bool staged = over_input(vel_k) || over_input(omg_k);
-    if (staged) {
-      double* stage = (double*)(base + pl.off_stage);
-      q.out_stride = len;
-      if (vel_k) { q.vel = stage; stage += K * len; }
-      if (omg_k) q.omg = stage;
-    }
     launch_direct(pl.domain, pl.mask, pl.prec, K, q, wgs, st);
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
-    if (staged) {
-      if (vel_k) launch_copy_rows(q.vel, len, vel_k, stride, len, K, st);
-      if (omg_k) launch_copy_rows(q.omg, len, omg_k, stride, len, K, st);
-    }
+  }
+}
+
+static void run_ordered(const Plan& pl, const double* r, const double* f, const double* t, double* vel, double* omg,
+                        int k, int64_t stride, int64_t out_stride, double a, double inva, double c1, double c2,
+                        const rmw_tuning* tuning, char* base, hipStream_t st, int periodic, const double* Lp,
+                        bool ragged)
+{
+  const bool HU = (pl.mask & (kUF | kUT)) != 0, HW = (pl.mask & (kWF | kWT)) != 0;
+  const bool NF = (pl.mask & (kUF | kWF)) != 0, NT = (pl.mask & (kUT | kWT)) != 0;
+  SysInfo* dtable = nullptr;
+  if (ragged) {
+    dtable = (SysInfo*)(base + pl.off_table);
+    stage_upload(dtable, pl.sys.data(), pl.sys.size() * sizeof(SysInfo), st);
+  }
+
+  int grid = (int)std::min<int64_t>(pl.total_items, (int64_t)INT32_MAX);
+  if (ragged || (tuning && tuning->max_wgs > 0)) {
+    const int cap = tuning && tuning->max_wgs > 0 ? tuning->max_wgs : std::max(pl.slots, 1);
+    grid = (int)std::min<int64_t>(grid, cap);
+  }
+
+  const int kcap = pl.domain == kDomWall ? rhs_cap(tuning) : 1;
+  for (int k0 = 0, K = group_k(k, kcap); k0 < k; k0 += K) {
+    K = group_k(k - k0, kcap);
+    PairParams q{};
+    q.r = r;
+    q.f = NF ? f + (size_t)k0 * stride : nullptr;
+    q.t = NT ? t + (size_t)k0 * stride : nullptr;
+    q.rhs_stride = stride;
+    q.a = a; q.inva = inva; q.c1 = c1; q.c2 = c2;
+    q.partial = (double*)(base + pl.off_partial);
+    q.table = dtable;
+    q.single = pl.sys.empty() ? SysInfo{} : pl.sys[0];
+    q.nsys = (int)pl.sys.size();
+    q.ntot = pl.ntot;
+    q.total_items = pl.total_items;
+    q.periodic = periodic;
+    for (int d = 0; d < 3; ++d) { q.L[d] = Lp[d]; q.iL[d] = Lp[d] > 0.0 ? 1.0 / Lp[d] : 0.0; }
+    q.domain = pl.domain;
+    // The partial layout was planned for kmax RHS; a smaller trailing group
+    // reuses it with its own K (items only touch their own slots).
+    ProfRec rec{};
+    bool prof = false;
+    prof_begin(rec, prof, st);
+    if (pl.domain == kDomWall) dispatch_pair(pl.mask, pl.prec, K, q, grid, st);
+    else dispatch_pair_domain(pl.domain, pl.mask, pl.prec, q, grid, st);
+    RMW_CHECK_HIP(hipGetLastError());
+    prof_end(rec, prof, st);
+
+    ReduceParams rp{};
+    rp.r = r;
+    rp.f = q.f; rp.t = q.t;
+    rp.vel = HU ? vel + (size_t)k0 * out_stride : nullptr;
+    rp.omg = HW ? omg + (size_t)k0 * out_stride : nullptr;
+    rp.partial = q.partial;
+    rp.table = dtable;
+    rp.single = q.single;
+    rp.nsys = q.nsys;
+    rp.mask = pl.mask;
+    rp.K = K;
+    rp.ntot = pl.ntot;
+    rp.rhs_stride = stride;
+    rp.out_stride = out_stride;
+    rp.a = a; rp.inva = inva; rp.c1 = c1; rp.c2 = c2;
+    rp.domain = pl.domain;
+    const int OCr = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
+    const int64_t nthreads = pl.ntot * K * OCr;
+    hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((nthreads + 255) / 256)), dim3(256), 0, st, rp);
+    RMW_CHECK_HIP(hipGetLastError());
   }
 }
 
@@ -1641,6 +1700,18 @@ static void check_outputs(const Plan& pl, const double* vel, const double* omg, 
   if (bad)
     throw Error(RMW_E_NOTFINITE, std::to_string(bad) + " output entries are inf or NaN (coincident distinct "
                                                        "blobs or non-finite inputs)");
+}
+
+// Does an output of the product lie over one of its inputs?
+static bool in_place(int mask, int64_t ntot, int k, int64_t stride, const double* r, const double* f, const double* t,
+                     const double* vel, const double* omg)
+{
+  const int64_t len = 3 * ntot, span = (k - 1) * stride + len;
+  auto over = [&](const double* out) {
+    return overlap(out, span, r, len) || ((mask & (kUF | kWF)) && overlap(out, span, f, span)) ||
+           ((mask & (kUT | kWT)) && overlap(out, span, t, span));
+  };
+  return ((mask & (kUF | kUT)) && over(vel)) || ((mask & (kWF | kWT)) && over(omg));
 }
 
 static bool has_images(const double* L)
@@ -1692,80 +1763,32 @@ static void run_plan(const Plan& pl, const double* r, const double* f, const dou
   const double c2 = c1 / a;
 
   const int64_t stride = ld > 0 ? ld : 3 * pl.ntot;
-  if (pl.path == kDirectPath) {
-    run_direct(pl, r, NF ? f : nullptr, NT ? t : nullptr, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, a, inva, c1,
-               c2, base, st, periodic, Lp);
-    check_outputs(pl, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, base, st);
-    return;
+  // A product in place (an output over an input): every launch that writes
+  // outputs reads inputs of blobs that other workgroups write, so the outputs
+  // go to the workspace and are copied when all right-hand sides are done.
+  const bool staged = in_place(pl.mask, pl.ntot, k, stride, r, f, t, vel, omg);
+  const int64_t len = 3 * pl.ntot, out_stride = staged ? len : stride;
+  double *out_u = vel, *out_w = omg;
+  if (staged) {
+    RMW_REQUIRE(pl.stage_bytes > 0, "no room for the outputs of a product in place");
+    out_u = (double*)(base + pl.off_stage);
+    out_w = out_u + (HU ? k * len : 0);
   }
-  if (pl.path != kOrderedPath) {
-    run_mutual(pl, r, f, t, vel, omg, k, stride, a, inva, c1, c2, tuning, base, st, periodic, Lp);
-    check_outputs(pl, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, base, st);
-    return;
-  }
-
-  SysInfo* dtable = nullptr;
-  if (ragged) {
-    dtable = (SysInfo*)(base + pl.off_table);
-    stage_upload(dtable, pl.sys.data(), pl.sys.size() * sizeof(SysInfo), st);
-  }
-
-  int grid = (int)std::min<int64_t>(pl.total_items, (int64_t)INT32_MAX);
-  if (ragged || (tuning && tuning->max_wgs > 0)) {
-    const int cap = tuning && tuning->max_wgs > 0 ? tuning->max_wgs : std::max(pl.slots, 1);
-    grid = (int)std::min<int64_t>(grid, cap);
-  }
-
-  const int kcap = pl.domain == kDomWall ? rhs_cap(tuning) : 1;
-  for (int k0 = 0, K = group_k(k, kcap); k0 < k; k0 += K) {
-    K = group_k(k - k0, kcap);
-    PairParams q{};
-    q.r = r;
-    q.f = NF ? f + (size_t)k0 * stride : nullptr;
-    q.t = NT ? t + (size_t)k0 * stride : nullptr;
-    q.rhs_stride = stride;
-    q.a = a; q.inva = inva; q.c1 = c1; q.c2 = c2;
-    q.partial = (double*)(base + pl.off_partial);
-    q.table = dtable;
-    q.single = pl.sys.empty() ? SysInfo{} : pl.sys[0];
-    q.nsys = (int)pl.sys.size();
-    q.ntot = pl.ntot;
-    q.total_items = pl.total_items;
-    q.periodic = periodic;
-    for (int d = 0; d < 3; ++d) { q.L[d] = Lp[d]; q.iL[d] = Lp[d] > 0.0 ? 1.0 / Lp[d] : 0.0; }
-    q.domain = pl.domain;
-    // The partial layout was planned for kmax RHS; a smaller trailing group
-    // reuses it with its own K (items only touch their own slots).
-    ProfRec rec{};
-    bool prof = false;
-    prof_begin(rec, prof, st);
-    if (pl.domain == kDomWall) dispatch_pair(kmask, pl.prec, K, q, grid, st);
-    else dispatch_pair_domain(pl.domain, kmask, pl.prec, q, grid, st);
-    RMW_CHECK_HIP(hipGetLastError());
-    prof_end(rec, prof, st);
-
-    ReduceParams rp{};
-    rp.r = r;
-    rp.f = q.f; rp.t = q.t;
-    rp.vel = HU ? vel + (size_t)k0 * stride : nullptr;
-    rp.omg = HW ? omg + (size_t)k0 * stride : nullptr;
-    rp.partial = q.partial;
-    rp.table = dtable;
-    rp.single = q.single;
-    rp.nsys = q.nsys;
-    rp.mask = pl.mask;
-    rp.K = K;
-    rp.ntot = pl.ntot;
-    rp.rhs_stride = stride;
-    rp.a = a; rp.inva = inva; rp.c1 = c1; rp.c2 = c2;
-    rp.domain = pl.domain;
-    const int OCr = 3 * ((HU ? 1 : 0) + (HW ? 1 : 0));
-    const int64_t nthreads = pl.ntot * K * OCr;
-    hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)((nthreads + 255) / 256)), dim3(256), 0, st, rp);
-    RMW_CHECK_HIP(hipGetLastError());
+  if (pl.path == kDirectPath)
+    run_direct(pl, r, NF ? f : nullptr, NT ? t : nullptr, HU ? out_u : nullptr, HW ? out_w : nullptr, k, stride,
+               out_stride, a, inva, c1, c2, base, st, periodic, Lp);
+  else if (pl.path != kOrderedPath)
+    run_mutual(pl, r, f, t, out_u, out_w, k, stride, out_stride, a, inva, c1, c2, tuning, base, st, periodic, Lp);
+  else
+    run_ordered(pl, r, f, t, out_u, out_w, k, stride, out_stride, a, inva, c1, c2, tuning, base, st, periodic, Lp,
+                ragged);
+  if (staged) {
+    if (HU) launch_copy_rows(out_u, len, vel, stride, len, k, st);
+    if (HW) launch_copy_rows(out_w, len, omg, stride, len, k, st);
   }
   check_outputs(pl, HU ? vel : nullptr, HW ? omg : nullptr, k, stride, base, st);
 }
+
 
 // ---------------------------------------------------------------------------
 // No-allocation entry point: the partial sums live in a fixed device array
@@ -1794,31 +1817,34 @@ static void* scratch_address()
   return ptrs[dev];
 }
 
-// The plan of rmw_wall_rpy_apply for these sizes if its partial sums fit
-// in `cap` bytes; otherwise (unless the tuning requires the symmetric
+// The plan of rmw_wall_rpy_apply for these sizes if its partial sums (and, for
+// a product in place, its outputs: stage) fit in `cap` bytes; otherwise (unless the tuning requires the symmetric
 // kernel) the ordered kernel with source chunks as long as the fit needs,
 // and fewer right-hand sides per pass if one chunk of k_group is still too
 // large.  Throws RMW_E_LIMIT when nothing fits.
-static Plan plan_within(int mask, int prec, int64_t n, int k, const rmw_tuning* tuning, size_t cap, bool periodic)
+static Plan plan_within(int mask, int prec, int64_t n, int k, const rmw_tuning* tuning, size_t cap, bool periodic,
+                        bool stage)
 {
   const int64_t off[2] = {0, n};
-  Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, cap);
+  const int OC = 3 * (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0));
+  const size_t staged = stage ? align_up((size_t)k * n * OC * sizeof(double)) : 0;
+  const size_t sums = cap > staged ? cap - staged : 0;
+  Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, stage, sums);
   if (pl.total <= cap) return pl;
   const bool sym_required = tuning && tuning->symmetric > 0;
-  if (!sym_required) {
-    const int OC = 3 * (((mask & (kUF | kUT)) ? 1 : 0) + ((mask & (kWF | kWT)) ? 1 : 0));
+  if (!sym_required && sums > 256) {
     rmw_tuning t = tuning ? *tuning : rmw_tuning{};
     t.symmetric = -1;
     for (int g : {4, 2, 1}) {
       if (t.rhs_group != 0 && g > t.rhs_group) continue;
       const int kg = group_k(k, g);
       const double per_chunk = (double)kg * (double)n * OC * sizeof(double);
-      const int64_t chunks = (int64_t)std::floor((double)(cap - 256) / per_chunk);
+      const int64_t chunks = (int64_t)std::floor((double)(sums - 256) / per_chunk);
       if (chunks < 1) continue;
       const int64_t len = (n + chunks - 1) / chunks;
       t.chunk_len = std::max<int64_t>(t.chunk_len, (len + kChunkQuantum - 1) / kChunkQuantum * kChunkQuantum);
       t.rhs_group = kg;
-      Plan p2 = make_plan(mask, prec, off, 1, k, &t, false, kDomWall, periodic);
+      Plan p2 = make_plan(mask, prec, off, 1, k, &t, false, kDomWall, periodic, stage);
       if (p2.total <= cap) return p2;
     }
   }
@@ -1893,7 +1919,8 @@ extern "C" int rmw_wall_rpy_apply_noalloc(int mask, int prec, const double* r_ve
     RMW_REQUIRE(n >= 0, "n must be >= 0");
     RMW_REQUIRE(!(tuning && (tuning->flags & RMW_FLAG_CHECK_FINITE)),
                 "the finite check waits for the stream; use rmw_wall_rpy_apply for it");
-    Plan pl = plan_within(mask, prec, n, k, tuning, RMW_NOALLOC_SCRATCH_BYTES, has_images(L));
+    const bool stage = in_place(mask, n, k, ld > 0 ? ld : 3 * n, r_vectors, force, torque, velocity, omega);
+    Plan pl = plan_within(mask, prec, n, k, tuning, RMW_NOALLOC_SCRATCH_BYTES, has_images(L), stage);
     if (pl.ntot == 0) return;
     // the plan may differ from the caller's tuning (longer ordered chunks);
     // run_plan reads only max_wgs and rhs_group from it
