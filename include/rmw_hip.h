@@ -447,8 +447,6 @@ int rmw_rigid_block_apply(const int64_t* body_offsets, int nbodies, const double
                           const double* x, double* y, int k, int64_t ld, void* workspace, size_t workspace_bytes,
                           void* stream);
 
-/* y = P^-1 x, the body preconditioner apply of multi_bodies/multi_bodies.py:
- * 825-849 (x != y). */
 /* Velocity (nblobs, 3) at every blob induced by the net forces (first three
  * entries of each force_stride-long row of `force`) of all other bodies,
  * each body a sphere of radius `radius` at its centre, through the
@@ -462,6 +460,9 @@ int rmw_rigid_point_field(const double* r_blobs, const double* centres, const do
                           int64_t force_stride, const int64_t* body_offsets, int nbodies, double radius,
                           double a, double eta, int wall, double* velocity, void* workspace,
                           size_t workspace_bytes, void* stream);
+/* y = P^-1 x, the body preconditioner apply of multi_bodies/multi_bodies.py:
+ * 825-849.  x and y (3 nblobs + 6 nbodies entries) must not overlap
+ * (RMW_E_ARG). */
 int rmw_rigid_pc_apply(const int64_t* body_offsets, int nbodies, const double* minv,
                        const double* minvk, const double* nbody, const double* r_rel,
                        const double* x, double* y, void* workspace, size_t workspace_bytes,

@@ -263,12 +263,14 @@ __global__ void dense_mobility_kernel(int dom, const double* __restrict__ r, con
 }
 
 // ---------------------------------------------------------------------------
-// Symmetric 6x6 pseudo-inverse by Jacobi rotations, run by one whole wave:
-// lane 6 i + j holds element (i, j) of A and of the eigenvectors, and the
-// three disjoint rotations of a round (five rounds of a round robin make a
-// sweep) are applied together through lane exchanges.  By one thread, with
-// the matrices in scratch memory, this was most of the preconditioner build
-// (YY us of 256 for bodies of 42 blobs).  a6: the matrix in LDS, P: output.
+// Symmetric 6x6 pseudo-inverse, run by one whole wave: lane 6 i + j holds
+// element (i, j).  Ordinarily the matrix is regular and is inverted by
+// elimination: every pivot (a diagonal entry of a Schur complement) must exceed
+// 1e-8 of the largest diagonal entry.  Otherwise (K^T M^-1 K of a single blob or
+// of blobs on a line, of few blobs in large units) the eigenvalues are found by
+// Jacobi rotations, the three disjoint ones of a round (five rounds of a round
+// robin make a sweep) applied together through lane exchanges, and those
+// beyond numpy's cut-off inverted.  a6: the matrix in LDS, P: output.
 // ---------------------------------------------------------------------------
 __device__ void pinv6_wave(const double* a6, double* __restrict__ P)
 {
@@ -1234,7 +1236,9 @@ extern "C" int rmw_rigid_pc_apply(const int64_t* body_offsets, int nbodies, cons
   return guarded([&] {
     RigidLayout L = rigid_layout(body_offsets, nbodies);
     RMW_REQUIRE(workspace_bytes >= L.total, "workspace too small");
-    RMW_REQUIRE(x != y, "pc apply is out of place");
+    // several workgroups share a body: each reads all of its x while others write y
+    const int64_t size = 3 * L.nblobs + 6 * (int64_t)nbodies;
+    RMW_REQUIRE(!overlap(x, size, y, size), "pc apply is out of place: x and y must not overlap");
     hipStream_t st = (hipStream_t)stream;
     char* ws = (char*)workspace;
     const size_t lds = 2 * (size_t)L.max_n * sizeof(double);

@@ -55,6 +55,20 @@ def test_error_path_reports_without_gpu():
     assert rc == -1 and b"precision" in lib.rmw_last_error()
 
 
+def test_preconditioner_apply_refuses_overlapping_vectors():
+    """Several workgroups share a body, so x and y must not overlap, at one
+    address or shifted; the check comes before any launch."""
+    from rigidmultiblobswall_amd import _lib
+    lib = _lib.load()
+    off = np.array([0, 12, 17], dtype=np.int64)
+    offp = off.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
+    n = 3 * 17 + 6 * 2
+    base = 1 << 20
+    for shift in (0, 1, n - 1, 1 - n):
+        rc = lib.rmw_rigid_pc_apply(offp, 2, None, None, None, None, base, base + 8 * shift, None, 1 << 20, None)
+        assert rc == _lib.RMW_E_ARG and b"overlap" in lib.rmw_last_error()
+
+
 def _host_lib():
     path = os.path.join(REPO, "tests", "helpers", "libpair_terms_host.so")
     if not os.path.exists(path):
