@@ -76,6 +76,9 @@ __device__ __forceinline__ double root1(double g)
 // (lane i holds d_i and e_i), m <= 64: on return lane i holds eigenvalue i,
 // and Z (m x m in LDS, column-major, identity on entry) the eigenvectors, row
 // `lane` of which only this lane touches.  Returns 1 if it does not converge.
+// (With d and e in LDS, as tridiag_ql keeps them for larger m, the recurrence
+// waits for their reads: 11 steps 65 us instead of 53, 25 314 / 236, 64 1737 / 1265,
+// for a T with a negative eigenvalue.)
 __device__ int tridiag_ql_lanes(int m, double& d, double& e, double* __restrict__ Z)
 {
   const int lane = threadIdx.x;

@@ -697,9 +697,8 @@ RMW_HD Vec3<T> apply_radii(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, 
 }
 
 // M_ij^T v (the coefficients as computed for the ordered pair (i, j)).
-template <typename T, bool ADD = false>
-RMW_HD Vec3<T> apply_radii_t(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz,
-                             const Vec3<T>& acc = Vec3<T>{})
+template <typename T>
+RMW_HD Vec3<T> apply_radii_t(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx, T vy, T vz)
 {
   const T p = fma_(dx, vx, dy * vy);
   const T dv = fma_(dz, vz, p);
@@ -708,9 +707,9 @@ RMW_HD Vec3<T> apply_radii_t(T dx, T dy, T dz, T Rz, const CoefRadii<T>& c, T vx
   const T q = c.C2 * dv;
   const T k = c.C1 - c.al, e = q - h;
   Vec3<T> u;
-  u.x = fma_(k, vx, fma_or_mul<ADD>(e, dx, acc.x));
-  u.y = fma_(k, vy, fma_or_mul<ADD>(e, dy, acc.y));
-  u.z = fma_(c.C1 + c.al + c.de, vz, fma_(q, dz, fma_(h, Rz, fma_or_mul<ADD>(c.g1, Rv, acc.z))));
+  u.x = fma_(k, vx, e * dx);
+  u.y = fma_(k, vy, e * dy);
+  u.z = fma_(c.C1 + c.al + c.de, vz, fma_(q, dz, fma_(h, Rz, c.g1 * Rv)));
   return u;
 }
 
