@@ -868,6 +868,7 @@ struct Plan {
   size_t partial_doubles = 0;
   size_t off_partial = 0, off_table = 0, total = 0;
   // symmetric paths
+  bool over_cap = false;     // symmetric by its size, ordered because no layout fits
   int kmax_mut = 1;
   int64_t mut_items = 0, mut_tiles = 0, chunk_blocks = 4;   // symmetric work item: chunk_blocks 64-source blocks
   SmallVec<MutSys> msys;     // non-empty systems only
@@ -1199,6 +1200,7 @@ static Plan make_plan(int mask, int prec, const int64_t* offsets, int nsys, int 
       pl.mut_tiles = tiles;
     }
     if (!fits) {
+      pl.over_cap = true;
       pl.path = kOrderedPath;
       pl.msys.clear();
       o = 0;
@@ -1830,7 +1832,9 @@ static Plan plan_within(int mask, int prec, int64_t n, int k, const rmw_tuning* 
   const size_t staged = stage ? align_up((size_t)k * n * OC * sizeof(double)) : 0;
   const size_t sums = cap > staged ? cap - staged : 0;
   Plan pl = make_plan(mask, prec, off, 1, k, tuning, false, kDomWall, periodic, stage, sums);
-  if (pl.total <= cap) return pl;
+  // (an ordered kernel in the place of a symmetric one takes the chunks below,
+  // as short as the array allows: 40000 blobs 2.15 ms, 2.27 with its own)
+  if (pl.total <= cap && !pl.over_cap) return pl;
   const bool sym_required = tuning && tuning->symmetric > 0;
   if (!sym_required && sums > 256) {
     rmw_tuning t = tuning ? *tuning : rmw_tuning{};
