@@ -188,7 +188,9 @@ __global__ void radii_zero_kernel(double* __restrict__ out, int64_t n)
 //    64 / 128 / 192 / 256: 12000 x 400 59 / 67 / 87 / 108, 20000 x 2000
 //    140 / 125 / 140 / 145, 30000 x 1000 151 / 121 / 125 / 128, 45000 x 600
 //    186 / 150 / 135 / 158, 65536 x 64 182 / 126 / 129 / 136, 65536 x 700
-//    252 / 190 / 193 / 170, 1000000 x 5 2462 / 1510 / 1184 / 1031.
+//    252 / 190 / 193 / 170, 1000000 x 5 2462 / 1510 / 1184 / 1031.  With images,
+//    whose pairs take nine times as long, 64 sources up to 65536 of them (64 / 256:
+//    65536 x 64 407 / 616).
 constexpr int kRDT = 4;      // targets of a workgroup of the direct kernel
 constexpr double kRDirectPairs = 2304.0 * 2304.0, kRDirectSelf = 1600.0 * 1600.0;
 constexpr int64_t kRDirectSources = 8192, kRDirectTargets = 256;   // targets per source
@@ -205,7 +207,8 @@ struct RadiiPlan {
   size_t off_stage = 0, bytes = 0;   // off_stage: the output of a product in place
 };
 
-static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* tuning,
+// images: the call has periodic images, or (in a size query) may have.
+static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* tuning, bool images,
                             double direct_pairs = kRDirectPairs)
 {
   RMW_REQUIRE(prec == RMW_PREC_F32_F64ACC || prec == RMW_PREC_F32_KAHAN || prec == RMW_PREC_F64 ||
@@ -224,7 +227,8 @@ static RadiiPlan radii_plan(int prec, int64_t ns, int64_t nt, const rmw_tuning* 
   int64_t chunk = tuning && tuning->chunk_len > 0 ? tuning->chunk_len : 0;
   if (chunk <= 0) {
     const double c = (double)ns * (double)nt / (16.0 * std::max(device_props().cu_count, 1) * kRBlock);
-    const int64_t least = std::min<int64_t>(kRBlock, std::max<int64_t>(64, (ns / 256 + 63) / 64 * 64));
+    int64_t least = ns <= 65536 ? 64 : kRBlock;
+    if (!images) least = std::min<int64_t>(kRBlock, std::max<int64_t>(64, (ns / 256 + 63) / 64 * 64));
     chunk = std::max<int64_t>(least, (int64_t)std::ceil(c / 64.0) * 64);
   }
   chunk = std::max<int64_t>(64, (chunk + 63) / 64 * 64);
@@ -634,7 +638,7 @@ struct RadiiSelfPlan {
 static RadiiSelfPlan radii_self_plan(int prec, int64_t n, bool periodic, const rmw_tuning* tuning)
 {
   RadiiSelfPlan pl;
-  pl.ordered = radii_plan(prec, n, n, tuning, periodic ? kRDirectPairs : kRDirectSelf);
+  pl.ordered = radii_plan(prec, n, n, tuning, periodic, periodic ? kRDirectPairs : kRDirectSelf);
   const int sym = tuning ? tuning->symmetric : 0;
   const int cu = std::max(device_props().cu_count, 1);
   pl.blocks = !shaped(tuning) && !pl.ordered.direct && !periodic && n <= kRBlockBlobs;
@@ -668,7 +672,7 @@ extern "C" int rmw_radii_workspace_size(int prec, int64_t ns, int64_t nt, const 
 {
   return guarded([&] {
     RMW_REQUIRE(bytes != nullptr, "bytes is null");
-    *bytes = radii_plan(prec, ns, nt, tuning).bytes;
+    *bytes = radii_plan(prec, ns, nt, tuning, true).bytes;
   });
 }
 
@@ -780,7 +784,7 @@ extern "C" int rmw_radii_apply(int prec, int boundary, const double* source, con
                                void* workspace, size_t workspace_bytes, void* stream)
 {
   return guarded([&] {
-    const RadiiPlan pl = radii_plan(prec, ns, nt, tuning);
+    const RadiiPlan pl = radii_plan(prec, ns, nt, tuning, any_periodic(L));
     check_boundary(boundary);
     RMW_REQUIRE(workspace_bytes >= pl.bytes, "workspace too small: need " + std::to_string(pl.bytes) + " bytes");
     RMW_REQUIRE(eta > 0.0 && std::isfinite(eta), "eta must be positive");
