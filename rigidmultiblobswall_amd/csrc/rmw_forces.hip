@@ -364,7 +364,7 @@ __global__ __launch_bounds__(kFBlock) void force_direct_kernel(ForceParams p, do
 // If more than a quarter of all ordered pairs would be visited (by the
 // estimate, which depends on the blobs and their order alone), or a blob
 // does not fit the cell arithmetic, the last launch evaluates all pairs
-// instead: as the direct kernel does up to direct_fallback blobs, by the
+// instead: as the direct kernel does up to kCellsDirectFallback blobs, by the
 // symmetric (or the ordered) kernel, whose reduce follows, beyond.
 // ---------------------------------------------------------------------------
 struct CellTotals {
@@ -733,12 +733,15 @@ static int64_t direct_blobs(bool f64, bool periodic, bool cutoff)
   if (!cutoff) return periodic ? 5120 : 6144;
   return periodic ? 2304 : 3072;
 }
-// Blobs up to which a suspension that the cells turn out not to suit goes
-// through the direct kernel; direct / symmetric kernel and reduce (us): fp32
-// open 35 / 51 at 6000, 46 / 52 at 7000, 60 / 67 at 8192, periodic 82 / 102 at
-// 6000, 110 / 103 at 7000; FP64 open 71 / 87 and 95 / 88, periodic 114 / 136 and
+// Blobs up to which all pairs are evaluated by the direct kernel where the cells
+// cannot serve the call; direct / symmetric kernel and reduce (us): fp32 open
+// 35 / 51 at 6000, 46 / 52 at 7000, 60 / 67 at 8192, periodic 82 / 102 at 6000,
+// 110 / 103 at 7000; FP64 open 71 / 87 and 95 / 88, periodic 114 / 136 and
 // 152 / 137.
 static int64_t direct_fallback(bool f64, bool periodic) { return f64 || periodic ? 6400 : 8192; }
+// The same where the cells may turn out not to suit the suspension: the symmetric
+// kernel's reduce is then launched whether they do or not, 3 us of 24 when they do.
+constexpr int64_t kCellsDirectFallback = 8192;
 // Beyond these exponents (r - 2a)/b the exponential is exactly 0.
 constexpr double kRangeF64 = 746.0, kRangeF32 = 104.5;
 
@@ -847,7 +850,7 @@ static void launch_force(bool mutual, const ForceParams& q, int grid, hipStream_
 
 template <bool F64, bool CUT>
 static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const CellParams& c, double scale,
-                               bool small, double* force, hipStream_t st)
+                               double* force, hipStream_t st)
 {
   const dim3 b(kFBlock), nb((unsigned)((q.n + 255) / 256)), hb(pl.buckets / 256);
   hipLaunchKernelGGL(cells_zero_kernel, hb, b, 0, st, c);
@@ -855,6 +858,7 @@ static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const 
   hipLaunchKernelGGL(cells_place_kernel, hb, b, 0, st, c);
   hipLaunchKernelGGL(cells_list_kernel, nb, b, 0, st, q, c);
   hipLaunchKernelGGL(cells_sort_kernel<F64>, nb, b, 0, st, q, c);
+  const bool small = q.n <= kCellsDirectFallback;
   const int64_t all = small ? (q.n + kDT - 1) / kDT : pl.total_items;
   const int64_t wgs = (q.n * kCellLanes + kFBlock - 1) / kFBlock;
   const dim3 g((unsigned)std::min<int64_t>(std::max(wgs, all), (int64_t)INT32_MAX));
@@ -869,12 +873,12 @@ static void launch_force_cells(const ForcePlan& pl, const ForceParams& q, const 
 
 template <bool F64, bool CUT>
 static void launch_any(const ForcePlan& pl, const ForceParams& q, const CellParams& c, bool direct, bool cells,
-                       bool small, double scale, double* force, int grid, hipStream_t st)
+                       double scale, double* force, int grid, hipStream_t st)
 {
   if (direct)
     hipLaunchKernelGGL((force_direct_kernel<F64, CUT>), dim3((unsigned)((q.n + kDT - 1) / kDT)), dim3(kFBlock), 0, st, q,
                        scale, force);
-  else if (cells) launch_force_cells<F64, CUT>(pl, q, c, scale, small, force, st);
+  else if (cells) launch_force_cells<F64, CUT>(pl, q, c, scale, force, st);
   else launch_force<F64, CUT>(pl.mutual, q, grid, st);
 }
 
@@ -978,20 +982,19 @@ extern "C" int rmw_blob_forces(int prec, const double* r_vectors, const double* 
     }
     // what the cells cannot serve goes the same way as what they turn out not
     // to suit
-    const bool small = n <= direct_fallback(f64, boxed);
-    const bool direct = pl.direct || (pl.cells && !cells && !in_place && small);
+    const bool direct = pl.direct || (pl.cells && !cells && !in_place && n <= direct_fallback(f64, boxed));
     double* const out = direct && in_place ? (double*)workspace : force;
     if (f64) {
-      if (cut) launch_any<true, true>(pl, q, c, direct, cells, small, scale, out, grid, st);
-      else launch_any<true, false>(pl, q, c, direct, cells, small, scale, out, grid, st);
+      if (cut) launch_any<true, true>(pl, q, c, direct, cells, scale, out, grid, st);
+      else launch_any<true, false>(pl, q, c, direct, cells, scale, out, grid, st);
     } else {
-      if (cut) launch_any<false, true>(pl, q, c, direct, cells, small, scale, out, grid, st);
-      else launch_any<false, false>(pl, q, c, direct, cells, small, scale, out, grid, st);
+      if (cut) launch_any<false, true>(pl, q, c, direct, cells, scale, out, grid, st);
+      else launch_any<false, false>(pl, q, c, direct, cells, scale, out, grid, st);
     }
     RMW_CHECK_HIP(hipGetLastError());
     prof_end(rec, prof, st);
     if (out != force) launch_copy_rows(out, 3 * n, force, 3 * n, 3 * n, 1, st);
-    if (direct || (cells && small)) return;
+    if (direct || (cells && n <= kCellsDirectFallback)) return;
     const dim3 rg((unsigned)((n * 3 + 255) / 256)), rb(256);
     if (pl.mutual)
       hipLaunchKernelGGL(force_mutual_reduce_kernel, dim3((unsigned)((n * 3 + kFRedOut - 1) / kFRedOut)), rb, 0, st,
